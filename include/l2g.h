@@ -188,7 +188,9 @@ int l2g_eri_plan_device_output(l2g_eri_plan plan, double** d_out);
  * the number of quartets, the number of primitive quartets (before the
  * per-primitive screen) and the duration in ms of its last execution
  * (HIP events on the context stream).  The code adds 10000 for an FP32
- * kernel, 20000 for the generic kernel and 100000 for a wave per quartet
+ * kernel, 20000 for the generic kernel and for the classes beyond the node
+ * limit of the per-lane kernels ((df|ff), (ff|ff)), and 100000 where the
+ * primitive loops of the class's quartets are split over lanes or blocks
  * (l2g_eri_plan_set_wave_split). */
 int l2g_eri_plan_stats(l2g_eri_plan plan, int cap, int* nclasses, int* class_code, int64_t* nquartets,
                        int64_t* nprim_quartets, float* ms);
@@ -215,25 +217,23 @@ int l2g_eri_plan_set_graph(l2g_eri_plan plan, int on);
 #define L2G_OPER_ERFC_COULOMB 2
 int l2g_eri_plan_set_operator(l2g_eri_plan plan, int oper, double omega);
 
-/* Wave split (on by default; on = 0 turns it off): classes of few, deeply
- * contracted quartets run a wave per quartet whose 64 lanes split the
- * primitive loop, instead of one lane per quartet, so that a handful of
- * long contractions no longer serialise on a few lanes.  With on = 1 a
- * class measured faster there on the generic kernel (its quartets split
- * over blocks by primitive range, summed per quartet in a fixed order) runs
- * on it instead when it holds at least half of the plan's quartets; on = 2
- * keeps every such class on its register kernel.  Each contraction
- * is then summed as 64 serial partial sums joined by a fixed butterfly,
+/* Split of deep primitive loops (default on).  Classes with a Rys kernel (all
+ * but (ss|..)) whose deepest quartets would outlast the rest of their launch
+ * are cut into pieces of their primitive loops, evaluated by separate blocks
+ * and summed per quartet in piece order; (ss|..) classes of few quartets
+ * (fewer than a quarter of the chip's lanes at one wave per SIMD) averaging
+ * at least 16 primitive quartets run a wave per quartet, its contraction
+ * summed as 64 serial partial sums joined by a fixed butterfly.  Both are
  * another order than libint's serial primitive loop
- * (engine.impl.h:1306-1766).  Well-conditioned integrals agree with the
- * lane-per-quartet order to rounding; on ill-conditioned ones (large
- * cancelling terms) both orders stay within the error the reference's own
- * FP64 algorithm makes against the exact integral.  Off: such classes of
- * total angular momentum 7 and more run on the generic kernel (a block per
- * quartet, serial order), the rest a lane per quartet.  Whether a class
- * runs a wave per quartet depends on how many quartets of it the plan holds,
- * so the same quartet in plans of another composition can differ in its last
- * bits; with the split off a quartet's values depend on the quartet only.
+ * (engine.impl.h:1306-1766): well-conditioned integrals agree with it to
+ * rounding, ill-conditioned ones (large cancelling terms) stay within the
+ * error the reference's own FP64 algorithm makes against the exact integral.
+ * on = 2 is accepted as 1.  Off: classes of few quartets averaging at least
+ * 64 primitive quartets with a total angular momentum of 7 and more run on
+ * the generic kernel (a block per quartet), the rest unsplit.  Whether a
+ * class is split depends on how many quartets of it the plan holds, so the
+ * same quartet in plans of another composition can differ in its last bits;
+ * with the split off an unsplit quartet's values depend on the quartet only.
  * No counterpart in the reference. */
 int l2g_eri_plan_set_wave_split(l2g_eri_plan plan, int on);
 

@@ -464,12 +464,10 @@ class EriPlan:
         _check(lib().l2g_eri_plan_set_operator(self._h, int(oper), float(omega)))
 
     def set_wave_split(self, on=True):
-        """Classes of few, deeply contracted quartets run a wave per quartet
-        (lanes split the primitive loop; on by default): each contraction is
-        summed as 64 partial sums and a fixed butterfly instead of libint's
-        serial order.  True (1) routes the classes measured faster on the
-        generic kernel there instead; 2 keeps them all on their register
-        kernels; False (0) turns the split off."""
+        """Split of deep primitive loops over lanes or blocks (on by default;
+        2 is accepted as 1): each contraction is then summed as partial sums
+        in a fixed order instead of libint's serial one.  False (0) turns it
+        off (l2g_eri_plan_set_wave_split)."""
         _check(lib().l2g_eri_plan_set_wave_split(self._h, int(on)))
 
     def elapsed_ms(self):

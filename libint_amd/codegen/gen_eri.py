@@ -1031,7 +1031,7 @@ def class_waves(plan, budget, waves):
 
 
 def generate(outdir, lmax=2, budget=160, nfiles=8, waves=0, only=None, budgets=None,
-             modes=('eri', 'fock', 'schwarz', 'fp32', 'erf'), generic_lmax=3, max_nodes=0, fp32_lmax=2,
+             modes=('eri', 'fock', 'schwarz', 'fp32', 'erf', 'rys'), generic_lmax=3, max_nodes=0, fp32_lmax=2,
              erf_lmax=2, mfma_acc=False):
     """Write the kernels and the dispatch tables.  `budgets` maps a class name
     ('2222') to its own (budget, waves).  Classes with an l above 2 whose
@@ -1047,7 +1047,7 @@ def generate(outdir, lmax=2, budget=160, nfiles=8, waves=0, only=None, budgets=N
 
     def cfg(c):
         v = budgets.get("".join(map(str, c)), (budget, waves))
-        return tuple(v) + (0,) * (4 - len(v))  # (budget, waves, FP32 pays, generic for few deep quartets)
+        return tuple(v) + (0,) * (3 - len(v))  # (budget, waves, FP32 pays)
 
     plans = [plan_class(*c, budget=cfg(c)[0]) for c in classes]
     if max_nodes:
@@ -1055,16 +1055,18 @@ def generate(outdir, lmax=2, budget=160, nfiles=8, waves=0, only=None, budgets=N
     # reduced-precision variants hold twice as many values per register
     plans32 = [plan_class(p.la, p.lb, p.lc, p.ld, budget=2 * cfg((p.la, p.lb, p.lc, p.ld))[0]) for p in plans
                if max(p.la, p.lb, p.lc, p.ld) <= fp32_lmax] if 'fp32' in modes else []
+    # classes on the Rys kernels (gen_rys.py) have no other FP64 ERI, erf or Fock kernel
+    sys.path.insert(0, os.path.dirname(os.path.abspath(__file__)))
+    import gen_rys
+    ryscls = [c for c in classes if gen_rys.use(*c)] if 'rys' in modes else []
     jobs = []  # (plan, mode, real)
     for p in plans:
-        if 'eri' in modes:
-            jobs.append((p, 'eri', 'double'))
-        if 'fock' in modes:
-            jobs.append((p, 'fock', 'double'))
+        if (p.la, p.lb, p.lc, p.ld) not in ryscls:
+            jobs += [(p, m, 'double') for m in ('eri', 'fock') if m in modes]
         if 'schwarz' in modes and (p.la, p.lb) == (p.lc, p.ld):
             jobs.append((p, 'schwarz', 'double'))
     for p in plans:
-        if 'erf' in modes and max(p.la, p.lb, p.lc, p.ld) <= erf_lmax:
+        if 'erf' in modes and max(p.la, p.lb, p.lc, p.ld) <= erf_lmax and (p.la, p.lb, p.lc, p.ld) not in ryscls:
             jobs.append((p, 'erf', 'double'))
     for p in plans32:
         if 'eri' in modes:
@@ -1110,10 +1112,28 @@ def generate(outdir, lmax=2, budget=160, nfiles=8, waves=0, only=None, budgets=N
     for p, k, _ in table + stable + ftable + table32 + ftable32 + etable:
         lines.append(f"void {k}_launch(const L2gEriArgs& A, int grid, int block, hipStream_t s);")
     lines.append('')
+    rys = {m: gen_rys.generate(ryscls, m) for m in ('eri', 'fock') if m in modes}
+    for k, v in enumerate(gen_rys.files(rys.get('eri', []) + rys.get('fock', []), nfiles)):
+        fn = os.path.join(outdir, f"rys_gen_{k}.hip")
+        new = '// generated by libint_amd/codegen/gen_rys.py - do not edit\n#include "rys_device.h"\n\n' + '\n'.join(v)
+        if not (os.path.exists(fn) and open(fn).read() == new):
+            with open(fn, 'w') as f:
+                f.write(new)
+        written.append(fn)
+    import rys_table
+    fn = os.path.join(outdir, "rys_table.cpp")
+    new = rys_table.emit()
+    if not (os.path.exists(fn) and open(fn).read() == new):
+        with open(fn, 'w') as f:
+            f.write(new)
+    written.append(fn)
+    for v in rys.values():
+        for _, n, _ in v:
+            lines.append(f"void {n}_launch(const L2gEriArgs& A, int grid, int block, hipStream_t s);")
     lines.append(f"extern const int l2g_gen_lmax = {lmax};")
     for name, tab in (("l2g_gen_classes", table), ("l2g_gen_schwarz", stable), ("l2g_gen_fock", ftable),
                       ("l2g_gen_classes32", table32), ("l2g_gen_fock32", ftable32),
-                      ("l2g_gen_classes_erf", etable)):
+                      ("l2g_gen_classes_erf", etable), ("l2g_gen_rys", [])):
         lines.append(f"extern const L2gClassInfo {name}[] = {{")
         for p, k, in_regs in tab:
             ybuf = 0 if in_regs else len(p.ecomps) * ncart(p.lc) * ncart(p.ld) + \
@@ -1121,15 +1141,19 @@ def generate(outdir, lmax=2, budget=160, nfiles=8, waves=0, only=None, budgets=N
             if not in_regs and name in ("l2g_gen_classes", "l2g_gen_classes32", "l2g_gen_classes_erf"):
                 ybuf += ncart(p.la) * ncart(p.lb) * ncart(p.lc) * ncart(p.ld)  # staged output
             pays = cfg((p.la, p.lb, p.lc, p.ld))[2] if name in ("l2g_gen_classes32", "l2g_gen_fock32") else 0
-            fewgen = cfg((p.la, p.lb, p.lc, p.ld))[3] if name == "l2g_gen_classes" else 0
             lines.append(f"  {{{p.la}, {p.lb}, {p.lc}, {p.ld}, {len(p.groups)}, {ybuf}, "
-                         f"{sum(p.group_nodes)}, {pays}, {fewgen}, &{k}_launch}},")
-        if not tab:
-            lines.append("  {0, 0, 0, 0, 0, 0, 0, 0, 0, nullptr},")
+                         f"{sum(p.group_nodes)}, {pays}, 0, 0, &{k}_launch}},")
+        rest = rys.get({'l2g_gen_fock': 'fock', 'l2g_gen_rys': 'eri'}.get(name), [])
+        for p, n, _ in rest:
+            over = int(not any((x.la, x.lb, x.lc, x.ld) == p.l for x in plans))
+            lines.append(f"  {{{', '.join(map(str, p.l))}, 1, 0, {int(p.cost())}, 0, {over}, {p.nt // p.q}, &{n}_launch}},")
+        if not tab and not rest:
+            lines.append("  {0, 0, 0, 0, 0, 0, 0, 0, 0, 0, nullptr},")
         lines.append("};")
     lines.append(f"extern const int l2g_gen_nclasses = {len(table)};")
     lines.append(f"extern const int l2g_gen_nschwarz = {len(stable)};")
-    lines.append(f"extern const int l2g_gen_nfock = {len(ftable)};")
+    lines.append(f"extern const int l2g_gen_nfock = {len(ftable) + len(rys.get('fock', []))};")
+    lines.append(f"extern const int l2g_gen_nrys = {len(rys.get('eri', []))};")
     lines.append(f"extern const int l2g_gen_nclasses32 = {len(table32)};")
     lines.append(f"extern const int l2g_gen_nfock32 = {len(ftable32)};")
     lines.append(f"extern const int l2g_gen_nclasses_erf = {len(etable)};")
@@ -1140,7 +1164,6 @@ def generate(outdir, lmax=2, budget=160, nfiles=8, waves=0, only=None, budgets=N
             f.write(new)
     written.append(fn)
     # programs of the generic kernel: every canonical class up to generic_lmax
-    sys.path.insert(0, os.path.dirname(os.path.abspath(__file__)))
     import gen_generic
     fn = os.path.join(outdir, "generic_table.cpp")
     new = gen_generic.emit_tables(canonical_classes(generic_lmax), generic_lmax)
@@ -1163,7 +1186,7 @@ if __name__ == '__main__':
                     help="per class budget:waves[:fp32], e.g. 2222=64:2,2122=80:2:1 (fp32 1: the class's FP32 "
                          "variant measured faster than its FP64 kernel, so mixed batches route quartets to it)")
     ap.add_argument("--nfiles", type=int, default=8)
-    ap.add_argument("--modes", default="eri,fock,schwarz,fp32,erf")
+    ap.add_argument("--modes", default="eri,fock,schwarz,fp32,erf,rys")
     ap.add_argument("--generic-lmax", type=int, default=3, help="highest l of the generic kernel's classes")
     ap.add_argument("--max-nodes", type=int, default=0,
                     help="classes with l > 2 and more recursion nodes than this run on the generic kernel")

@@ -88,6 +88,7 @@ struct L2gEriArgs {
   const double2* __restrict__ pp_aux;
   const double* __restrict__ pp_nonsph;
   const double* __restrict__ boys;  // [m][iv][8]
+  const double* __restrict__ rys;   // Rys nodes and weights (codegen/rys_table.py)
   double precision, ln_precision, scale;
   int method;
   int shg_gaussian;
@@ -121,10 +122,19 @@ struct L2gEriArgs {
   // item = quartet; sums rows gpart_first[item] .. gpart_first[item + 1] - 1
   // in order, then HRR and store); 0 = neither
   int gpart_mode;
+  // Rys ERI kernels: work items at the front of the list with at least
+  // L2G_RYS_DEEP0 and L2G_RYS_DEEP1 primitive quartets (rys_tier_of)
+  int rys_deep[2];
   long long gpart_stride;
   double* __restrict__ gpart;
   const int* __restrict__ gpart_first;
 };
+
+// Tier of a quartet of w primitive quartets on a Rys kernel: 0 and 1 share
+// their primitive loop between 16 and 4 slots of a block, 2 runs on one.
+#define L2G_RYS_DEEP0 128
+#define L2G_RYS_DEEP1 32
+inline int rys_tier_of(long long w) { return w >= L2G_RYS_DEEP0 ? 0 : w >= L2G_RYS_DEEP1 ? 1 : 2; }
 
 typedef void (*L2gLaunchFn)(const L2gEriArgs&, int grid, int block, hipStream_t s);
 
@@ -154,7 +164,8 @@ struct L2gClassInfo {
   int ybuf_doubles;  // per lane; 0 = rows kept in registers
   int nodes;         // VRR graph nodes per primitive quartet (all groups)
   int fp32_pays;     // FP32 variants: measured faster than the class's FP64 kernel
-  int few_generic;   // FP64 ERI kernels: few deep quartets measured faster on the generic kernel
+  int over_limit;    // Rys kernels: the class is beyond the node limit of the per-lane kernels
+  int lanes;         // Rys kernels: lanes per work item (0: a lane per item, with lane scratch)
   L2gLaunchFn launch;
 };
 

@@ -309,6 +309,10 @@ int split_chunk(int cls, int64_t m, int64_t total, int lanes) {
   if (m == 0) return INT_MAX;
   if (fock_is_generic(cls))
     return m < 4096 ? std::max(16, 2000000 / std::max(1, fock_gclass(cls).nvals)) : INT_MAX;
+  if (const int per = fock_info(cls).lanes) {  // a tile of lanes per item, at 2 waves per SIMD
+    const int64_t slots = std::max<int64_t>(1, 2ll * lanes / per);
+    return (int)std::min<int64_t>(INT_MAX, std::max<int64_t>(32, (total + 2 * slots - 1) / (2 * slots)));
+  }
   const int minc = std::max(8, std::min(16, 140000 / std::max(1, fock_info(cls).nodes)));
   const int64_t share = (total + 2ll * lanes - 1) / (2ll * std::max(1, lanes));
   return (int)std::min<int64_t>(INT_MAX, std::max<int64_t>(minc, share));
@@ -476,6 +480,7 @@ L2gEriArgs fock_args(l2g_context_s* ctx, int method, const int* pair_first, cons
   A.pp_aux = aux;
   A.pp_nonsph = ns;
   A.boys = ctx->boys.as<double>();
+  A.rys = ctx->rys.as<double>();
   A.scale = 1.0;
   A.method = method;
   A.shg_gaussian = ctx->shg_gaussian;
@@ -871,7 +876,7 @@ int l2g_fock_build(l2g_fock f, const double* D, double precision, double* J, dou
         if (m == 0) continue;
         // the generic kernel runs a block per item, no lane scratch, a few
         // blocks per CU: up to 4 items per CU count as small (side streams)
-        lanes[c] = fock_is_generic(c) ? m * 64 : m;
+        lanes[c] = fock_is_generic(c) ? m * 64 : m * std::max(1, fock_info(c).lanes);
         yd[c] = fock_ybuf(c);
         ymax = std::max<int64_t>(ymax, yd[c]);
       }
@@ -1351,7 +1356,7 @@ void run_round(l2g_server_s* S, const std::vector<ServerRequest*>& act) {
   std::vector<int64_t> lanes(rv.count.size(), 0), yd(rv.count.size(), 0);
   for (size_t c = 0; c < rv.count.size(); ++c) {
     if (rv.count[c] == 0) continue;
-    lanes[c] = fock_is_generic((int)c) ? rv.count[c] * 64 : rv.count[c];
+    lanes[c] = fock_is_generic((int)c) ? rv.count[c] * 64 : rv.count[c] * std::max(1, fock_info((int)c).lanes);
     yd[c] = fock_ybuf((int)c);
   }
   std::vector<ClassSlot> slots;  // within the server's scratch (sized for the full grid)

@@ -87,6 +87,9 @@ struct ClassWork {
   bool generic = false;
   bool native_generic = false;  // no register kernel for this class
   bool coop = false;  // a wave per quartet (few, deeply contracted quartets)
+  int rys = -1;       // index into l2g_gen_rys where the class runs on its Rys kernel
+  int rys_cls = -1;   // the class's Rys kernel, whether it runs on it or not
+  int rys_deep[2] = {0, 0};  // items in its tiers of deep quartets (rys_tier_of)
   int gidx = -1;      // the class's program in the generic kernel's tables
   int64_t first, count;
   ClassSlot slot;     // grid, scratch region and stream of the launch
@@ -116,7 +119,6 @@ struct l2g_eri_plan_s {
   int64_t ymax = 0;  // largest scratch doubles per lane over the classes
   int block = 128;
   bool wave_split = true;  // classes of few deep quartets run a wave per quartet
-  bool few_generic = true;  // ... or the generic kernel, where measured faster
   int oper = 0;             // 0 Coulomb, 1 erf-attenuated, 2 erfc-attenuated
   double omega = 0;
   // hipGraph mode: the class launches are captured once per output buffer
@@ -265,6 +267,8 @@ int l2g_init(int device, l2g_context* out) {
     const auto& t = boys_table().t;
     ctx->boys.alloc(t.size() * sizeof(double));
     HIPCHK(hipMemcpy(ctx->boys.p, t.data(), t.size() * sizeof(double), hipMemcpyHostToDevice));
+    ctx->rys.alloc((size_t)l2g_rys_table_size * sizeof(double));
+    HIPCHK(hipMemcpy(ctx->rys.p, l2g_rys_table, (size_t)l2g_rys_table_size * sizeof(double), hipMemcpyHostToDevice));
     for (auto& a : ctx->class_of)
       for (auto& b : a)
         for (auto& c : b)
@@ -285,6 +289,7 @@ int l2g_init(int device, l2g_context* out) {
     fill(ctx->class32_of, l2g_gen_classes32, l2g_gen_nclasses32);
     fill(ctx->classerf_of, l2g_gen_classes_erf, l2g_gen_nclasses_erf);
     fill(ctx->fock32_of, l2g_gen_fock32, l2g_gen_nfock32);
+    fill(ctx->rys_of, l2g_gen_rys, l2g_gen_nrys);
     for (auto& a : ctx->schwarz_of)
       for (auto& b : a) b = -1;
     for (int i = 0; i < l2g_gen_nschwarz; ++i) {
@@ -477,6 +482,12 @@ static int plan_create_impl(l2g_basis B, int64_t nq, const int32_t* quartets, do
       int64_t w;
     };
     const int nc32 = l2g_gen_nclasses32;
+    auto bucket64 = [&](int a, int b, int c, int d) {
+      const int r = ctx->force_generic ? -1 : ctx->class_of[a][b][c][d];
+      if (r >= 0) return r;
+      const int g = ctx->generic_of[a][b][c][d];
+      return g < 0 ? -1 : nc64 + nc32 + g;
+    };
     std::vector<std::vector<Item>> buckets(l2g_gen_nclasses + l2g_gen_nclasses32 + l2g_gen_ngeneric);
     plan->offsets.resize(nq);
     int64_t total = 0;
@@ -491,14 +502,13 @@ static int plan_create_impl(l2g_basis B, int64_t nq, const int32_t* quartets, do
       const int b2 = sbk ? (stk ? s[2] : s[3]) : (stb ? s[0] : s[1]);
       const int k1 = sbk ? (stb ? s[1] : s[0]) : (stk ? s[3] : s[2]);
       const int k2 = sbk ? (stb ? s[0] : s[1]) : (stk ? s[2] : s[3]);
-      int cls = ctx->force_generic ? -1 : ctx->class_of[B->l[b1]][B->l[b2]][B->l[k1]][B->l[k2]];
-      if (cls < 0) {
-        const int g = ctx->generic_of[B->l[b1]][B->l[b2]][B->l[k1]][B->l[k2]];
-        if (g < 0) throw L2gError(L2G_E_LMAX, "no kernel for this angular momentum class");
-        cls = nc64 + nc32 + g;  // FP64 only
-      } else if (fp32_threshold > 0 && use_fp32(s)) {
+      // FP64: the class's register kernel where it has one, else the bucket of
+      // its generic program (its Rys kernel, or the generic kernel)
+      int cls = bucket64(B->l[b1], B->l[b2], B->l[k1], B->l[k2]);
+      if (cls < 0) throw L2gError(L2G_E_LMAX, "no kernel for this angular momentum class");
+      if (!ctx->force_generic && fp32_threshold > 0) {
         const int c32 = ctx->class32_of[B->l[b1]][B->l[b2]][B->l[k1]][B->l[k2]];
-        if (c32 >= 0 && (ctx->fp32_policy || l2g_gen_classes32[c32].fp32_pays)) cls = nc64 + c32;
+        if (c32 >= 0 && (ctx->fp32_policy || l2g_gen_classes32[c32].fp32_pays) && use_fp32(s)) cls = nc64 + c32;
       }
       auto purebit = [&](int sh) { return (B->pure[sh] && B->l[sh] > 0) ? 1 : 0; };
       const int meta = (stb ? 1 : 0) | (stk ? 2 : 0) | (sbk ? 4 : 0) | (purebit(b1) << 3) | (purebit(b2) << 4) |
@@ -525,7 +535,7 @@ static int plan_create_impl(l2g_basis B, int64_t nq, const int32_t* quartets, do
         auto& v = buckets[nc64 + c32];
         if (v.empty() || v.size() >= min_items) continue;
         const L2gClassInfo& ci = l2g_gen_classes32[c32];
-        const int c64 = ctx->class_of[ci.la][ci.lb][ci.lc][ci.ld];
+        const int c64 = bucket64(ci.la, ci.lb, ci.lc, ci.ld);
         if (c64 < 0) continue;
         auto& d = buckets[c64];
         d.insert(d.end(), v.begin(), v.end());
@@ -561,6 +571,10 @@ static int plan_create_impl(l2g_basis B, int64_t nq, const int32_t* quartets, do
       {
         const L2gClassInfo* ci = isgen ? nullptr : &(is32 ? l2g_gen_classes32 : l2g_gen_classes)[c];
         cw.gidx = isgen ? c : ctx->generic_of[ci->la][ci->lb][ci->lc][ci->ld];
+        if (!is32 && !ctx->force_generic) {
+          const L2gGenericClass* gi = isgen ? &l2g_gen_generic[c] : nullptr;
+          cw.rys_cls = gi ? ctx->rys_of[gi->la][gi->lb][gi->lc][gi->ld] : ctx->rys_of[ci->la][ci->lb][ci->lc][ci->ld];
+        }
       }
       cw.first = (int64_t)bra.size();
       cw.count = (int64_t)v.size();
@@ -573,6 +587,7 @@ static int plan_create_impl(l2g_basis B, int64_t nq, const int32_t* quartets, do
         qidx.push_back(it.q);
         plan->itemw.push_back(it.w);
         cw.nprimq += it.w;
+        if (const int t = rys_tier_of(it.w); t < 2) ++cw.rys_deep[t];
       }
       HIPCHK(hipEventCreate(&cw.ev0));
       HIPCHK(hipEventCreate(&cw.ev1));
@@ -605,21 +620,19 @@ static int plan_create_impl(l2g_basis B, int64_t nq, const int32_t* quartets, do
 
 namespace {
 
-// Launch layout of a plan: a persistent grid with enough blocks to fill
-// every CU several times over, and the lane-private scratch for it.  A class
-// of few quartets (fewer than a quarter of the chip's lanes at one wave per
-// SIMD) with deep primitive loops would, at one lane per quartet, leave most
-// of the chip idle while a few lanes run their loops serially.  With
-// wave_split (the default) such a class runs a wave per quartet whose lanes
-// split the loop (summing each contraction as 64 serial partial sums and a
-// fixed butterfly, another order than libint's serial loop, no less
-// accurate); without it, a class of total angular momentum 7 or more averaging at least
-// 64 primitive quartets per quartet runs on the generic kernel, a block per
-// quartet whose threads split the targets and keep each contraction's
-// serial order.  Lower classes have too few targets per quartet to occupy
-// a block and stay at a lane per quartet (on 400k quartets of an s-f basis
-// with K up to 8, the cut at L >= 7 measured 180 ms, at 5, 6, 8 339, 276
-// and 207 ms, and 1556 ms without the generic kernel).
+// Launch layout of a plan.  A class with a Rys kernel runs on it, a tile of
+// lanes per quartet; with wave_split (the default) a class whose deepest
+// quartets would outlast the rest has its primitive loops cut into pieces
+// (plan_pieces).  The other classes run on their per-lane kernels: a
+// persistent grid with enough blocks to fill every CU several times over, and
+// the lane-private scratch for it; of these, a class of few quartets (fewer
+// than a quarter of the chip's lanes at one wave per SIMD) with deep
+// primitive loops runs, with wave_split, a wave per quartet whose lanes split
+// the loop (summing each contraction as 64 serial partial sums and a fixed
+// butterfly, another order than libint's serial loop, no less accurate).
+// Without wave_split, a class of few deep quartets (averaging at least 64
+// primitive quartets) and total angular momentum 7 or more runs on the
+// generic kernel, a block per quartet whose threads split the targets.
 #ifndef L2G_GENERIC_MIN_DEPTH
 #define L2G_GENERIC_MIN_DEPTH 64
 #endif
@@ -627,9 +640,12 @@ namespace {
 #define L2G_GENERIC_MIN_L 7
 #endif
 
-// total angular momentum of a class with a register kernel
+// total angular momentum of a class
 int class_l(const ClassWork& c) {
-  if (c.native_generic) return 99;
+  if (c.native_generic) {
+    const L2gGenericClass& g = l2g_gen_generic[c.spec_cls];
+    return g.la + g.lb + g.lc + g.ld;
+  }
   const L2gClassInfo& ci = (c.fp32 ? l2g_gen_classes32 : l2g_gen_classes)[c.spec_cls];
   return ci.la + ci.lb + ci.lc + ci.ld;
 }
@@ -651,12 +667,22 @@ void plan_pieces(l2g_eri_plan_s* p, l2g_context_s* ctx) {
   int64_t gtotal = 0;
   for (auto& c : p->classes) {
     c.npieces = 0;
-    if (!c.generic || c.count > (int64_t)ctx->ncu * 16) continue;
+    if (c.rys >= 0 ? !p->wave_split : !c.generic || c.count > (int64_t)ctx->ncu * 16) continue;
     int wmax = 0;
     for (int64_t i = c.first; i < c.first + c.count; ++i) wmax = std::max(wmax, p->itemw[(size_t)i]);
-    int64_t chunk = std::max<int64_t>(32, (c.nprimq + 4 * ctx->ncu - 1) / (4 * ctx->ncu));
-    chunk += chunk & 1;  // even: the two-primitive pass stays full
-    if (wmax <= chunk) continue;
+    int64_t chunk;
+    if (c.rys >= 0) {
+      const int64_t slots = (int64_t)ctx->ncu * 512 / l2g_gen_rys[c.rys].lanes;  // quartets at 2 waves per SIMD
+      chunk = std::max<int64_t>(48, (c.nprimq + slots - 1) / slots);
+      // the longest serial loop: the deepest quartet's, shared by up to 16 slots
+      const int64_t serial = wmax / std::min<int64_t>(wmax >= L2G_RYS_DEEP0 ? 16 : wmax >= L2G_RYS_DEEP1 ? 4 : 1,
+                                                      std::max(1, 64 / l2g_gen_rys[c.rys].lanes));
+      if (serial <= 2 * chunk) continue;
+    } else {
+      chunk = std::max<int64_t>(32, (c.nprimq + 4 * ctx->ncu - 1) / (4 * ctx->ncu));
+      chunk += chunk & 1;  // even: the two-primitive pass stays full
+      if (wmax <= chunk) continue;
+    }
     if (!have) {  // the plan's work-item arrays, read back once
       HIPCHK(hipMemcpy(hb.data(), p->bra.p, hb.size() * sizeof(int), hipMemcpyDeviceToHost));
       HIPCHK(hipMemcpy(hk.data(), p->ket.p, hk.size() * sizeof(int), hipMemcpyDeviceToHost));
@@ -664,8 +690,19 @@ void plan_pieces(l2g_eri_plan_s* p, l2g_context_s* ctx) {
       HIPCHK(hipMemcpy(hq.data(), p->qidx.p, hq.size() * sizeof(long long), hipMemcpyDeviceToHost));
       have = true;
     }
-    const L2gGenericClass& g = l2g_gen_generic[c.cls];
-    c.gstride = (int64_t)g.ne * g.accs + 1;
+    if (c.rys >= 0) {
+      const L2gClassInfo& ci = l2g_gen_rys[c.rys];
+      auto nc = [](int l1, int l2) {
+        int n = 0;
+        for (int l = l1; l <= l1 + l2; ++l) n += ncart(l);
+        return n;
+      };
+      c.gstride = (int64_t)nc(ci.la, ci.lb) * nc(ci.lc, ci.ld) + 1;
+      if ((c.count + c.nprimq / chunk) * c.gstride > (int64_t(1) << 27)) continue;  // 1 GiB of pieces
+    } else {
+      const L2gGenericClass& g = l2g_gen_generic[c.cls];
+      c.gstride = (int64_t)g.ne * g.accs + 1;
+    }
     c.piece_off = (int64_t)pb.size();
     c.pfirst_off = (int64_t)pf.size();
     for (int64_t i = c.first; i < c.first + c.count; ++i) {
@@ -704,19 +741,17 @@ void plan_layout(l2g_eri_plan_s* p, l2g_context_s* ctx) {
     c.generic = c.native_generic;
     c.cls = c.spec_cls;
     const bool few = c.count * 4 <= (int64_t)ctx->ncu * 256;
-    // few deep quartets of a class whose register kernel was measured slower
-    // there than the generic kernel (with its quartets split over blocks),
-    // in a plan that is mostly this class: the split generic passes fill
-    // the chip's LDS, and beside other classes (a mixed batch) the wave per
-    // quartet, which leaves most of the chip to them, measured faster overall
-    if (p->wave_split && p->few_generic && !c.generic && !c.fp32 && few && c.nprimq >= 16 * c.count &&
-        c.gidx >= 0 && l2g_gen_classes[c.spec_cls].few_generic && c.count * 2 >= p->nq) {
-      c.generic = true;
-      c.cls = c.gidx;
+    const bool deep_generic = !p->wave_split && !c.fp32 && c.gidx >= 0 && few &&
+                              c.nprimq >= L2G_GENERIC_MIN_DEPTH * c.count && class_l(c) >= L2G_GENERIC_MIN_L;
+    c.rys = deep_generic ? -1 : c.rys_cls;
+    if (c.rys >= 0) {
+      c.coop = c.generic = false;
+      lanes.push_back(c.count * l2g_gen_rys[c.rys].lanes);
+      yd.push_back(0);
+      continue;
     }
     c.coop = p->wave_split && !c.generic && few && c.nprimq >= 16 * c.count;
-    if (!c.generic && !c.coop && !c.fp32 && c.gidx >= 0 && few && c.nprimq >= L2G_GENERIC_MIN_DEPTH * c.count &&
-        class_l(c) >= L2G_GENERIC_MIN_L) {
+    if (deep_generic) {
       c.generic = true;
       c.cls = c.gidx;
     }
@@ -729,13 +764,18 @@ void plan_layout(l2g_eri_plan_s* p, l2g_context_s* ctx) {
   }
   plan_pieces(p, ctx);
   for (size_t i = 0; i < p->classes.size(); ++i)
-    if (p->classes[i].npieces) lanes[i] = p->classes[i].npieces * 64;
+    if (const ClassWork& c = p->classes[i]; c.npieces)
+      lanes[i] = c.npieces * (c.rys >= 0 ? l2g_gen_rys[c.rys].lanes : 64);
   // expected time for the side-stream packing: recursion values per
   // primitive quartet times primitive quartets, at each kernel kind's rate
   // (ns per value, measured on an s-f batch: the generic kernel 0.005 with
   // its quartets split over blocks, 0.03 without; a wave per quartet 0.0025;
   // a lane per quartet 0.02), plus 100 ns per quartet
   for (const auto& c : p->classes) {
+    if (c.rys >= 0) {  // lane operations per primitive quartet, at 2 waves per SIMD on a part of the chip
+      cost.push_back((double)c.nprimq * l2g_gen_rys[c.rys].nodes * 1e-4 + 3.0 * (double)c.count);
+      continue;
+    }
     const double vals = c.generic ? (double)l2g_gen_generic[c.cls].nvals
                                   : (double)(c.fp32 ? l2g_gen_classes32 : l2g_gen_classes)[c.cls].nodes;
     const double rate = c.generic ? (c.npieces ? 0.005 : 0.03) : (c.coop ? 0.0025 : 0.02);
@@ -801,6 +841,7 @@ int l2g_eri_plan_execute(l2g_eri_plan p, double* d_out) {
     A.pp_aux = p->ppAux.as<double2>();
     A.pp_nonsph = p->ppNs.as<double>();
     A.boys = ctx->boys.as<double>();
+    A.rys = ctx->rys.as<double>();
     A.precision = p->precision;
     A.ln_precision = p->ln_precision;
     A.scale = p->scale;
@@ -864,6 +905,32 @@ int l2g_eri_plan_execute(l2g_eri_plan p, double* d_out) {
       A.qidx = p->qidx.as<long long>() + c.first;
       A.n = (int)c.count;
       if (!capture && ps == 0) HIPCHK(hipEventRecord(c.ev0, cs));
+      if (c.rys >= 0) {
+        const L2gClassInfo& ci = l2g_gen_rys[c.rys];
+        L2gEriArgs P = A;
+        if (c.npieces) {  // pieces of the primitive loops, then the sum per quartet
+          P.bra_pair = p->gp_bra.as<int>() + c.piece_off;
+          P.ket_pair = p->gp_ket.as<int>() + c.piece_off;
+          P.meta = p->gp_meta.as<int>() + c.piece_off;
+          P.q_prange = p->gp_range.as<int2>() + c.piece_off;
+          P.n = (int)c.npieces;
+          P.gpart_mode = 1;
+          P.gpart = p->gpart.as<double>() + c.gpart_off;
+          P.gpart_stride = c.gstride;
+          ci.launch(P, 0, 0, cs);
+          LAUNCHCHK(std::string("Rys ERI kernel (pieces) of class ") + std::to_string(c.rys));
+          P = A;
+          P.gpart_mode = 2;
+          P.gpart = p->gpart.as<double>() + c.gpart_off;
+          P.gpart_stride = c.gstride;
+          P.gpart_first = p->gp_first.as<int>() + c.pfirst_off;
+        }
+        if (!c.npieces) P.rys_deep[0] = c.rys_deep[0], P.rys_deep[1] = c.rys_deep[1];
+        ci.launch(P, 0, 0, cs);
+        LAUNCHCHK(std::string("Rys ERI kernel of class ") + std::to_string(c.rys));
+        if (!capture && ps + 1 == passes.size()) HIPCHK(hipEventRecord(c.ev1, cs));
+        continue;
+      }
       int erf_idx = -1;  // the class's erf-attenuated register kernel, for an attenuated pass
       if (A.omega > 0 && !c.generic && !c.fp32) {
         const L2gClassInfo& ci = l2g_gen_classes[c.cls];
@@ -983,7 +1050,6 @@ int l2g_eri_plan_set_wave_split(l2g_eri_plan p, int on) {
     HIPCHK(hipStreamSynchronize(ctx->stream));
     if (on < 0 || on > 2) throw std::invalid_argument("wave split mode must be 0, 1 or 2");
     p->wave_split = on != 0;
-    p->few_generic = on != 2;
     p->drop_graph();
     plan_layout(p, ctx);
   });
@@ -1039,16 +1105,17 @@ int l2g_eri_plan_stats(l2g_eri_plan p, int cap, int* ncls, int* code, int64_t* n
     for (int i = 0; i < (int)p->classes.size() && i < cap; ++i) {
       auto& c = p->classes[i];
       int la, lb, lc, ld;
-      if (c.generic) {
+      if (c.generic || c.native_generic) {
         const auto& g = l2g_gen_generic[c.cls];
         la = g.la, lb = g.lb, lc = g.lc, ld = g.ld;
       } else {
         const auto& ci = (c.fp32 ? l2g_gen_classes32 : l2g_gen_classes)[c.cls];
         la = ci.la, lb = ci.lb, lc = ci.lc, ld = ci.ld;
       }
+      const bool generic = c.rys >= 0 ? l2g_gen_rys[c.rys].over_limit != 0 : c.generic;
       if (code)
-        code[i] = la * 1000 + lb * 100 + lc * 10 + ld + (c.fp32 ? 10000 : 0) + (c.generic ? 20000 : 0) +
-                  (c.coop ? 100000 : 0);
+        code[i] = la * 1000 + lb * 100 + lc * 10 + ld + (c.fp32 ? 10000 : 0) + (generic ? 20000 : 0) +
+                  (c.coop || (c.rys >= 0 && c.npieces) ? 100000 : 0);
       if (nquart) nquart[i] = c.count;
       if (nprimq) nprimq[i] = c.nprimq;
       if (ms) {

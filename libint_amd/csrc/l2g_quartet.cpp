@@ -166,6 +166,7 @@ void quartet_compute_impl(l2g_context_s* ctx, const QuartetBuffers& qb, const in
                    (purebit(k1) << 5) | (purebit(k2) << 6);
   const int64_t n = (int64_t)nfun(l[0], pure[0]) * nfun(l[1], pure[1]) * nfun(l[2], pure[2]) * nfun(l[3], pure[3]);
   const int cls = ctx->force_generic ? -1 : ctx->class_of[l[b1]][l[b2]][l[k1]][l[k2]];
+  const int rys = ctx->force_generic ? -1 : ctx->rys_of[l[b1]][l[b2]][l[k1]][l[k2]];
   const int gcls = ctx->generic_of[l[b1]][l[b2]][l[k1]][l[k2]];
   if (cls < 0 && gcls < 0) throw L2gError(L2G_E_LMAX, "no kernel for this angular momentum class");
   // stage the inputs
@@ -207,6 +208,7 @@ void quartet_compute_impl(l2g_context_s* ctx, const QuartetBuffers& qb, const in
   A.pp_nonsph = reinterpret_cast<const double*>(d + L.ns);
   A.n = 1;
   A.boys = ctx->boys.as<double>();
+  A.rys = ctx->rys.as<double>();
   A.precision = prec;
   A.ln_precision = ln_prec;
   A.scale = scale;
@@ -229,7 +231,12 @@ void quartet_compute_impl(l2g_context_s* ctx, const QuartetBuffers& qb, const in
     A.store_sub = ps.second;
     int erf_idx = -1;
     if (A.omega > 0 && cls >= 0) erf_idx = ctx->classerf_of[l[b1]][l[b2]][l[k1]][l[k2]];
-    if (erf_idx >= 0) {
+    if (rys >= 0) {
+      const int tier = rys_tier_of((long long)pb.np[0] * pb.np[1]);
+      if (tier < 2) A.rys_deep[tier] = 1;
+      l2g_gen_rys[rys].launch(A, 1, kQuartetBlock, st);
+      LAUNCHCHK("Rys ERI kernel (quartet engine)");
+    } else if (erf_idx >= 0) {
       l2g_gen_classes_erf[erf_idx].launch(A, 1, kQuartetBlock, st);
       LAUNCHCHK("erf ERI kernel (quartet engine)");
     } else if (cls < 0 || A.omega > 0) {

@@ -1,0 +1,224 @@
+// Device code shared by the generated Rys-quadrature kernels
+// (codegen/gen_rys.py): nodes and weights, synchronisation within a block,
+// the J/K digest of a quartet block held in LDS.
+#pragma once
+#include "eri_device.h"
+
+#define L2G_RYS_NI 128  // unit intervals of T in the table (codegen/rys_table.py)
+#define L2G_RYS_ND 12   // coefficients per polynomial
+
+// l2g_uniform_cart_scale for l <= 3
+static __constant__ double l2g_uniform_scale[4][10] = {
+    {1.0},
+    {1.0, 1.0, 1.0},
+    {1.0, 1.7320508075688772, 1.7320508075688772, 1.0, 1.7320508075688772, 1.0},
+    {1.0, 2.23606797749979, 2.23606797749979, 2.23606797749979, 3.872983346207417, 2.23606797749979, 1.0,
+     2.23606797749979, 2.23606797749979, 1.0}};
+
+// Order between LDS writes and reads of different lanes of a block.  A block
+// of one wave needs no barrier: its LDS operations complete in order, so only
+// the compiler has to keep them.
+template <int NW>
+__device__ __forceinline__ void rys_sync() {
+  if (NW == 1) {
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+  } else {
+    __syncthreads();
+  }
+}
+
+// Node u (= t^2) and weight w of root r of the NR-point rule at T; tab is the
+// rule's section of the table.
+template <int NR>
+__device__ __forceinline__ void rys_root(double T, const double* __restrict__ tab, int r, double& u, double& w) {
+  const int iv = T < (double)L2G_RYS_NI ? (int)T : L2G_RYS_NI;
+  const double* __restrict__ c = tab + ((size_t)iv * NR + r) * (2 * L2G_RYS_ND);
+  if (iv == L2G_RYS_NI) {
+    const double rs = rsqrt(T);
+    u = c[0] * (rs * rs);
+    w = c[L2G_RYS_ND] * rs;
+    return;
+  }
+  const double x = 2.0 * (T - (double)iv) - 1.0;
+  const double2* __restrict__ c2 = reinterpret_cast<const double2*>(c);
+  double2 a[L2G_RYS_ND];
+#pragma unroll
+  for (int k = 0; k < L2G_RYS_ND; ++k) a[k] = c2[k];
+  double p = a[L2G_RYS_ND / 2 - 1].y, q = a[L2G_RYS_ND - 1].y;
+#pragma unroll
+  for (int k = L2G_RYS_ND / 2 - 1; k >= 0; --k) {
+    if (k < L2G_RYS_ND / 2 - 1) {
+      p = fma(p, x, a[k].y);
+      q = fma(q, x, a[L2G_RYS_ND / 2 + k].y);
+    }
+    p = fma(p, x, a[k].x);
+    q = fma(q, x, a[L2G_RYS_ND / 2 + k].x);
+  }
+  u = p;
+  w = q;
+}
+
+// One primitive quartet as a Rys kernel's root stage leaves it in LDS: per
+// axis PA, QC, WP, WQ, then 1/2z, rho/2z^2, 1/2e, rho/2e^2, 1/2(z+e).
+#define L2G_RYS_REC 17
+
+// Shell quartet of a work item (LDS, one per quartet of the block).
+struct RysItem {
+  int pb0, pk0, npk, pbeg, pend, bp, kp, meta;
+  int qi;       // index in the work list, -1 past its end
+  int nsurv;    // non-zero once a primitive quartet survived the screening
+  double lnprec, qprec, npbk;
+};
+
+// The work items of a block of Q slots.  The list is sorted by decreasing
+// primitive count and its first rys_deep[0] items take min(16, Q) slots each,
+// the next rys_deep[1] min(4, Q), the rest one: a deep quartet's primitive
+// loop would otherwise run serially on one slot while the chip drains, and
+// its sums are shorter.  The share depends on the quartet alone
+// (rys_tier_of), so its bits do not depend on the batch it is in.
+template <int Q>
+struct RysTier {
+  static constexpr int S0 = Q < 16 ? Q : 16, S1 = Q < 4 ? Q : 4;
+  int S, NI, first, end;
+  static __host__ __device__ int ceil_div(int a, int b) { return (a + b - 1) / b; }
+  static int blocks(const L2gEriArgs& A) {
+    const int a = A.rys_deep[0], b = A.rys_deep[1];
+    return ceil_div(a, Q / S0) + ceil_div(b, Q / S1) + ceil_div(A.n - a - b, Q);
+  }
+  __device__ __forceinline__ RysTier(const L2gEriArgs& A, int blk) {
+    const int a = A.rys_deep[0], b = A.rys_deep[1], na = ceil_div(a, Q / S0), nb = ceil_div(b, Q / S1);
+    if (blk < na) {
+      S = S0, NI = Q / S0, first = blk * NI, end = a;
+    } else if (blk < na + nb) {
+      S = S1, NI = Q / S1, first = a + (blk - na) * NI, end = a + b;
+    } else {
+      S = 1, NI = Q, first = a + b + (blk - na - nb) * Q, end = A.n;
+    }
+  }
+};
+
+// Primitive quartet p of an item (act false: a stand-in that contributes
+// nothing): screening as the per-lane kernels do it, the record (rec, by the
+// lane of root 0) and node and weight of root r.
+template <int NR>
+__device__ __forceinline__ void rys_prim(const L2gEriArgs& A, RysItem& I, int p, int r, double* rec, double* uw,
+                                         const double* __restrict__ tab) {
+  const bool act = p < I.pend;
+  const int ib = act ? p / I.npk : 0;
+  const int gb = act ? I.pb0 + ib : 0, gk = act ? I.pk0 + (p - ib * I.npk) : 0;
+  const double4 P = A.pp_P[gb], PA = A.pp_PA[gb], Q = A.pp_P[gk], QC = A.pp_PA[gk];
+  const double2 xb = A.pp_aux[gb], xk = A.pp_aux[gk];
+  const double rs = rsqrt(P.w + Q.w);
+  const double oos = rs * rs;
+  const double pf = PA.w * QC.w * rs * A.scale;
+  bool ok = act && xb.x + xk.x > I.lnprec;
+  if (A.method == L2G_SCREEN_ORIGINAL)
+    ok = ok && !(fabs(pf) < I.qprec);
+  else if (A.method == L2G_SCREEN_CONSERVATIVE)
+    ok = ok && !(fabs(pf) * fmax(1.0, A.pp_nonsph[gb] * A.pp_nonsph[gk]) * I.npbk < I.qprec);
+  const double PQx = P.x - Q.x, PQy = P.y - Q.y, PQz = P.z - Q.z;
+  const double goq = Q.w * oos, gop = P.w * oos;
+  const double rho = P.w * Q.w * oos;
+  double T = rho * (PQx * PQx + PQy * PQy + PQz * PQz), s = 1.0;
+  if (A.omega > 0) {  // erf(w r)/r: nodes s u(sT), weights sqrt(s) w(sT), s = w^2 / (w^2 + rho)
+    s = A.omega * A.omega / (A.omega * A.omega + rho);
+    T *= s;
+  }
+  double u, w;
+  rys_root<NR>(T, tab, r, u, w);
+  if (A.omega > 0) {
+    u *= s;
+    w *= sqrt(s);
+  }
+  uw[0] = u;
+  uw[1] = ok ? w * pf : 0.0;
+  if (r == 0) {
+    if (ok) I.nsurv = 1;
+    rec[0] = PA.x, rec[1] = QC.x, rec[2] = -goq * PQx, rec[3] = gop * PQx;
+    rec[4] = PA.y, rec[5] = QC.y, rec[6] = -goq * PQy, rec[7] = gop * PQy;
+    rec[8] = PA.z, rec[9] = QC.z, rec[10] = -goq * PQz, rec[11] = gop * PQz;
+    rec[12] = xb.y, rec[13] = xb.y * goq;
+    rec[14] = xk.y, rec[15] = xk.y * gop;
+    rec[16] = 0.5 * oos;
+  }
+}
+
+// Integrals of a canonical quartet with the pure flags of meta.
+__device__ __forceinline__ int rys_size(int meta, int l1, int l2, int l3, int l4) {
+  return ((meta >> 3) & 1 ? 2 * l1 + 1 : l2g_ncart(l1)) * ((meta >> 4) & 1 ? 2 * l2 + 1 : l2g_ncart(l2)) *
+         ((meta >> 5) & 1 ? 2 * l3 + 1 : l2g_ncart(l3)) * ((meta >> 6) & 1 ? 2 * l4 + 1 : l2g_ncart(l4));
+}
+
+// A canonical quartet's four shells for the digest (LDS): sizes, first
+// functions, strides in the block V[i1][i2][i3][i4], and the offsets of the
+// six shell-pair blocks 12 34 13 14 23 24 in their concatenation.
+struct RysDigest {
+  int n[4], l[4], bf[4], sv[4], off[7], nv;
+  long long mo, N;
+  double deg;
+  __device__ __forceinline__ int fn(int k, int i, int gauss) const {
+    const int m = i - l[k];  // l < 0: Cartesian, or the Standard order
+    return bf[k] + (!gauss || l[k] < 0 ? i : (m == 0 ? 0 : (m > 0 ? 2 * m - 1 : -2 * m)));
+  }
+  __device__ __forceinline__ int block(int o) const {
+    return (o >= off[1]) + (o >= off[2]) + (o >= off[3]) + (o >= off[4]) + (o >= off[5]);
+  }
+};
+__device__ __forceinline__ int rys_bi(int b) { return (0x110020 >> (4 * b)) & 3; }
+__device__ __forceinline__ int rys_bj(int b) { return (0x323231 >> (4 * b)) & 3; }
+
+__device__ __forceinline__ void rys_digest_setup(const L2gEriArgs& A, const RysItem& I, int l1, int l2, int l3, int l4,
+                                                 RysDigest& g) {
+  const int ll[4] = {l1, l2, l3, l4};
+  const int4 bf = A.q_bf[I.qi];
+  const int b[4] = {bf.x, bf.y, bf.z, bf.w};
+  int n[4];
+#pragma unroll
+  for (int k = 0; k < 4; ++k) {
+    const int pure = (I.meta >> (3 + k)) & 1;
+    n[k] = pure ? 2 * ll[k] + 1 : l2g_ncart(ll[k]);
+    g.n[k] = n[k];
+    g.l[k] = pure ? ll[k] : -1;
+    g.bf[k] = b[k];
+  }
+  g.sv[0] = n[1] * n[2] * n[3], g.sv[1] = n[2] * n[3], g.sv[2] = n[3], g.sv[3] = 1;
+  g.nv = n[0] * g.sv[0];
+  g.off[0] = 0;
+  g.off[1] = n[0] * n[1];
+  g.off[2] = g.off[1] + n[2] * n[3];
+  g.off[3] = g.off[2] + n[0] * n[2];
+  g.off[4] = g.off[3] + n[0] * n[3];
+  g.off[5] = g.off[4] + n[1] * n[2];
+  g.off[6] = g.off[5] + n[1] * n[3];
+  const L2gMatDesc md = A.mats[A.q_req ? A.q_req[I.qi] : 0];
+  g.mo = md.off, g.N = md.n;
+  g.deg = A.q_scale[I.qi];
+}
+
+// Element o of the six blocks of the density.
+__device__ __forceinline__ double rys_density(const L2gEriArgs& A, const RysDigest& g, int o) {
+  const int b = g.block(o), i = rys_bi(b), j = rys_bj(b), k = o - g.off[b];
+  const int r = k / g.n[j], c = k - r * g.n[j];
+  return A.dens[g.mo + g.fn(i, r, A.shg_gaussian) * g.N + g.fn(j, c, A.shg_gaussian)];
+}
+
+// Element o of the six blocks of a quartet's J and K contributions, from its
+// integrals V and density blocks D: J12 takes D34, K13 takes D24, and so on,
+// as compute_2body_fock digests them (tests/hartree-fock/
+// hartree-fock++.cc:1709-1743).  A lane sums one element over the two shells
+// of the partner block, so a quartet leaves one atomic per element.
+__device__ __forceinline__ void rys_digest(const L2gEriArgs& A, const RysDigest& g, int o, const double* V,
+                                           const double* D) {
+  const int b = g.block(o), i = rys_bi(b), j = rys_bj(b), k = o - g.off[b];
+  const int r = k / g.n[j], c = k - r * g.n[j];
+  const int pb = b < 2 ? 1 - b : 7 - b, pi = rys_bi(pb), pj = rys_bj(pb);
+  const int nx = g.n[pi], ny = g.n[pj], sx = g.sv[pi], sy = g.sv[pj];
+  const double* v = V + r * g.sv[i] + c * g.sv[j];
+  const double* d = D + g.off[pb];
+  double s = 0.0;
+  for (int x = 0; x < nx; ++x, v += sx, d += ny)
+    for (int y = 0; y < ny; ++y) s = fma(d[y], v[y * sy], s);
+  double* m = b < 2 ? A.jg : A.kg;
+  l2g_acc(&m[g.mo + g.fn(i, r, A.shg_gaussian) * g.N + g.fn(j, c, A.shg_gaussian)], g.deg * s, A.fx_hoff);
+}
