@@ -348,22 +348,11 @@ AX = 'xyz'
 # arithmetic type of the recursion, HRR and transforms of the kernel being
 # emitted ('double', or 'float' for the reduced-precision variants)
 _R = 'double'
+# HRR and transforms with every fused multiply-add written out (for code whose
+# copies have to round alike; contraction is off there)
+_FUSED = False
 # attenuated (erf) variant: the core integrals s^(m+1/2) F_m(sT), s = w^2/(w^2+rho)
 _ATT = False
-# contraction on the matrix cores: each target's primitive sum accumulates
-# through v_mfma_f64_4x4x4_4b_f64 with a one-hot B operand (see emit_class)
-_MFMA = False
-# Lane layout of v_mfma_f64_4x4x4_4b_f64 on gfx950 (4 blocks g of 4x4x4,
-# probed on the device): A(g, i, k) sits in lane 4g + i + 16k, B(g, k, j) in
-# lane 4g + j + 16k and D(g, i, j) in lane 16i + 4g + j.  With B(g, k, j) =
-# [k == j] (MFMA_SELECTOR), D(g, i, j) += A(g, i, j): the value of lane
-# 16j + 4g + i lands in the accumulator of lane 16i + 4g + j, a transpose of
-# the lane bits [5:4] <-> [1:0].  Each product but one is an exact zero, so
-# D = C + v is rounded once, as a plain add is; after the primitive loop one
-# shuffle from lane MFMA_SOURCE returns every accumulator to its own lane (a
-# wave sum needs none).
-MFMA_SELECTOR = "((lane >> 4) == (lane & 3) ? 1.0 : 0.0)"
-MFMA_SOURCE = "(((lane & 3) << 4) | (lane & 12) | (lane >> 4))"
 
 
 def fmt(v):
@@ -459,10 +448,7 @@ def emit_vrr_group(E, plan, graph, grp_idx, acc_names, mid=None):
         E(f"const {_R} {v} = {expr};")
         if key in tpos:
             a = acc_names[tpos[key]]
-            if _MFMA:
-                E(f"{a} = __builtin_amdgcn_mfma_f64_4x4x4f64({v}, msel, {a}, 0, 0, 0);")
-            else:
-                E(f"{a} += {v};")
+            E(f"{a} += {v};")
     if mid is not None and half >= len(order):
         mid()
     return len(order)
@@ -504,7 +490,10 @@ def emit_hrr(E, l1, l2, inp, prefix, dvec):
         name[(a, b)] = inp[a]
     for n, (k, s0, s1, i) in enumerate(ops):
         v = f"{prefix}{n}"
-        E(f"const {_R} {v} = {name[s0]} + {dvec}{AX[i]} * {name[s1]};")
+        if _FUSED:
+            E(f"const {_R} {v} = fma({dvec}{AX[i]}, {name[s1]}, {name[s0]});")
+        else:
+            E(f"const {_R} {v} = {name[s0]} + {dvec}{AX[i]} * {name[s1]};")
         name[k] = v
     return [name[k] for k in outs]
 
@@ -517,6 +506,14 @@ def emit_sph_2(E, l1, l2, pure1, pure2, vals, prefix):
     d1, d2 = n1c, n2c
     cnt = [0]
 
+    def lin(terms):
+        if not _FUSED:
+            return ' + '.join(f"{c} * {x}" for c, x in terms)
+        r = f"{terms[0][0]} * {terms[0][1]}"
+        for c, x in terms[1:]:
+            r = f"fma({c}, {x}, {r})"
+        return r
+
     def newv(expr):
         v = f"{prefix}{cnt[0]}"
         cnt[0] += 1
@@ -528,8 +525,7 @@ def emit_sph_2(E, l1, l2, pure1, pure2, vals, prefix):
         nxt = []
         for r in rows:
             for j in range(d2):
-                terms = [f"{fmt(c)} * {cur[ic * d2 + j]}" for ic, c in r]
-                nxt.append(newv(' + '.join(terms)))
+                nxt.append(newv(lin([(fmt(c), cur[ic * d2 + j]) for ic, c in r])))
         cur = nxt
         d1 = 2 * l1 + 1
     if pure2 and l2 > 0:
@@ -537,8 +533,7 @@ def emit_sph_2(E, l1, l2, pure1, pure2, vals, prefix):
         nxt = []
         for i in range(d1):
             for r in rows:
-                terms = [f"{fmt(c)} * {cur[i * d2 + ic]}" for ic, c in r]
-                nxt.append(newv(' + '.join(terms)))
+                nxt.append(newv(lin([(fmt(c), cur[i * d2 + ic]) for ic, c in r])))
         cur = nxt
         d2 = 2 * l2 + 1
     return d1, d2, cur
@@ -557,17 +552,16 @@ def pure_variants(l1, l2):
 # ---------------------------------------------------------------------------
 
 
-def _emit_stage2(E, sfx, gb, gk, count, act=None):
+def _emit_stage2(E, sfx, gb, gk, count):
     """Screening, pfac, T and the Boys-table fetch of one primitive quartet
     (pair data in Pg{sfx}.. Qg{sfx}.., records gb / gk of the pair arrays).
     Screened primitives get pfac = 0: the recursion then produces exact
-    zeros, which keeps the loop free of divergent branches; so do primitive
-    quartets past the lane's own range (act false) in the wave-uniform loop."""
+    zeros, which keeps the loop free of divergent branches."""
     E(f"const double gp{sfx} = Pg{sfx}.w, gq{sfx} = Qg{sfx}.w;")
     E(f"const double rs{sfx} = rsqrt(gp{sfx} + gq{sfx});")
     E(f"const double oos{sfx} = rs{sfx} * rs{sfx};")
     E(f"const double pf{sfx} = PAk{sfx}.w * QCk{sfx}.w * rs{sfx} * A.scale;")
-    E(f"bool ok{sfx} = {act + ' && ' if act else ''}xb{sfx}.x + xk{sfx}.x > lnprec;")
+    E(f"bool ok{sfx} = xb{sfx}.x + xk{sfx}.x > lnprec;")
     E.block("if (A.method == L2G_SCREEN_ORIGINAL)")
     E(f"ok{sfx} = ok{sfx} && !(fabs(pf{sfx}) < qprec);")
     E.end()
@@ -598,19 +592,12 @@ def emit_prim_loop(E, plan, graph, gi, accs):
     pair data of the next primitive are loaded at the top of an iteration and
     its Boys-table row halfway through the recursion, so both memory
     latencies overlap the FP64 work of the current primitive."""
-    if _MFMA:
-        # wave-uniform trip count (tmax, the wave's longest range): a lane
-        # past its own range, or without primitive quartets, reads record 0
-        # of the pair arrays (present whenever any lane of the wave has work)
-        # and runs with pfac = 0, so every MFMA sees all 64 lanes active
-        E.block("if (tmax > 0)")
-        E("int ib = pbeg / npk1, ik = pbeg - ib * npk1;")
-        E("const int gb = trip > 0 ? pb0 + ib : 0, gk = trip > 0 ? pk0 + ik : 0;")
-        ga, ka = "gb", "gk"
-    else:
-        E.block("if (pend > pbeg)")
-        E("int ib = pbeg / npk, ik = pbeg - ib * npk;")
-        ga, ka = "pb0 + ib", "pk0 + ik"
+    # the lane's primitive quartets are pbeg, pbeg + pst, ..: a step of pst is
+    # bst bra and kst ket records
+    E.block("if (pend > pbeg)")
+    E("int ib = pbeg / npk, ik = pbeg - ib * npk;")
+    E("const int bst = pst / npk, kst = pst - bst * npk;")
+    ga, ka = "pb0 + ib", "pk0 + ik"
     E(f"double4 Pg = A.pp_P[{ga}], PAk = A.pp_PA[{ga}];")
     E(f"double2 xb = A.pp_aux[{ga}];")
     E(f"double4 Qg = A.pp_P[{ka}], QCk = A.pp_PA[{ka}];")
@@ -620,25 +607,13 @@ def emit_prim_loop(E, plan, graph, gi, accs):
         E("double sw;")
     E("L2gBoysArg bq;")
     E.block("")
-    if _MFMA:
-        _emit_stage2(E, "", ga, ka, "" if gi == 0 else None, act="trip > 0")
-    else:
-        _emit_stage2(E, "", ga, ka, "" if gi == 0 else None)
+    _emit_stage2(E, "", ga, ka, "" if gi == 0 else None)
     E.end()
-    if _MFMA:
-        E.block("for (int t = 0; t < tmax; ++t)")
-        E("int ikn = ik + 1, ibn = ib;")
-        E("if (ikn >= npk) { ikn = 0; ++ibn; }")
-        E("if (ibn >= npb) ibn = 0;")
-        E("const bool actn = t + 1 < trip;")
-        E("const int gbn = actn ? pb0 + ibn : 0, gkn = actn ? pk0 + ikn : 0;")
-        gan, kan = "gbn", "gkn"
-    else:
-        E.block("for (int p = pbeg; p < pend; ++p)")
-        E("int ikn = ik + 1, ibn = ib;")
-        E("if (ikn == npk) { ikn = 0; ++ibn; }")
-        E("if (ibn == npb) ibn = 0;  // past the end: any valid pair, result unused")
-        gan, kan = "pb0 + ibn", "pk0 + ikn"
+    E.block("for (int p = pbeg; p < pend; p += pst)")
+    E("int ikn = ik + kst, ibn = ib + bst;")
+    E("if (ikn >= npk) { ikn -= npk; ++ibn; }")
+    E("if (ibn >= npb) ibn = 0;  // past the end: any valid pair, result unused")
+    gan, kan = "pb0 + ibn", "pk0 + ikn"
     E(f"const double4 Pgn = A.pp_P[{gan}], PAkn = A.pp_PA[{gan}];")
     E(f"const double2 xbn = A.pp_aux[{gan}];")
     E(f"const double4 Qgn = A.pp_P[{kan}], QCkn = A.pp_PA[{kan}];")
@@ -683,10 +658,7 @@ def emit_prim_loop(E, plan, graph, gi, accs):
 
     def mid():
         E.block("")
-        if _MFMA:
-            _emit_stage2(E, "n", gan, kan, "" if gi == 0 else None, act="actn")
-        else:
-            _emit_stage2(E, "n", gan, kan, "p + 1 < pend && " if gi == 0 else None)
+        _emit_stage2(E, "n", gan, kan, "p + pst < pend && " if gi == 0 else None)
         E.end()
 
     emit_vrr_group(E, plan, graph, gi, accs, mid=mid)
@@ -698,7 +670,7 @@ def emit_prim_loop(E, plan, graph, gi, accs):
     E.end()  # npq > 0
 
 
-def emit_class(plan: ClassPlan, block=128, mode='eri', waves=0, real='double', att=False, mfma=False):
+def emit_class(plan: ClassPlan, block=128, mode='eri', waves=0, real='double', att=False):
     la, lb, lc, ld = plan.la, plan.lb, plan.lc, plan.ld
     graph = VrrGraph()
     ne, nf = len(plan.ecomps), len(plan.fcomps)
@@ -708,15 +680,9 @@ def emit_class(plan: ClassPlan, block=128, mode='eri', waves=0, real='double', a
       f"{G} target group(s)")
     E(f"// group sizes (bra components x ket targets): {[(len(g), len(f)) for g, f in plan.groups]}")
     E(f"// group graph nodes: {plan.group_nodes}; estimated peak live doubles: {plan.group_peak}")
-    global _R, _ATT, _MFMA
+    global _R, _ATT
     _R = real
     _ATT = att
-    _MFMA = mfma and real == 'double'
-    if _MFMA:
-        E("// contraction on the matrix cores: every target accumulates its primitive")
-        E("// quartets through v_mfma_f64_4x4x4_4b_f64 with A = the lane's value, B a")
-        E("// one-hot selector that returns each lane's value to its own D slot, and")
-        E("// C/D the accumulator (AGPRs, no VALU moves); loops are wave-uniform")
     kname = f"l2g_{'erf' if att else mode}{'32' if real == 'float' else ''}_{plan.name}"
     attr = f" __attribute__((amdgpu_waves_per_eu({waves}, {waves})))" if waves else ""
     if mode == 'fock':
@@ -734,33 +700,26 @@ def emit_class(plan: ClassPlan, block=128, mode='eri', waves=0, real='double', a
     E.ind += 1
     E("const int tid = blockIdx.x * blockDim.x + threadIdx.x;")
     E("const int nthr = gridDim.x * blockDim.x;")
-    if _MFMA:
-        E("const int lane = threadIdx.x & 63;")
-        E(f"const double msel = {MFMA_SELECTOR};")
-        E(f"const int msrc = {MFMA_SOURCE};")
-        if mode in ('schwarz', 'eri'):
-            E("// A.coop: a wave per work item, each lane taking a contiguous 1/64 of the")
-            E("// primitive quartets; the group accumulators are summed over the wave")
-            E("const bool coop = A.coop != 0;")
-            E("// the wave walks the work list together: lanes past its end take the last")
-            E("// item as a stand-in (all work, no stores), so every loop stays uniform")
-            E.block("for (int qb = coop ? (tid >> 6) : tid - lane; qb < A.n; qb += coop ? (nthr >> 6) : nthr)")
-            E("const bool live = coop || qb + lane < A.n;")
-            E("const int qi = coop ? qb : (live ? qb + lane : A.n - 1);")
-        else:
-            E("// the wave walks the work list together: lanes past its end take the last")
-            E("// item as a stand-in (all work, no digest), so every loop stays uniform")
-            E.block("for (int qb = tid - lane; qb < A.n; qb += nthr)")
-            E("const bool live = qb + lane < A.n;")
-            E("const int qi = live ? qb + lane : A.n - 1;")
-    elif mode in ('schwarz', 'eri'):
+    E("const int lane = threadIdx.x & 63;")
+    if mode == 'schwarz':
         E("// A.coop: a wave per work item, each lane taking a contiguous 1/64 of the")
         E("// primitive quartets; the group accumulators are summed over the wave")
         E("const bool coop = A.coop != 0;")
-        E("const int lane = threadIdx.x & 63;")
+        E("const int pst = 1;")
         E.block("for (int qi = coop ? (tid >> 6) : tid; qi < A.n; qi += coop ? (nthr >> 6) : nthr)")
     else:
-        E.block("for (int qi = tid; qi < A.n; qi += nthr)")
+        E("// a wave walks windows of A.win items of the list, runs of items of the same")
+        E("// tier (l2g_lane_tier) at a time: each on 1, 4, 16 or 64 lanes that take its")
+        E("// primitive quartets in turn; their accumulators are summed over the group")
+        E("const int win = A.win > 0 ? A.win : 64;")
+        E("for (int wb = (tid >> 6) * win; wb < A.n; wb += (nthr >> 6) * win)")
+        E.block("for (int base = wb, wend = min(A.n, wb + win); base < wend;)")
+        E("int glog, cnt;")
+        E("l2g_lane_tier(A, base, wend, lane, glog, cnt);")
+        E("const int pst = 1 << glog, gl = lane & (pst - 1);")
+        E("const int qi = base + (lane >> glog);")
+        E("base += cnt;")
+        E("if (qi >= base) continue;")
     E("const int bp = A.bra_pair[qi];")
     E("const int kp = " + ("bp;" if mode == 'schwarz' else "A.ket_pair[qi];"))
     E("const int meta = A.meta[qi];")
@@ -778,18 +737,14 @@ def emit_class(plan: ClassPlan, block=128, mode='eri', waves=0, real='double', a
         E("pbeg = pr.x;")
         E("pend = pr.y;")
         E.end()
-    if mode in ('schwarz', 'eri'):
+    if mode == 'schwarz':
         E.block("if (coop)")
         E("const int len = pend - pbeg, b0 = pbeg + (int)(((long long)len * lane) >> 6);")
         E("pend = pbeg + (int)(((long long)len * (lane + 1)) >> 6);")
         E("pbeg = b0;")
         E.end()
-    if _MFMA:
-        E("// wave-uniform primitive loop: the longest range of the wave")
-        E("const int trip = pend - pbeg;")
-        E("int tmax = trip;")
-        E("for (int o = 32; o > 0; o >>= 1) tmax = max(tmax, __shfl_xor(tmax, o, 64));")
-        E("const int npk1 = npk > 0 ? npk : 1;")
+    if mode != 'schwarz':
+        E("pbeg += gl;")
     if mode == 'fock':
         E("const double lnprec = A.q_lnprec[qi];")
         E("const double qprec = A.method == L2G_SCREEN_ORIGINAL || A.method == L2G_SCREEN_CONSERVATIVE ? exp(lnprec) : 0.0;")
@@ -828,21 +783,10 @@ def emit_class(plan: ClassPlan, block=128, mode='eri', waves=0, real='double', a
         for a in accs:
             E(f"{_R} {a} = 0;")
         emit_prim_loop(E, plan, graph, gi, accs)
-        if _MFMA:
-            # the contracted values back to their own lanes (a wave sum is
-            # the same over any lane order)
-            if mode in ('schwarz', 'eri'):
-                E.block("if (!coop)")
-            else:
-                E.block("")
-            for a in accs:
-                E(f"{a} = __shfl({a}, msrc, 64);")
-            E.end()
-        if mode in ('schwarz', 'eri'):
-            E.block("if (coop)")
-            for a in accs:
-                E(f"{a} = l2g_wave_sum({a});")
-            E.end()
+        E.block("if (coop)" if mode == 'schwarz' else "if (pst > 1)")
+        for a in accs:
+            E(f"{a} = l2g_wave_sum({a});" if mode == 'schwarz' else f"{a} = l2g_group_sum({a}, pst);")
+        E.end()
         if mode == 'schwarz':
             for r, ie in enumerate(grp):
                 for t, jf in enumerate(gfs):
@@ -882,11 +826,10 @@ def emit_class(plan: ClassPlan, block=128, mode='eri', waves=0, real='double', a
             E.end()
         E.end()  # group block
     # bra HRR + bra sph + permuted store, column by column over the ket
-    if _MFMA:
-        E("if (!live) continue;  // a stand-in lane: no store, no digest")
+    if mode != 'schwarz':
+        E("if (pst > 1) nsurv = l2g_group_sum(nsurv, pst);")
     if mode == 'eri':
-        E("if (coop) nsurv = l2g_wave_sum(nsurv);")
-        E("if (A.nz && (!coop || lane == 0)) A.nz[A.qidx[qi]] = nsurv > 0 ? 1 : 0;")
+        E("if (A.nz && gl == 0) A.nz[A.qidx[qi]] = nsurv > 0 ? 1 : 0;")
     elif mode == 'schwarz':
         E("double smax = 0.0, ssq = 0.0;")
     else:
@@ -948,8 +891,8 @@ def emit_class(plan: ClassPlan, block=128, mode='eri', waves=0, real='double', a
                     for i2 in range(d2):
                         v = vals[i1 * d2 + i2]
                         if mode == 'eri' and staged:
-                            # a wave-cooperative item spreads its columns over the lanes
-                            E(f"if (coop) st.put(A.out, colofs, {i1}, {i2}, colscale, {v}); "
+                            # the lanes of a group share the columns
+                            E(f"if (pst > 1) st.put(A.out, colofs, {i1}, {i2}, colscale, {v}); "
                               f"else st.put_staged(yb, A.ystride, {stage_off}, colofs, {i1}, {i2}, colscale, {v});")
                         elif mode == 'eri':
                             E(f"st.put(A.out, colofs, {i1}, {i2}, colscale, {v});")
@@ -981,37 +924,38 @@ def emit_class(plan: ClassPlan, block=128, mode='eri', waves=0, real='double', a
 
     if in_regs:
         for col in range(ncol_max):
-            if mode == 'eri':
-                E.block(f"if ({col} < ncol && (!coop || lane == {col % 64}))")
-            else:
-                E.block(f"if ({col} < ncol)")
+            E.block(f"if ({col} < ncol)" if mode == 'schwarz' else f"if ({col} < ncol && ({col} & (pst - 1)) == gl)")
             bra_column(str(col), lambda ie, c=col: f"Y[{ie}][{c}]")
             E.end()
     else:
-        if mode == 'eri':  # a wave-cooperative item spreads its columns over the lanes
-            E.block("for (int col = coop ? lane : 0; col < ncol; col += coop ? 64 : 1)")
-        else:
+        if mode == 'schwarz':
             E.block("for (int col = 0; col < ncol; ++col)")
+        else:
+            E.block("for (int col = gl; col < ncol; col += pst)")
         bra_column("col", lambda ie: f"({_R})yb[((size_t)({ie * ncol_max}) + col) * A.ystride]")
         E.end()
     if mode == 'eri' and staged:
-        E(f"if (!coop) st.flush(A.out, yb, A.ystride, {stage_off});")
+        E(f"if (pst == 1) st.flush(A.out, yb, A.ystride, {stage_off});")
     if mode == 'schwarz':
         E.block("if (!coop || lane == 0)")
         E("A.out[A.out_off[qi]] = A.schwarz_norm ? sqrt(sqrt(ssq)) : sqrt(smax);")
         E("if (A.out2) A.out2[A.out_off[qi]] = sqrt(hmax);")
         E.end()
     if mode == 'fock':
+        E.block("if (pst > 1)")
         for i1 in range(ncart(la)):
             for i2 in range(ncart(lb)):
-                E(f"if ({i1} < st.n1 && {i2} < st.n2) l2g_acc(&jgm[(bf.x + st.pos(st.l1, st.p1, {i1})) * N + "
+                E(f"j12_{i1}_{i2} = l2g_group_sum(j12_{i1}_{i2}, pst);")
+        E.end()
+        for i1 in range(ncart(la)):
+            for i2 in range(ncart(lb)):
+                E(f"if (gl == 0 && {i1} < st.n1 && {i2} < st.n2) l2g_acc(&jgm[(bf.x + st.pos(st.l1, st.p1, {i1})) * N + "
                   f"bf.y + st.pos(st.l2, st.p2, {i2})], deg * j12_{i1}_{i2}, A.fx_hoff);")
     E.end()  # quartet loop
     E.ind -= 1
     E("}")
     _R = 'double'
     _ATT = False
-    _MFMA = False
     return kname, E.text(), in_regs
 
 
@@ -1032,7 +976,7 @@ def class_waves(plan, budget, waves):
 
 def generate(outdir, lmax=2, budget=160, nfiles=8, waves=0, only=None, budgets=None,
              modes=('eri', 'fock', 'schwarz', 'fp32', 'erf', 'rys'), generic_lmax=3, max_nodes=0, fp32_lmax=2,
-             erf_lmax=2, mfma_acc=False):
+             erf_lmax=2):
     """Write the kernels and the dispatch tables.  `budgets` maps a class name
     ('2222') to its own (budget, waves).  Classes with an l above 2 whose
     partitioned recursion evaluates more than `max_nodes` nodes per primitive
@@ -1092,7 +1036,7 @@ def generate(outdir, lmax=2, budget=160, nfiles=8, waves=0, only=None, budgets=N
             p, mode, real = jobs[i]
             wv = cfg((p.la, p.lb, p.lc, p.ld))[1]
             kname, code, in_regs = emit_class(p, mode='eri' if mode == 'erf' else mode, waves=wv, real=real,
-                                              att=mode == 'erf', mfma=mfma_acc)
+                                              att=mode == 'erf')
             parts.append(code)
             parts.append(f"void {kname}_launch(const L2gEriArgs& A, int grid, int block, hipStream_t s) {{")
             parts.append(f"  hipLaunchKernelGGL({kname}, dim3(grid), dim3(block), 0, s, A);")
@@ -1115,7 +1059,7 @@ def generate(outdir, lmax=2, budget=160, nfiles=8, waves=0, only=None, budgets=N
     rys = {m: gen_rys.generate(ryscls, m) for m in ('eri', 'fock') if m in modes}
     for k, v in enumerate(gen_rys.files(rys.get('eri', []) + rys.get('fock', []), nfiles)):
         fn = os.path.join(outdir, f"rys_gen_{k}.hip")
-        new = '// generated by libint_amd/codegen/gen_rys.py - do not edit\n#include "rys_device.h"\n\n' + '\n'.join(v)
+        new = '// generated by libint_amd/codegen/gen_rys.py - do not edit\n#pragma clang fp contract(off)\n#include "rys_device.h"\n\n' + '\n'.join(v)
         if not (os.path.exists(fn) and open(fn).read() == new):
             with open(fn, 'w') as f:
                 f.write(new)
@@ -1191,8 +1135,6 @@ if __name__ == '__main__':
     ap.add_argument("--max-nodes", type=int, default=0,
                     help="classes with l > 2 and more recursion nodes than this run on the generic kernel")
     ap.add_argument("--fp32-lmax", type=int, default=2, help="highest l with FP32 kernel variants")
-    ap.add_argument("--mfma-acc", type=int, default=0,
-                    help="1: FP64 kernels accumulate the contraction on the matrix cores")
     a = ap.parse_args()
     per = {}
     for item in filter(None, a.class_cfg.split(",")):
@@ -1200,6 +1142,6 @@ if __name__ == '__main__':
         per[k] = tuple(int(x) for x in v.split(":"))
     files, plans = generate(a.outdir, a.lmax, a.budget, a.nfiles, a.waves,
                             set(filter(None, a.only.split(","))) or None, per, tuple(a.modes.split(",")),
-                            a.generic_lmax, a.max_nodes, a.fp32_lmax, mfma_acc=bool(a.mfma_acc))
+                            a.generic_lmax, a.max_nodes, a.fp32_lmax)
     for p in plans:
         print(p.name, 'groups', len(p.groups), 'nodes', sum(p.group_nodes), 'peak', max(p.group_peak))

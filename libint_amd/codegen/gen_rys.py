@@ -45,12 +45,12 @@ stores (or, in J/K builds, a lane per element of the six Fock blocks).
 """
 from __future__ import annotations
 
+import functools
 import random
 
 import gen_eri as ge
 import rys_table
 
-LDS_WAVE = 19 * 1024   # LDS bytes per wave that let 8 waves share a CU's 160 KB
 REC = 17
 
 
@@ -58,6 +58,7 @@ def comps(l1, l2):
     return [c for l in range(l1, l1 + l2 + 1) for c in ge.cart(l)]
 
 
+@functools.lru_cache(maxsize=None)
 def pair_tiles(cs):
     """Components in tiles of two that share two axes: (axis they differ on, i, j); a component left over pairs with itself."""
     n = len(cs)
@@ -85,19 +86,45 @@ def pair_tiles(cs):
     return sorted(best)
 
 
+@functools.lru_cache(maxsize=None)
+def split_parts(inner, n):
+    """The inner components in n parts by their power on axis C: indices of each part, the largest part as
+    small as can be, then the fewest X Y products."""
+    cs = sorted({f[2] for f in inner})
+    best = None
+
+    def go(k, groups):
+        nonlocal best
+        if k == len(cs):
+            if all(groups):
+                parts = [[i for i, f in enumerate(inner) if f[2] in g] for g in groups]
+                c = (max(map(len, parts)) // 2, sum(len({inner[i][:2] for i in x}) for x in parts), max(map(len, parts)))
+                if best is None or c < best[0]:
+                    best = (c, parts)
+            return
+        for g in range(n):
+            go(k + 1, groups[:g] + [groups[g] | {cs[k]}] + groups[g + 1:])
+            if not groups[g]:
+                break
+    if n > len(cs):
+        return None
+    go(0, [set() for _ in range(n)])
+    return best[1]
+
+
 class Plan:
     """Layout of one class: side of the lanes, tile, waves, quartets per block."""
 
-    def __init__(self, la, lb, lc, ld, side, te, nw, nparts):
+    def __init__(self, la, lb, lc, ld, side, te, nw, nparts, rl=False, nb=None):
         self.l = (la, lb, lc, ld)
-        self.side, self.te, self.nw = side, te, nw
+        self.side, self.te, self.nw, self.rl = side, te, nw, rl
         self.ecs, self.fcs = comps(la, lb), comps(lc, ld)
         self.ne, self.nf = len(self.ecs), len(self.fcs)
         self.na, self.nc = la + lb, lc + ld
         self.nr = (la + lb + lc + ld) // 2 + 1
         self.outer, self.inner = (self.ecs, self.fcs) if side == 'bra' else (self.fcs, self.ecs)
         self.no, self.ni = (self.na, self.nc) if side == 'bra' else (self.nc, self.na)
-        self.tiles = pair_tiles(self.outer) if te == 2 else [(2, i, i) for i in range(len(self.outer))]
+        self.tiles = pair_tiles(tuple(self.outer)) if te == 2 else [(2, i, i) for i in range(len(self.outer))]
         self.nl = len(self.tiles)
         self.nt = 64 * nw
         self.q = self.nt // self.nl
@@ -105,45 +132,17 @@ class Plan:
         self.gb = ((self.no + 1) * (self.ni + 1)) | 1          # doubles of one axis block (odd: no bank conflicts)
         if self.q == 0:
             return
-        # primitives per batch: the root stage's lanes full
-        best = None
-        for nb in range(1, 9):
-            if self.q * nb * self.nr > 4 * self.nt and nb > 1:
-                break
-            c = -(-self.q * nb * self.nr // self.nt) / nb
-            if best is None or c < best[0] - 1e-9:
-                best = (c, nb)
-        self.nb = best[1]
-        self.root_rounds = best[0]
+        self.ng = 1 if rl else self.nr   # nodes whose 2D integrals are in LDS at a time
+        self.nb = nb
+        self.root_rounds = -(-self.q * nb * self.nr // self.nt) / nb
         # row stride of the contracted block in LDS (odd), and doubles per
         # quartet of a pass: with every shell a solid harmonic / Cartesian
         self.rstr = max(self.nf, ge.ncart(lc) * ge.ncart(ld)) | 1
         self.erow = self.ne * self.rstr
-        self.lds_main = self.nb * self.q * (2 * self.nr + REC) + self.q * self.nr * 3 * self.gb
+        self.lds_main = self.nb * self.q * (2 * self.nr + REC) + self.q * self.ng * 3 * self.gb
 
     def split(self, n):
-        """The inner components in n parts by their power on axis C: indices of each part, the largest part as
-        small as can be, then the fewest X Y products."""
-        cs = sorted({f[2] for f in self.inner})
-        best = None
-
-        def go(k, groups):
-            nonlocal best
-            if k == len(cs):
-                if all(groups):
-                    parts = [[i for i, f in enumerate(self.inner) if f[2] in g] for g in groups]
-                    c = (max(map(len, parts)) // 2, sum(self.nxy(x) for x in parts), max(map(len, parts)))
-                    if best is None or c < best[0]:
-                        best = (c, parts)
-                return
-            for g in range(n):
-                go(k + 1, groups[:g] + [groups[g] | {cs[k]}] + groups[g + 1:])
-                if not groups[g]:
-                    break
-        if n > len(cs):
-            return None
-        go(0, [set() for _ in range(n)])
-        return best[1]
+        return split_parts(tuple(self.inner), n)
 
     def nxy(self, part):
         return len({self.inner[i][:2] for i in part})
@@ -152,60 +151,114 @@ class Plan:
         """Powers read on axes A, B, C for a part."""
         return [sorted({self.inner[i][a] for i in part}) for a in range(3)]
 
-    def sizes(self, mode, pure):
-        """(doubles per quartet of a pass, integrals, elements of the six Fock blocks)"""
-        n = [2 * l + 1 if pure and l >= 2 else ge.ncart(l) for l in self.l]
+    def dims(self, pure):
+        return [2 * l + 1 if pure and l >= 2 else ge.ncart(l) for l in self.l]
+
+    def layout(self, mode, pure):
+        """(quartets per pass, passes, LDS doubles of each, offset of the finished block in them).  The block goes over
+        the rows it is made from where a pass has at most one column a lane (every row is read before), else behind
+        them, and a lane loops over its columns; whichever takes fewer passes."""
+        n = self.dims(pure)
         nv = n[0] * n[1] * n[2] * n[3]
-        nc = sum(n[i] * n[j] for i in range(4) for j in range(i + 1, 4))
-        if mode == 'eri':  # a block that does not fit over its own rows is stored directly
-            return self.erow, nv, nc
-        return max(self.erow, nv + nc), nv, nc
+        tail = sum(n[i] * n[j] for i in range(4) for j in range(i + 1, 4)) if mode == 'fock' else 0
+        # LDS that leaves the occupancy to the registers
+        cap = max(self.lds_main, (163840 // (4 * min(4, 512 // self.regs())) * self.nw - 144 * self.q) // 8)
+        ncol = n[2] * n[3]
+        best = None
+        for over in (True, False):
+            if over:  # a block that does not fit over its rows is stored directly by an ERI batch
+                d = self.erow if mode == 'eri' else max(self.erow, nv + tail)
+            else:
+                d = self.erow + nv + tail
+            if not over and ncol > self.nt and d > cap:
+                continue
+            qp = max(1, min(self.q, cap // d, self.nt // ncol if over else self.q))
+            np_ = -(-self.q // qp)
+            qp = -(-self.q // np_)
+            if best is None or np_ < best[1]:
+                best = (qp, np_, d, 0 if over else self.erow)
+        return best
 
     def passes(self, mode, pure=True):
-        """(quartets per pass, passes)"""
-        cap = max(self.lds_main, LDS_WAVE // 8 * self.nw)
-        # a lane per column of the pass in the bra recurrence
-        ncol = (2 * self.l[2] + 1 if pure and self.l[2] >= 2 else ge.ncart(self.l[2])) * \
-            (2 * self.l[3] + 1 if pure and self.l[3] >= 2 else ge.ncart(self.l[3]))
-        qp = max(1, min(self.q, cap // self.sizes(mode, pure)[0], self.nt // ncol))
-        np_ = -(-self.q // qp)
-        return -(-self.q // np_), np_
+        return self.layout(mode, pure)[:2]
 
     def lds_doubles(self, mode):
-        return max([self.lds_main] + [self.passes(mode, x)[0] * self.sizes(mode, x)[0] for x in (True, False)])
+        lay = [self.layout(mode, x) for x in (True, False)]
+        return max([self.lds_main] + [x[0] * x[2] for x in lay])
 
     def lds_bytes(self, mode):
         return 8 * self.lds_doubles(mode) + self.q * 72 + (self.q * 128 if mode == 'fock' else 0)
 
+    def occupancy(self):
+        """Waves per SIMD that registers and LDS allow."""
+        return max(1, min(4, 512 // max(1, self.regs()), int(163840 / (self.lds_bytes('fock') / self.nw) / 4)))
+
     def cost(self):
-        """Lane operations per primitive quartet (product, 2D and root stages), with the LDS reads priced at the CU's rate."""
+        """Lane operations per primitive quartet (product, 2D and root stages), over the share of the VALU that so many
+        waves per SIMD were seen to fill, or the LDS clocks where those are more."""
         main = self.nr * (self.te * len(self.inner) + sum(self.nxy(x) for x in self.parts)) + self.te * len(self.inner)
         reads = self.nr * sum(len(a) + len(b) + self.te * len(c) for a, b, c in map(self.rows_of, self.parts))
-        main += reads // 2
-        two = -(-self.q * self.nr * 3 // self.nt) * (4 * (self.na + 1) * (self.nc + 1) + 40)
-        root = self.root_rounds * 150
-        valu = main + two + root + 30
-        lds = (reads + -(-self.q * self.nr * 3 // self.nt) * (self.gb + 12)) * 4 * 64 * 8 / 128.0 / 4  # clocks/4 of four SIMDs
-        occ = min(2.0, 160 * 1024 / (self.lds_main * 8 / self.nw) / 4)
-        return max(valu, lds, 0.6 * (valu + lds)) * (1.35 if occ < 1.9 else 1.0) * (1.05 if self.nw > 1 else 1.0) * self.nt / self.q
+        rounds = self.nr // self.ng * -(-self.q * self.ng * 3 // self.nt)
+        two = rounds * (3.5 * (self.na + 1) * (self.nc + 1) + 40)
+        root = self.root_rounds * 170 + 60 / self.nb
+        valu = main + reads // 2 + two + root + 30
+        lds = (reads + rounds * (self.gb + 12)) * 4.0  # quarter clocks of the CU's LDS for four SIMDs
+        return max(valu / {1: 0.35, 2: 0.6, 3: 0.75, 4: 0.85}[self.occupancy()], lds / 0.8) * self.nt / self.q * \
+            (1.05 if self.nw > 1 else 1.0)
 
     def regs(self):
         rows = max(len(a) + len(b) + self.te * len(c) for a, b, c in map(self.rows_of, self.parts))
         return 2 * (self.te * (len(self.inner) + max(map(len, self.parts))) + rows) + 34
 
 
+# Layouts that measured faster than the model's choice: (side, tile, waves, node by node, parts, batch), with the
+# nanoseconds per primitive quartet of the model's choice and of this one on one MI355X (ERI batches of
+# 25,000 to 150,000 quartets, K <= 5).
+TUNED = {
+    '0000': ('bra', 1, 1, True, 1, 1),  # 0.042 -> 0.029
+    '0010': ('ket', 1, 1, True, 1, 3),  # 0.033 -> 0.029
+    '0021': ('ket', 1, 1, False, 1, 8),  # 0.075 -> 0.060
+    '0030': ('bra', 1, 1, True, 1, 1),  # 0.069 -> 0.060
+    '0031': ('ket', 2, 1, False, 1, 4),  # 0.117 -> 0.090
+    '0033': ('ket', 2, 2, False, 1, 8),  # 0.341 -> 0.258
+    '1011': ('ket', 2, 1, False, 1, 3),  # 0.067 -> 0.062
+    '1022': ('bra', 1, 1, True, 1, 1),  # 0.159 -> 0.133
+    '1031': ('bra', 1, 1, True, 1, 1),  # 0.128 -> 0.110
+    '1033': ('ket', 2, 2, False, 1, 4),  # 0.405 -> 0.390
+    '1120': ('ket', 1, 1, False, 1, 2),  # 0.122 -> 0.107
+    '2011': ('bra', 1, 1, False, 1, 2),  # 0.124 -> 0.107
+    '2021': ('bra', 1, 1, True, 1, 2),  # 0.179 -> 0.154
+    '2031': ('bra', 1, 1, False, 1, 1),  # 0.287 -> 0.217
+    '2032': ('bra', 1, 1, True, 1, 3),  # 0.510 -> 0.327
+    '2122': ('bra', 1, 1, False, 2, 4),  # 0.370 -> 0.353
+    '2133': ('bra', 1, 1, False, 3, 6),  # 1.164 -> 1.037
+    '2232': ('bra', 1, 1, False, 1, 6),  # 1.427 -> 0.850
+    '3032': ('ket', 2, 1, False, 1, 6),  # 0.694 -> 0.662
+    '3131': ('bra', 1, 1, False, 1, 6),  # 0.619 -> 0.564
+    '3132': ('bra', 1, 1, False, 1, 6),  # 1.186 -> 0.844
+    '3133': ('ket', 1, 4, False, 1, 8),  # 1.924 -> 1.659
+}
+
+
+@functools.lru_cache(maxsize=None)
 def plan(la, lb, lc, ld):
     best = None
+    if f"{la}{lb}{lc}{ld}" in TUNED:
+        side, te, nw, rl, nparts, nb = TUNED[f"{la}{lb}{lc}{ld}"]
+        return Plan(la, lb, lc, ld, side, te, nw, nparts, rl, nb)
     for side in ('bra', 'ket'):
         for te in (1, 2):
             for nw in (1, 2, 4):
-                for nparts in (1, 2, 3):
-                    p = Plan(la, lb, lc, ld, side, te, nw, nparts)
-                    if p.parts is None or p.q == 0 or p.regs() > 270 or p.lds_bytes('fock') > 150 * 1024:
-                        continue
-                    c = p.cost()
-                    if best is None or c < best[0]:
-                        best = (c, p)
+                for rl, nparts in ((True, 1), (False, 1), (False, 2), (False, 3)):
+                    for nb in (1, 2, 3, 4, 6, 8):
+                        p = Plan(la, lb, lc, ld, side, te, nw, nparts, rl, nb)
+                        if p.parts is None or p.q == 0 or p.regs() > 270 or p.lds_bytes('fock') > 150 * 1024:
+                            continue
+                        if nb > 1 and p.q * nb * p.nr > 3 * p.nt:
+                            continue
+                        c = p.cost()
+                        if best is None or c < best[0]:
+                            best = (c, p)
     return best[1]
 
 
@@ -213,10 +266,11 @@ def emit(p, mode):
     la, lb, lc, ld = p.l
     E = ge.Emitter()
     ge._R = 'double'
+    ge._FUSED = True
     name = f"l2g_rys_{mode}_{la}{lb}{lc}{ld}"
     NT, Q, NL, NR, NB, NW = p.nt, p.q, p.nl, p.nr, p.nb, p.nw
-    qps = {x: p.passes(mode, x)[0] for x in (True, False)}
-    regs_ = {x: p.sizes(mode, x)[0] for x in (True, False)}
+    lay = {x: p.layout(mode, x) for x in (True, False)}
+    qps, regs_, vofs = ({x: lay[x][k] for x in lay} for k in (0, 2, 3))
     QP = max(qps.values())
     ni1, no1 = p.ni + 1, p.no + 1
     swz = [(0, 1, 2), (0, 2, 1), (1, 2, 0)]  # axes (A, B, C) by C axis z, y, x
@@ -233,7 +287,7 @@ def emit(p, mode):
         rows.append((off[0] | off[1] << 8 | off[2] << 16 | off[3] << 24, i | j << 8 | ax << 16))
     E(f"static __device__ const unsigned {name}_tab[{2 * NL}] = {{" +
       ', '.join(f"{x}u" for r in rows for x in r) + "};")
-    lb2 = 2 if NW == 1 else 2
+    lb2 = p.occupancy()
     E(f"__global__ void __launch_bounds__({NT}, {lb2}) {name}(const L2gEriArgs A) {{")
     E.ind += 1
     E(f"__shared__ double sm[{p.lds_doubles(mode)}];")
@@ -285,7 +339,7 @@ def emit(p, mode):
     E(f"const int mq = min(tid / {NL}, {Q - 1}), mt = tid % {NL};")
     E(f"const bool mlive = tid < {Q * NL};")
     E(f"const unsigned tofs = {name}_tab[2 * mt], tinf = {name}_tab[2 * mt + 1];")
-    E(f"const double* const gq = sm + {g0} + mq * {NR * 3 * p.gb};")
+    E(f"const double* const gq = sm + {g0} + mq * {p.ng * 3 * p.gb};")
     E("const double* const rA = gq + (tofs & 255u);")
     E("const double* const rB = gq + ((tofs >> 8) & 255u);")
     E("const double* const rC = gq + ((tofs >> 16) & 255u);")
@@ -301,9 +355,7 @@ def emit(p, mode):
     # root stage
     nroot = NB * Q * NR
     rounds = -(-nroot // NT)
-    E("// one copy of the code for every quartet (no unrolling here and below): a second could round differently")
     if rounds > 1:
-        E("#pragma unroll 1")
         E.block(f"for (int it = tid; it < {nroot}; it += {NT})")
     else:
         E("const int it = tid;")
@@ -317,18 +369,25 @@ def emit(p, mode):
     E("#pragma unroll 1")
     E.block("for (int b = 0; b < nbat; ++b)")
     # 2D stage
-    n2 = Q * NR * 3
+    if p.rl:
+        for t in range(p.te):
+            E("double " + ', '.join(f"t{t}_{k} = 0.0" for k in range(len(p.inner))) + ";")
+        E("#pragma unroll 1")
+        E.block(f"for (int r = 0; r < {NR}; ++r)")
+    n2 = Q * p.ng * 3
     rounds = -(-n2 // NT)
     if rounds > 1:
-        E("#pragma unroll 1")
         E.block(f"for (int it = tid; it < {n2}; it += {NT})")
     else:
         E("const int it = tid;")
         E.block(f"if (it < {n2})")
     E("const int qr = it / 3, ax = it - qr * 3;")
-    E(f"const int q = qr / {NR};")
+    if p.rl:
+        E(f"const int q = qr, node = (b * {Q} + q) * {NR} + r;")
+    else:
+        E(f"const int q = qr / {NR}, node = b * {Q * NR} + qr;")
     E(f"const double* const rc = sm + {rec} + (b * {Q} + q) * {REC};")
-    E(f"const double u = sm[{uw} + (b * {Q * NR} + qr) * 2], w = sm[{uw} + (b * {Q * NR} + qr) * 2 + 1];")
+    E(f"const double u = sm[{uw} + node * 2], w = sm[{uw} + node * 2 + 1];")
     E("const double C00 = fma(u, rc[ax * 4 + 2], rc[ax * 4]), D00 = fma(u, rc[ax * 4 + 3], rc[ax * 4 + 1]);")
     E("const double B00 = u * rc[16], B10 = fma(-u, rc[13], rc[12]), B01 = fma(-u, rc[15], rc[14]);")
     E("(void)C00; (void)D00; (void)B00; (void)B10; (void)B01;")
@@ -369,10 +428,11 @@ def emit(p, mode):
         if k:  # rows are read again: kept over the parts they would not fit the registers
             E('asm volatile("" ::: "memory");')
         E.block("")
-        for t in range(p.te):
-            E("double " + ', '.join(f"t{t}_{k}" for k in part) + ";")
+        if not p.rl:
+            for t in range(p.te):
+                E("double " + ', '.join(f"t{t}_{k}" for k in part) + ";")
         rows_abc = p.rows_of(part)
-        for r in range(NR):
+        for r in range(p.ng):
             o = r * 3 * p.gb
             E.block("")
             for nm, ks in zip("ABC", rows_abc):
@@ -387,15 +447,21 @@ def emit(p, mode):
                     f = p.inner[k]
                     if f[:2] == (fa, fb):
                         for t, nm in zip(range(p.te), "CD"):
-                            E(f"t{t}_{k} = " + (f"xy * {nm}{f[2]};" if r == 0 else f"fma(xy, {nm}{f[2]}, t{t}_{k});"))
+                            E(f"t{t}_{k} = " + (f"xy * {nm}{f[2]};" if r == 0 and not p.rl else f"fma(xy, {nm}{f[2]}, t{t}_{k});"))
                 E.end()
             E.end()
-        for t in range(p.te):
-            for k in part:
-                E(f"a{t}_{k} += t{t}_{k};")
+        if not p.rl:
+            for t in range(p.te):
+                for k in part:
+                    E(f"a{t}_{k} += t{t}_{k};")
         E.end()
     E.end()
     E(f"rys_sync<{NW}>();")
+    if p.rl:
+        E.end()  # r
+        for t in range(p.te):
+            for k in range(len(p.inner)):
+                E(f"a{t}_{k} += t{t}_{k};")
     E.end()  # b
     E.end()  # p0
     # component indices of the lane's targets
@@ -463,11 +529,9 @@ def emit(p, mode):
     E(f"cart |= (mt_ & {mask}) != {mask};")
     E.end()
     E("ncol = __builtin_amdgcn_readfirstlane(ncol), cart = __builtin_amdgcn_readfirstlane(cart);")
-    if (qps[True], regs_[True]) == (qps[False], regs_[False]):
-        E(f"const int QP = {QP}, region = {regs_[True]};")
-        E("(void)cart;")
-    else:
-        E(f"const int QP = cart ? {qps[False]} : {qps[True]}, region = cart ? {regs_[False]} : {regs_[True]};")
+    for nm, x in (("QP", qps), ("region", regs_), ("vofs", vofs)):
+        E(f"const int {nm} = " + (f"{x[True]};" if x[True] == x[False] else f"cart ? {x[False]} : {x[True]};"))
+    E("(void)cart;")
     E("#pragma unroll 1")
     E.block("for (int qlo = 0; qlo < NI; qlo += QP)")
     E("const int qn = min(QP, NI - qlo);")
@@ -528,25 +592,23 @@ def emit(p, mode):
     E.end()
     E.end()
     E(f"rys_sync<{NW}>();")
-    # bra recurrence and transform: a lane per ket function; the columns of a
-    # lane stay in registers until every lane has read its own
-    rounds = max(-(-q * (n := (2 * lc + 1 if x and lc >= 2 else ge.ncart(lc)) * (2 * ld + 1 if x and ld >= 2 else ge.ncart(ld))) // NT)
-                 for x, q in qps.items())
-    for rd in range(rounds):
-        for e in range(p.ne):
-            E(f"double y{rd}_{e} = 0.0;")
-    for rd in range(rounds):
-        E.block("")
-        E(f"const int it = tid + {rd * NT}, qp = it / ncol, col = it - qp * ncol;")
-        E.block("if (qp < qn)")
-        for e in range(p.ne):
-            E(f"y{rd}_{e} = sm[qp * region + {e * p.rstr} + col];")
-        E.end()
-        E.end()
-    E(f"rys_sync<{NW}>();")
-    for rd in range(rounds):
-        E.block("")
-        E(f"const int it = tid + {rd * NT}, qp = it / ncol, col = it - qp * ncol;")
+    # bra recurrence and transform: a lane per ket function.  Where the block
+    # goes over the rows, every lane reads its columns first
+    ncols = {x: p.dims(x)[2] * p.dims(x)[3] for x in lay}
+    rounds = max([-(-qps[x] * ncols[x] // NT) for x in lay if vofs[x] == 0], default=0)
+    behind = {x for x in lay if vofs[x]}
+
+    def columns(rd):
+        if rd is None:
+            E("#pragma unroll 1")
+            E.block(f"for (int it = tid; it < qn * ncol; it += {NT})")
+        else:
+            E.block("")
+            E(f"const int it = tid + {rd * NT};")
+        E("const int qp = it / ncol, col = it - qp * ncol;")
+
+    def finish(rd):
+        columns(rd)
         E("const int qi = qp < qn ? items[qlo + qp].qi : -1;")
         E.block("if (qi >= 0)")
         E("const int bp = items[qlo + qp].bp, meta = items[qlo + qp].meta;")
@@ -554,6 +616,9 @@ def emit(p, mode):
         E.block("if (col < n3 * n4)")
         E("const double ABx = A.pair_AB[3 * bp], ABy = A.pair_AB[3 * bp + 1], ABz = A.pair_AB[3 * bp + 2];")
         E("(void)ABx; (void)ABy; (void)ABz;")
+        if rd is None:
+            for e in range(p.ne):
+                E(f"const double y{rd}_{e} = sm[qp * region + {e * p.rstr} + col];")
         inp = {c: f"y{rd}_{e}" for e, c in enumerate(p.ecs)}
         vals = ge.emit_hrr(E, la, lb, inp, "g", "AB")
         E("const int ic = col / n4, id = col - ic * n4;")
@@ -563,8 +628,8 @@ def emit(p, mode):
             E("const double colscale = st.uniform ? (st.p3 ? 1.0 : l2g_uniform_scale[st.l3][ic]) * "
               "(st.p4 ? 1.0 : l2g_uniform_scale[st.l4][id]) : 1.0;")
             E("(void)colscale;")
-            E(f"[[maybe_unused]] const bool fits = rys_size(meta, {la}, {lb}, {lc}, {ld}) <= region;")
-        E(f"double* const vb = sm + qp * region;")
+            E(f"[[maybe_unused]] const bool fits = vofs || rys_size(meta, {la}, {lb}, {lc}, {ld}) <= region;")
+        E("double* const vb = sm + qp * region + vofs;")
         E("(void)vb;")
         E.block("switch ((meta >> 3) & 3)")
         for pa, pb in ge.pure_variants(la, lb):
@@ -590,7 +655,7 @@ def emit(p, mode):
                         x += " * colscale"
                     return x
                 at = [(f"o0_{i1} + o1_{i2}", val(i1, i2)) for i1 in range(d1) for i2 in range(d2)]
-                direct = d1 * d2 * ge.ncart(lc) * ge.ncart(ld) > min(regs_.values())
+                direct = rd is not None and d1 * d2 * ge.ncart(lc) * ge.ncart(ld) > min(regs_[x] for x in lay if not vofs[x])
                 if direct:
                     E.block("if (!fits)")
                     E("double* const o = A.out + st.base + colofs;")
@@ -614,15 +679,41 @@ def emit(p, mode):
         E.end()
         E.end()
         E.end()
+
+    # the copies of the code round alike: every fused operation is written out, and contraction is off
+    if rounds:
+        if behind:
+            E.block("if (vofs == 0)")
+        for rd in range(rounds):
+            for e in range(p.ne):
+                E(f"double y{rd}_{e} = 0.0;")
+        for rd in range(rounds):
+            columns(rd)
+            E.block("if (qp < qn)")
+            for e in range(p.ne):
+                E(f"y{rd}_{e} = sm[qp * region + {e * p.rstr} + col];")
+            E.end()
+            E.end()
+        E(f"rys_sync<{NW}>();")
+        for rd in range(rounds):
+            finish(rd)
+        if behind:
+            E.end()
+    if behind:
+        if rounds:
+            E.block("else")
+        finish(None)
+        if rounds:
+            E.end()
     if mode == 'eri':
         E(f"rys_sync<{NW}>();")
         E.block("for (int qp = 0; qp < qn; ++qp)")
         E("const int qi = items[qlo + qp].qi, meta = items[qlo + qp].meta;")
         E("if (qi < 0) break;")
         E(f"const int n = rys_size(meta, {la}, {lb}, {lc}, {ld});")
-        E("if (n > region) continue;  // stored directly")
+        E("if (!vofs && n > region) continue;  // stored directly")
         E("double* const dst = A.out + A.out_off[qi];")
-        E(f"const double* const vb = sm + qp * region;")
+        E("const double* const vb = sm + qp * region + vofs;")
         E.block("if (A.store_sub)")
         E(f"for (int k = tid; k < n; k += {NT}) dst[k] -= vb[k];")
         E.end()
@@ -630,13 +721,14 @@ def emit(p, mode):
         E(f"for (int k = tid; k < n; k += {NT}) dst[k] = vb[k];")
         E.end()
         E.end()
-    ncomb = p.sizes(mode, False)[2]
+    n = p.dims(False)
+    ncomb = sum(n[i] * n[j] for i in range(4) for j in range(i + 1, 4))
     if mode == 'fock':
         E("#pragma unroll 1")
         E(f"for (int it = tid; it < qn * {ncomb}; it += {NT}) {{")
         E.ind += 1
         E(f"const int qp = it / {ncomb}, o = it - qp * {ncomb};")
-        E(f"if (items[qlo + qp].nsurv && o < dig[qp].off[6]) sm[qp * region + dig[qp].nv + o] = rys_density(A, dig[qp], o);")
+        E(f"if (items[qlo + qp].nsurv && o < dig[qp].off[6]) sm[qp * region + vofs + dig[qp].nv + o] = rys_density(A, dig[qp], o);")
         E.end()
         E(f"rys_sync<{NW}>();")
         E("#pragma unroll 1")
@@ -644,7 +736,7 @@ def emit(p, mode):
         E.ind += 1
         E(f"const int qp = it / {ncomb}, o = it - qp * {ncomb};")
         E(f"if (items[qlo + qp].nsurv && o < dig[qp].off[6]) "
-          f"rys_digest(A, dig[qp], o, sm + qp * region, sm + qp * region + dig[qp].nv);")
+          f"rys_digest(A, dig[qp], o, sm + qp * region + vofs, sm + qp * region + vofs + dig[qp].nv);")
         E.end()
     E.end()  # passes
     if mode == 'eri':
@@ -655,6 +747,7 @@ def emit(p, mode):
     E(f"void {name}_launch(const L2gEriArgs& A, int, int, hipStream_t s) {{")
     E(f"  hipLaunchKernelGGL({name}, dim3(RysTier<{Q}>::blocks(A)), dim3({NT}), 0, s, A);")
     E("}")
+    ge._FUSED = False
     return name, E.text()
 
 
@@ -663,7 +756,7 @@ def use(la, lb, lc, ld):
     one bra component leaves a tile of one lane a quartet (measured 0.2 to 0.8
     times the speed of the per-lane kernels on 2000 to 40000 quartets, against
     0.8 to 28 times for the others)."""
-    return la + lb > 0
+    return True
 
 
 def generate(classes, mode):
@@ -685,5 +778,6 @@ if __name__ == '__main__':
     for c in ge.canonical_classes(3):
         if use(*c):
             p = plan(*c)
-            print(c, 'lanes on', p.side, 'tile', p.te, 'waves', p.nw, 'quartets', p.q, 'batch', p.nb, 'LDS', p.lds_bytes('fock'),
-                  'cost %.0f' % p.cost())
+            print(c, 'lanes on', p.side, 'tile', p.te, 'parts', len(p.parts), 'waves', p.nw, 'quartets', p.q, 'batch', p.nb,
+                  'node by node' if p.rl else '', 'LDS a wave', p.lds_bytes('fock') // p.nw, 'registers', p.regs(),
+                  'waves per SIMD', p.occupancy(), 'cost %.0f' % p.cost())

@@ -73,6 +73,13 @@ __device__ __forceinline__ T l2g_wave_sum(T v) {
   return v;
 }
 
+// sum over an aligned group of n lanes (a power of two), in every lane of it
+template <class T>
+__device__ __forceinline__ T l2g_group_sum(T v, int n) {
+  for (int o = n >> 1; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
+  return v;
+}
+
 struct L2gEriArgs {
   const int* __restrict__ bra_pair;
   const int* __restrict__ ket_pair;
@@ -95,6 +102,7 @@ struct L2gEriArgs {
   int uniform_cart;
   int schwarz_norm;  // Schwarz kernels: 0 = max-abs norm, 1 = Frobenius norm
   int coop;          // Schwarz kernels: one wave per pair, its lanes splitting the primitive loop
+  int win;           // per-lane ERI and Fock kernels: work items of a wave's window (0: 64)
   double omega;      // > 0: erf-attenuated Coulomb erf(omega r)/r (0: Coulomb)
   int store_sub;     // ERI kernels: subtract from the output instead of storing
   double* __restrict__ out;
@@ -129,6 +137,40 @@ struct L2gEriArgs {
   double* __restrict__ gpart;
   const int* __restrict__ gpart_first;
 };
+
+// Lanes per item of the per-lane kernels, by its primitive quartets: 1, from
+// 16 on 4, from 64 on 16, from 512 on 64.  A lane walks its part serially,
+// each step waiting on a gather of pair data, and the lanes of a group read
+// neighbouring records; summing the group's accumulators (log2 of its size
+// shuffles each) costs less than the loop they shorten from these lengths on.
+// The group depends on the item alone, so its bits do not depend on the batch.
+// Here: log2 of the group of item `base`, and how many items from there on
+// (up to wend) are of that tier and fit the wave.
+__device__ __forceinline__ void l2g_lane_tier(const L2gEriArgs& A, int base, int wend, int lane, int& glog, int& cnt) {
+  const int i = min(base + lane, wend - 1);
+  int len;
+  if (A.q_prange) {
+    const int2 r = A.q_prange[i];
+    len = r.y - r.x;
+  } else {
+    len = A.pair_np[A.bra_pair[i]] * A.pair_np[A.ket_pair[i]];
+  }
+  const int t = len >= 512 ? 6 : len >= 64 ? 4 : len >= 16 ? 2 : 0;
+  glog = __builtin_amdgcn_readfirstlane(t);
+  const unsigned long long other = ~__ballot(base + lane < wend && t == glog);
+  cnt = min(other ? __ffsll(other) - 1 : 64, 64 >> glog);
+}
+
+// Window of a wave for n items: at least 16 waves per CU where the list allows.
+inline int l2g_lane_window(long long n, int ncu) {
+  int w = 4;
+  while (w < 64 && n > (long long)w * ncu * 16) w *= 2;
+  return w;
+}
+inline long long l2g_window_lanes(long long n, int ncu) {
+  const long long w = l2g_lane_window(n, ncu);
+  return (n + w - 1) / w * 64;
+}
 
 // Tier of a quartet of w primitive quartets on a Rys kernel: 0 and 1 share
 // their primitive loop between 16 and 4 slots of a block, 2 runs on one.

@@ -252,6 +252,11 @@ const L2gGenericClass& fock_gclass(int c) { return l2g_gen_generic[c - l2g_gen_n
 const L2gClassInfo& fock_info(int c) {
   return c < l2g_gen_nfock ? l2g_gen_fock[c] : l2g_gen_fock32[c - l2g_gen_nfock];
 }
+// lanes of m items of a class with a kernel of its own
+int64_t fock_lanes(const l2g_context_s* ctx, int c, int64_t m) {
+  const int per = fock_info(c).lanes;
+  return per ? m * per : l2g_window_lanes(m, ctx->ncu);
+}
 int fock_ybuf(int c) { return fock_is_generic(c) ? 0 : fock_info(c).ybuf_doubles; }
 
 // The screened unique quartets of one Fock build, by kernel class.
@@ -289,22 +294,16 @@ void sort_by_depth(FockItems& it) {
   it = std::move(s);
 }
 
-// Classes with fewer items than the chip has lanes to fill are split by
-// primitive-quartet range: an item whose loop is longer than the class's
-// chunk (about 1.4e5 recursion-node evaluations) becomes several items on
-// several lanes.  The digest is linear in the integrals, so each range is
-// digested on its own; the cost is one more HRR, transform and digest per
-// range.  Without this, one (dd|dd) quartet with K = 6 on every shell runs
-// ~1300 primitive quartets x 19 groups on one lane, tens of ms.
+// Deep items are split by primitive-quartet range: an item whose loop is
+// longer than the class's chunk becomes several items.  The digest is linear
+// in the integrals, so each range is digested on its own; the cost is one
+// more HRR, transform and digest per range.
 // Longest primitive range of one work item of class cls, for m items with
 // `total` primitive quartets in all, on a chip of `lanes` lanes (one wave
-// per SIMD).  A lane runs its primitive loop serially, each iteration waiting
-// on table and pair loads, so a deep item would bound the whole class: items
-// are cut to half of the class's per-lane share, but not below 8-16
-// primitives (fewer for classes with large recursions), which keeps the
-// per-piece HRR and digest small against the loop.  The generic kernel runs
-// one item per block; only its classes with few items are split, to about
-// 2e6 recursion values per piece.
+// per SIMD): half of the class's share per item in flight, but not below the
+// length from which one more HRR and digest is small against the loop.  The
+// generic kernel runs one item per block; only its classes with few items
+// are split, to about 2e6 recursion values per piece.
 int split_chunk(int cls, int64_t m, int64_t total, int lanes) {
   if (m == 0) return INT_MAX;
   if (fock_is_generic(cls))
@@ -313,9 +312,10 @@ int split_chunk(int cls, int64_t m, int64_t total, int lanes) {
     const int64_t slots = std::max<int64_t>(1, 2ll * lanes / per);
     return (int)std::min<int64_t>(INT_MAX, std::max<int64_t>(32, (total + 2 * slots - 1) / (2 * slots)));
   }
-  const int minc = std::max(8, std::min(16, 140000 / std::max(1, fock_info(cls).nodes)));
+  // the per-lane kernels share an item of 512 or more between the lanes of a
+  // wave (l2g_lane_tier)
   const int64_t share = (total + 2ll * lanes - 1) / (2ll * std::max(1, lanes));
-  return (int)std::min<int64_t>(INT_MAX, std::max<int64_t>(minc, share));
+  return (int)std::min<int64_t>(INT_MAX, std::max<int64_t>(1024, share));
 }
 
 void split_deep(FockItems& it, int cls, int lanes) {
@@ -575,6 +575,7 @@ void fock_launch_all(l2g_context_s* ctx, L2gEriArgs A, const ItemsView& items, b
     A.q_req = with_req ? items.req + o : nullptr;
     A.q_prange = items.pr + o;
     A.n = (int)m;
+    A.win = l2g_lane_window(m, ctx->ncu);
     if (fock_is_generic((int)c)) {
       launch_generic(kGenericFock, A, fock_gclass((int)c), ctx->gprog.as<int4>(), ctx->gidx.as<int>(),
                      (int)std::min<int64_t>((int64_t)ctx->ncu * 8, m), cs);
@@ -876,7 +877,7 @@ int l2g_fock_build(l2g_fock f, const double* D, double precision, double* J, dou
         if (m == 0) continue;
         // the generic kernel runs a block per item, no lane scratch, a few
         // blocks per CU: up to 4 items per CU count as small (side streams)
-        lanes[c] = fock_is_generic(c) ? m * 64 : m * std::max(1, fock_info(c).lanes);
+        lanes[c] = fock_is_generic(c) ? m * 64 : fock_lanes(ctx, c, m);
         yd[c] = fock_ybuf(c);
         ymax = std::max<int64_t>(ymax, yd[c]);
       }
@@ -1356,7 +1357,7 @@ void run_round(l2g_server_s* S, const std::vector<ServerRequest*>& act) {
   std::vector<int64_t> lanes(rv.count.size(), 0), yd(rv.count.size(), 0);
   for (size_t c = 0; c < rv.count.size(); ++c) {
     if (rv.count[c] == 0) continue;
-    lanes[c] = fock_is_generic((int)c) ? rv.count[c] * 64 : rv.count[c] * std::max(1, fock_info((int)c).lanes);
+    lanes[c] = fock_is_generic((int)c) ? rv.count[c] * 64 : fock_lanes(ctx, (int)c, rv.count[c]);
     yd[c] = fock_ybuf((int)c);
   }
   std::vector<ClassSlot> slots;  // within the server's scratch (sized for the full grid)

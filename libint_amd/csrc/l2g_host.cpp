@@ -86,7 +86,6 @@ struct ClassWork {
   bool fp32 = false;
   bool generic = false;
   bool native_generic = false;  // no register kernel for this class
-  bool coop = false;  // a wave per quartet (few, deeply contracted quartets)
   int rys = -1;       // index into l2g_gen_rys where the class runs on its Rys kernel
   int rys_cls = -1;   // the class's Rys kernel, whether it runs on it or not
   int rys_deep[2] = {0, 0};  // items in its tiers of deep quartets (rys_tier_of)
@@ -745,12 +744,11 @@ void plan_layout(l2g_eri_plan_s* p, l2g_context_s* ctx) {
                               c.nprimq >= L2G_GENERIC_MIN_DEPTH * c.count && class_l(c) >= L2G_GENERIC_MIN_L;
     c.rys = deep_generic ? -1 : c.rys_cls;
     if (c.rys >= 0) {
-      c.coop = c.generic = false;
+      c.generic = false;
       lanes.push_back(c.count * l2g_gen_rys[c.rys].lanes);
       yd.push_back(0);
       continue;
     }
-    c.coop = p->wave_split && !c.generic && few && c.nprimq >= 16 * c.count;
     if (deep_generic) {
       c.generic = true;
       c.cls = c.gidx;
@@ -759,7 +757,7 @@ void plan_layout(l2g_eri_plan_s* p, l2g_context_s* ctx) {
     // blocks per CU (LDS bound): up to 4 quartets per CU leave the chip
     // underfilled, so such classes count as small and run beside each other
     // on the side streams
-    lanes.push_back(c.generic ? c.count * 64 : (c.coop ? 64 * c.count : c.count));
+    lanes.push_back(c.generic ? c.count * 64 : l2g_window_lanes(c.count, ctx->ncu));
     yd.push_back(c.generic ? 0 : (c.fp32 ? l2g_gen_classes32 : l2g_gen_classes)[c.cls].ybuf_doubles);
   }
   plan_pieces(p, ctx);
@@ -769,8 +767,8 @@ void plan_layout(l2g_eri_plan_s* p, l2g_context_s* ctx) {
   // expected time for the side-stream packing: recursion values per
   // primitive quartet times primitive quartets, at each kernel kind's rate
   // (ns per value, measured on an s-f batch: the generic kernel 0.005 with
-  // its quartets split over blocks, 0.03 without; a wave per quartet 0.0025;
-  // a lane per quartet 0.02), plus 100 ns per quartet
+  // its quartets split over blocks, 0.03 without; the per-lane kernels
+  // 0.0025), plus 100 ns per quartet
   for (const auto& c : p->classes) {
     if (c.rys >= 0) {  // lane operations per primitive quartet, at 2 waves per SIMD on a part of the chip
       cost.push_back((double)c.nprimq * l2g_gen_rys[c.rys].nodes * 1e-4 + 3.0 * (double)c.count);
@@ -778,7 +776,7 @@ void plan_layout(l2g_eri_plan_s* p, l2g_context_s* ctx) {
     }
     const double vals = c.generic ? (double)l2g_gen_generic[c.cls].nvals
                                   : (double)(c.fp32 ? l2g_gen_classes32 : l2g_gen_classes)[c.cls].nodes;
-    const double rate = c.generic ? (c.npieces ? 0.005 : 0.03) : (c.coop ? 0.0025 : 0.02);
+    const double rate = c.generic ? (c.npieces ? 0.005 : 0.03) : 0.0025;
     cost.push_back((double)c.nprimq * vals * rate + 100.0 * (double)c.count);
   }
   std::vector<ClassSlot> slots;
@@ -938,7 +936,7 @@ int l2g_eri_plan_execute(l2g_eri_plan p, double* d_out) {
       }
       if (erf_idx >= 0) {
         const L2gClassInfo& ci = l2g_gen_classes_erf[erf_idx];
-        A.coop = c.coop ? 1 : 0;
+        A.win = l2g_lane_window(c.count, ctx->ncu);
         ci.launch(A, c.slot.grid, p->block, cs);
         LAUNCHCHK(std::string("erf ERI kernel of class ") + std::to_string(c.cls));
       } else if (c.generic || A.omega > 0) {  // the attenuated pass of erf / erfc
@@ -971,7 +969,7 @@ int l2g_eri_plan_execute(l2g_eri_plan p, double* d_out) {
         }
       } else {
         const L2gClassInfo& ci = (c.fp32 ? l2g_gen_classes32 : l2g_gen_classes)[c.cls];
-        A.coop = c.coop ? 1 : 0;
+        A.win = l2g_lane_window(c.count, ctx->ncu);
         // exactly the slot's grid: the scratch region holds grid * block lanes
         ci.launch(A, c.slot.grid, p->block, cs);
         LAUNCHCHK(std::string("ERI kernel of class ") + std::to_string(c.cls));
@@ -1115,7 +1113,7 @@ int l2g_eri_plan_stats(l2g_eri_plan p, int cap, int* ncls, int* code, int64_t* n
       const bool generic = c.rys >= 0 ? l2g_gen_rys[c.rys].over_limit != 0 : c.generic;
       if (code)
         code[i] = la * 1000 + lb * 100 + lc * 10 + ld + (c.fp32 ? 10000 : 0) + (generic ? 20000 : 0) +
-                  (c.coop || (c.rys >= 0 && c.npieces) ? 100000 : 0);
+                  (c.rys >= 0 && c.npieces ? 100000 : 0);
       if (nquart) nquart[i] = c.count;
       if (nprimq) nprimq[i] = c.nprimq;
       if (ms) {

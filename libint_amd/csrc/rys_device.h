@@ -40,7 +40,7 @@ __device__ __forceinline__ void rys_root(double T, const double* __restrict__ ta
     w = c[L2G_RYS_ND] * rs;
     return;
   }
-  const double x = 2.0 * (T - (double)iv) - 1.0;
+  const double x = fma(2.0, T - (double)iv, -1.0);
   const double2* __restrict__ c2 = reinterpret_cast<const double2*>(c);
   double2 a[L2G_RYS_ND];
 #pragma unroll
@@ -117,12 +117,14 @@ __device__ __forceinline__ void rys_prim(const L2gEriArgs& A, RysItem& I, int p,
     ok = ok && !(fabs(pf) < I.qprec);
   else if (A.method == L2G_SCREEN_CONSERVATIVE)
     ok = ok && !(fabs(pf) * fmax(1.0, A.pp_nonsph[gb] * A.pp_nonsph[gk]) * I.npbk < I.qprec);
+  // contraction is off in the including files (copies of this code have to
+  // round alike): the fused operations are written out
   const double PQx = P.x - Q.x, PQy = P.y - Q.y, PQz = P.z - Q.z;
   const double goq = Q.w * oos, gop = P.w * oos;
   const double rho = P.w * Q.w * oos;
-  double T = rho * (PQx * PQx + PQy * PQy + PQz * PQz), s = 1.0;
+  double T = rho * fma(PQz, PQz, fma(PQy, PQy, PQx * PQx)), s = 1.0;
   if (A.omega > 0) {  // erf(w r)/r: nodes s u(sT), weights sqrt(s) w(sT), s = w^2 / (w^2 + rho)
-    s = A.omega * A.omega / (A.omega * A.omega + rho);
+    s = A.omega * A.omega / fma(A.omega, A.omega, rho);
     T *= s;
   }
   double u, w;
