@@ -320,6 +320,7 @@ int l2g_init(int device, l2g_context* out) {
           for (int y = l - x; y >= 0; --y, ++c) sh[(l * 7 + m + l) * 10 + c] = l2g_solid_harmonics_coeff(l, m, x, y, l - x - y);
       }
     generic_init(sh.data());
+    onebody_init(sh.data());
     noalloc_setup(device);  // this device's address of the no-allocation scratch array
     *out = ctx.release();
   });
@@ -1528,43 +1529,67 @@ int l2g_onebody(l2g_basis B, int ncharge, const double* charges, const double* x
     const long long nbf = bf0[n];
     if (n == 0) return;
     hipStream_t st = ctx->stream;
-    DevBuf dl, dp, doff, da, dc, dO, dbf, dq, dqx, dS, dT, dV;
-    upload(dl, B->l, st);
-    upload(dp, B->pure, st);
-    upload(doff, B->off, st);
-    upload(da, B->alpha, st);
-    upload(dc, B->coeff, st);
-    upload(dO, B->origin, st);
-    upload(dbf, bf0, st);
-    std::vector<double> q(charges, charges + ncharge), qx(xyz, xyz + 3 * ncharge);
-    upload(dq, q, st);
-    upload(dqx, qx, st);
-    const size_t bytes = (size_t)nbf * nbf * sizeof(double);
+    // shell pairs by class, the shell of higher l first
+    int first[17] = {};
+    for (int i = 0; i < n; ++i)
+      for (int j = 0; j <= i; ++j) ++first[std::max(B->l[i], B->l[j]) * 4 + std::min(B->l[i], B->l[j]) + 1];
+    for (int k = 0; k < 16; ++k) first[k + 1] += first[k];
+    int at[16];
+    std::copy(first, first + 16, at);
+    // one device block: the inputs back to back (each at a multiple of 16 bytes), then the matrices
+    std::vector<unsigned char> h;
+    auto room = [&](size_t bytes) {
+      const size_t o = (h.size() + 15) & ~size_t(15);
+      h.resize(o + bytes);
+      return o;
+    };
+    auto put = [&](const auto* p, size_t count) {
+      const size_t o = room(count * sizeof(*p));
+      if (count) std::memcpy(h.data() + o, p, count * sizeof(*p));
+      return o;
+    };
+    const size_t opairs = room((size_t)first[16] * sizeof(int2));
+    int2* hp = reinterpret_cast<int2*>(h.data() + opairs);
+    for (int i = 0; i < n; ++i)
+      for (int j = 0; j <= i; ++j) {
+        const bool sw = B->l[i] < B->l[j];
+        const int a = sw ? j : i, b = sw ? i : j;
+        hp[at[B->l[a] * 4 + B->l[b]]++] = make_int2(a, b);
+      }
+    const size_t ol = put(B->l.data(), B->l.size()), op = put(B->pure.data(), B->pure.size()),
+                 oo = put(B->off.data(), B->off.size()), oa = put(B->alpha.data(), B->alpha.size()),
+                 oc = put(B->coeff.data(), B->coeff.size()), oO = put(B->origin.data(), B->origin.size()),
+                 ob = put(bf0.data(), bf0.size()), oq = put(charges, ncharge), ox = put(xyz, 3 * (size_t)ncharge);
+    const size_t bytes = (size_t)nbf * nbf * sizeof(double), om = (h.size() + 255) & ~size_t(255);
+    DevBuf d;
+    d.alloc(om + 3 * bytes);
+    unsigned char* const dp = d.as<unsigned char>();
+    HIPCHK(hipMemcpyAsync(dp, h.data(), h.size(), hipMemcpyHostToDevice, st));
     L2gOneBodyArgs A;
     std::memset(&A, 0, sizeof(A));
-    A.l = dl.as<int>();
-    A.pure = dp.as<int>();
-    A.poff = doff.as<int>();
-    A.alpha = da.as<double>();
-    A.coeff = dc.as<double>();
-    A.origin = dO.as<double>();
-    A.bf0 = dbf.as<long long>();
+    A.l = reinterpret_cast<int*>(dp + ol);
+    A.pure = reinterpret_cast<int*>(dp + op);
+    A.poff = reinterpret_cast<int*>(dp + oo);
+    A.alpha = reinterpret_cast<double*>(dp + oa);
+    A.coeff = reinterpret_cast<double*>(dp + oc);
+    A.origin = reinterpret_cast<double*>(dp + oO);
+    A.bf0 = reinterpret_cast<long long*>(dp + ob);
     A.nshell = n;
     A.nbf = nbf;
     A.ncharge = ncharge;
-    A.q = dq.as<double>();
-    A.qxyz = dqx.as<double>();
-    A.boys = ctx->boys.as<double>();
+    A.q = reinterpret_cast<double*>(dp + oq);
+    A.qxyz = reinterpret_cast<double*>(dp + ox);
+    A.rys = ctx->rys.as<double>();
     A.gauss = ctx->shg_gaussian;
-    if (S) dS.alloc(bytes), A.S = dS.as<double>();
-    if (T) dT.alloc(bytes), A.T = dT.as<double>();
-    if (V) dV.alloc(bytes), A.V = dV.as<double>();
-    launch_onebody(A, st);
+    double* const dm = reinterpret_cast<double*>(dp + om);
+    double *const dS = dm, *const dT = dm + (size_t)nbf * nbf, *const dV = dT + (size_t)nbf * nbf;
+    A.S = S ? dS : nullptr, A.T = T ? dT : nullptr, A.V = V ? dV : nullptr;
+    launch_onebody(A, reinterpret_cast<const int2*>(dp + opairs), first, st);
     hipError_t e = hipStreamSynchronize(st);
     if (e != hipSuccess) throw L2gError(L2G_E_LAUNCH, std::string("kernel execution failed: ") + hipGetErrorString(e));
-    if (S) HIPCHK(hipMemcpy(S, dS.p, bytes, hipMemcpyDeviceToHost));
-    if (T) HIPCHK(hipMemcpy(T, dT.p, bytes, hipMemcpyDeviceToHost));
-    if (V) HIPCHK(hipMemcpy(V, dV.p, bytes, hipMemcpyDeviceToHost));
+    if (S) HIPCHK(hipMemcpy(S, dS, bytes, hipMemcpyDeviceToHost));
+    if (T) HIPCHK(hipMemcpy(T, dT, bytes, hipMemcpyDeviceToHost));
+    if (V) HIPCHK(hipMemcpy(V, dV, bytes, hipMemcpyDeviceToHost));
   });
 }
 

@@ -413,7 +413,7 @@ struct L2gDerivTab {
   double coef[4][7][4];
 };
 
-// l2g_generic.hip: one-body integrals over every shell pair of a basis.
+// l2g_onebody.hip: one-body integrals over shell pairs of a basis.
 // Per-shell arrays (poff = first primitive, size nshell + 1; bf0 = first
 // function), point charges q at qxyz; S, T, V (any may be null) are nbf x
 // nbf row-major on the device.
@@ -430,13 +430,15 @@ struct L2gOneBodyArgs {
   int ncharge;
   const double* q;
   const double* qxyz;
-  const double* boys;
+  const double* rys;  // node table (codegen/rys_table.py)
   int gauss;
   double* S;
   double* T;
   double* V;
 };
-void launch_onebody(const L2gOneBodyArgs& A, hipStream_t s);
+// pairs: (higher l, lower l) shells by class, class (la, lb) at first[la * 4 + lb]
+void launch_onebody(const L2gOneBodyArgs& A, const int2* pairs, const int (&first)[17], hipStream_t s);
+void onebody_init(const double* sh);  // sh[4][7][10] solid-harmonic coefficients
 
 // l2g_aux.hip: first-derivative shell sets from the raised and lowered ERIs
 // of a derivative plan (one block per quartet); raw_off[k * nq + q] and
