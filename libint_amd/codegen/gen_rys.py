@@ -541,16 +541,14 @@ def emit(p, mode):
         E.block(f"for (int it = tid; it < qn * {p.ne * p.nf}; it += {NT})")
         E(f"const int qp = it / {p.ne * p.nf}, k = it - qp * {p.ne * p.nf};")
         E("const int qi = items[qlo + qp].qi;")
-        E("double s = 0.0;")
-        E.block("if (qi >= 0)")
-        E("for (int x = A.gpart_first[qi]; x < A.gpart_first[qi + 1]; ++x) s += A.gpart[x * A.gpart_stride + k];")
-        E.end()
+        E("const int x0 = qi >= 0 ? A.gpart_first[qi] : 0, x1 = qi >= 0 ? A.gpart_first[qi + 1] : 0;")
+        E("const double s = rys_piece_sum(A.gpart + x0 * A.gpart_stride + k, A.gpart_stride, x1 - x0);")
         E(f"sm[qp * region + (k / {p.nf}) * {p.rstr} + k % {p.nf}] = s;")
         E.end()
         E.block("if (tid < qn && items[qlo + tid].qi >= 0)")
         E("const int qi = items[qlo + tid].qi;")
-        E("double s = 0.0;")
-        E(f"for (int x = A.gpart_first[qi]; x < A.gpart_first[qi + 1]; ++x) s += A.gpart[x * A.gpart_stride + {p.ne * p.nf}];")
+        E("const int x0 = A.gpart_first[qi], x1 = A.gpart_first[qi + 1];")
+        E(f"const double s = rys_piece_sum(A.gpart + x0 * A.gpart_stride + {p.ne * p.nf}, A.gpart_stride, x1 - x0);")
         E("items[qlo + tid].nsurv = s > 0.0;")
         E.end()
         E.end()

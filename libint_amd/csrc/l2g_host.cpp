@@ -657,6 +657,15 @@ int class_l(const ClassWork& c) {
 // gpart; a second pass sums each quartet's pieces in piece order and runs
 // the HRR and store.  A block per quartet would otherwise walk the deepest
 // quartet's primitive loop alone while the rest of the chip idles.
+//
+// Rys classes take pieces when a slot's longest serial loop passes kRysSerial
+// primitive quartets: the second launch costs a class of shallow quartets
+// more than the pieces save (22 s/p/d classes of 55 to 80
+// primitive quartets a quartet, erfc: 1.66 ms at 96, 1.79 at 64, 1.98 at 160).
+// At kRysPiece primitive quartets a piece the batch of 58 s..f classes, K to
+// 8, takes 3.0 ms at 48, 2.4 at 32, 2.05 at 24, 2.4 at 20, 3.1 at 16: shorter
+// pieces leave more partial sums than loops saved.
+constexpr int64_t kRysPiece = 24, kRysSerial = 96;
 void plan_pieces(l2g_eri_plan_s* p, l2g_context_s* ctx) {
   std::vector<int> pb, pk, pm, pf;
   std::vector<long long> pq;
@@ -673,11 +682,11 @@ void plan_pieces(l2g_eri_plan_s* p, l2g_context_s* ctx) {
     int64_t chunk;
     if (c.rys >= 0) {
       const int64_t slots = (int64_t)ctx->ncu * 512 / l2g_gen_rys[c.rys].lanes;  // quartets at 2 waves per SIMD
-      chunk = std::max<int64_t>(48, (c.nprimq + slots - 1) / slots);
+      chunk = std::max<int64_t>(kRysPiece, (c.nprimq + slots - 1) / slots);
       // the longest serial loop: the deepest quartet's, shared by up to 16 slots
       const int64_t serial = wmax / std::min<int64_t>(wmax >= L2G_RYS_DEEP0 ? 16 : wmax >= L2G_RYS_DEEP1 ? 4 : 1,
                                                       std::max(1, 64 / l2g_gen_rys[c.rys].lanes));
-      if (serial <= 2 * chunk) continue;
+      if (serial <= std::max<int64_t>(2 * chunk, kRysSerial)) continue;
     } else {
       chunk = std::max<int64_t>(32, (c.nprimq + 4 * ctx->ncu - 1) / (4 * ctx->ncu));
       chunk += chunk & 1;  // even: the two-primitive pass stays full

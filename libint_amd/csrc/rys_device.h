@@ -77,18 +77,23 @@ struct RysItem {
 // loop would otherwise run serially on one slot while the chip drains, and
 // its sums are shorter.  The share depends on the quartet alone
 // (rys_tier_of), so its bits do not depend on the batch it is in.
+// The finish launch after pieces has few quartets with many partial sums
+// each: a block per quartet.
 template <int Q>
 struct RysTier {
   static constexpr int S0 = Q < 16 ? Q : 16, S1 = Q < 4 ? Q : 4;
   int S, NI, first, end;
   static __host__ __device__ int ceil_div(int a, int b) { return (a + b - 1) / b; }
   static int blocks(const L2gEriArgs& A) {
+    if (A.gpart_mode == 2) return A.n;
     const int a = A.rys_deep[0], b = A.rys_deep[1];
     return ceil_div(a, Q / S0) + ceil_div(b, Q / S1) + ceil_div(A.n - a - b, Q);
   }
   __device__ __forceinline__ RysTier(const L2gEriArgs& A, int blk) {
     const int a = A.rys_deep[0], b = A.rys_deep[1], na = ceil_div(a, Q / S0), nb = ceil_div(b, Q / S1);
-    if (blk < na) {
+    if (A.gpart_mode == 2) {
+      S = 1, NI = 1, first = blk, end = A.n;
+    } else if (blk < na) {
       S = S0, NI = Q / S0, first = blk * NI, end = a;
     } else if (blk < na + nb) {
       S = S1, NI = Q / S1, first = a + (blk - na) * NI, end = a + b;
@@ -97,6 +102,22 @@ struct RysTier {
     }
   }
 };
+
+// Sum of one value over n pieces, in piece order; the loads of 16 pieces are
+// in flight together (one after the other, the sums of the 85 pieces of a
+// 4096-primitive (dp|ff) quartet took 0.6 ms).
+__device__ __forceinline__ double rys_piece_sum(const double* __restrict__ g, long long stride, int n) {
+  double s = 0.0;
+#pragma unroll 1
+  for (int x = 0; x < n; x += 16, g += 16 * stride) {
+    double v[16];
+#pragma unroll
+    for (int k = 0; k < 16; ++k) v[k] = x + k < n ? g[k * stride] : 0.0;
+#pragma unroll
+    for (int k = 0; k < 16; ++k) s += v[k];
+  }
+  return s;
+}
 
 // Primitive quartet p of an item (act false: a stand-in that contributes
 // nothing): screening as the per-lane kernels do it, the record (rec, by the
