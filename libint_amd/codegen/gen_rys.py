@@ -51,7 +51,7 @@ import random
 import gen_eri as ge
 import rys_table
 
-REC = 17
+REC = 15
 
 
 def comps(l1, l2):
@@ -135,6 +135,7 @@ class Plan:
         self.ng = 1 if rl else self.nr   # nodes whose 2D integrals are in LDS at a time
         self.nb = nb
         self.root_rounds = -(-self.q * nb * self.nr // self.nt) / nb
+        self.prim_rounds = -(-self.q * nb // self.nt) / nb
         # row stride of the contracted block in LDS (odd), and doubles per
         # quartet of a pass: with every shell a solid harmonic / Cartesian
         self.rstr = max(self.nf, ge.ncart(lc) * ge.ncart(ld)) | 1
@@ -194,13 +195,13 @@ class Plan:
         return max(1, min(4, 512 // max(1, self.regs()), int(163840 / (self.lds_bytes('fock') / self.nw) / 4)))
 
     def cost(self):
-        """Lane operations per primitive quartet (product, 2D and root stages), over the share of the VALU that so many
+        """Lane operations per primitive quartet (product, 2D, root and primitive stages), over the share of the VALU that so many
         waves per SIMD were seen to fill, or the LDS clocks where those are more."""
         main = self.nr * (self.te * len(self.inner) + sum(self.nxy(x) for x in self.parts)) + self.te * len(self.inner)
         reads = self.nr * sum(len(a) + len(b) + self.te * len(c) for a, b, c in map(self.rows_of, self.parts))
         rounds = self.nr // self.ng * -(-self.q * self.ng * 3 // self.nt)
         two = rounds * (3.5 * (self.na + 1) * (self.nc + 1) + 40)
-        root = self.root_rounds * 170 + 60 / self.nb
+        root = self.prim_rounds * 150 + self.root_rounds * 85 + 60 / self.nb
         valu = main + reads // 2 + two + root + 30
         lds = (reads + rounds * (self.gb + 12)) * 4.0  # quarter clocks of the CU's LDS for four SIMDs
         return max(valu / {1: 0.35, 2: 0.6, 3: 0.75, 4: 0.85}[self.occupancy()], lds / 0.8) * self.nt / self.q * \
@@ -213,30 +214,37 @@ class Plan:
 
 # Layouts that measured faster than the model's choice: (side, tile, waves, node by node, parts, batch), with the
 # nanoseconds per primitive quartet of the model's choice and of this one on one MI355X (ERI batches of
-# 25,000 to 150,000 quartets, K <= 5).
+# 25,000 to 150,000 quartets, 80 primitive quartets each on average).
 TUNED = {
-    '0000': ('bra', 1, 1, True, 1, 1),  # 0.042 -> 0.029
-    '0010': ('ket', 1, 1, True, 1, 3),  # 0.033 -> 0.029
-    '0021': ('ket', 1, 1, False, 1, 8),  # 0.075 -> 0.060
-    '0030': ('bra', 1, 1, True, 1, 1),  # 0.069 -> 0.060
-    '0031': ('ket', 2, 1, False, 1, 4),  # 0.117 -> 0.090
-    '0033': ('ket', 2, 2, False, 1, 8),  # 0.341 -> 0.258
-    '1011': ('ket', 2, 1, False, 1, 3),  # 0.067 -> 0.062
-    '1022': ('bra', 1, 1, True, 1, 1),  # 0.159 -> 0.133
-    '1031': ('bra', 1, 1, True, 1, 1),  # 0.128 -> 0.110
-    '1033': ('ket', 2, 2, False, 1, 4),  # 0.405 -> 0.390
-    '1120': ('ket', 1, 1, False, 1, 2),  # 0.122 -> 0.107
-    '2011': ('bra', 1, 1, False, 1, 2),  # 0.124 -> 0.107
-    '2021': ('bra', 1, 1, True, 1, 2),  # 0.179 -> 0.154
-    '2031': ('bra', 1, 1, False, 1, 1),  # 0.287 -> 0.217
-    '2032': ('bra', 1, 1, True, 1, 3),  # 0.510 -> 0.327
-    '2122': ('bra', 1, 1, False, 2, 4),  # 0.370 -> 0.353
-    '2133': ('bra', 1, 1, False, 3, 6),  # 1.164 -> 1.037
-    '2232': ('bra', 1, 1, False, 1, 6),  # 1.427 -> 0.850
-    '3032': ('ket', 2, 1, False, 1, 6),  # 0.694 -> 0.662
-    '3131': ('bra', 1, 1, False, 1, 6),  # 0.619 -> 0.564
-    '3132': ('bra', 1, 1, False, 1, 6),  # 1.186 -> 0.844
-    '3133': ('ket', 1, 4, False, 1, 8),  # 1.924 -> 1.659
+    '0021': ('ket', 1, 1, False, 1, 12),  # 0.064 -> 0.054
+    '0022': ('ket', 2, 1, False, 1, 12),  # 0.081 -> 0.076
+    '0030': ('bra', 1, 1, True, 1, 1),  # 0.059 -> 0.049
+    '0031': ('ket', 2, 1, False, 1, 12),  # 0.087 -> 0.074
+    '0033': ('ket', 2, 2, False, 1, 16),  # 0.276 -> 0.235
+    '1010': ('ket', 1, 1, True, 1, 3),  # 0.047 -> 0.043
+    '1020': ('bra', 1, 1, True, 1, 3),  # 0.052 -> 0.051
+    '1021': ('bra', 1, 1, True, 1, 2),  # 0.091 -> 0.088
+    '1022': ('bra', 1, 1, True, 1, 3),  # 0.144 -> 0.115
+    '1030': ('bra', 1, 1, True, 1, 2),  # 0.085 -> 0.082
+    '1031': ('bra', 1, 1, True, 1, 2),  # 0.103 -> 0.103, the loop of few quartets is shorter
+    '1033': ('ket', 2, 2, False, 1, 16),  # 0.428 -> 0.350
+    '1120': ('ket', 1, 1, False, 1, 4),  # 0.113 -> 0.097
+    '1132': ('bra', 1, 1, False, 1, 3),  # 0.496 -> 0.403
+    '2011': ('bra', 1, 1, False, 1, 4),  # 0.112 -> 0.098
+    '2020': ('bra', 1, 1, False, 1, 4),  # 0.099 -> 0.095
+    '2021': ('bra', 1, 1, True, 1, 4),  # 0.167 -> 0.135
+    '2022': ('ket', 2, 1, False, 1, 8),  # 0.202 -> 0.196
+    '2031': ('bra', 1, 1, False, 1, 4),  # 0.223 -> 0.197
+    '2032': ('bra', 1, 2, True, 1, 6),  # 0.304 -> 0.294
+    '2033': ('ket', 2, 2, False, 1, 16),  # 0.622 -> 0.568
+    '2121': ('ket', 1, 1, False, 1, 8),  # 0.212 -> 0.206
+    '2133': ('bra', 1, 1, False, 3, 16),  # 1.195 -> 1.021
+    '2232': ('bra', 1, 1, False, 1, 16),  # 1.312 -> 0.803
+    '3030': ('ket', 1, 1, False, 1, 8),  # 0.288 -> 0.274
+    '3032': ('bra', 1, 1, False, 1, 1),  # 0.666 -> 0.504
+    '3033': ('ket', 2, 2, False, 1, 16),  # 0.925 -> 0.895
+    '3132': ('bra', 1, 1, False, 1, 16),  # 1.115 -> 0.798
+    '3133': ('ket', 1, 4, False, 1, 16),  # 2.074 -> 1.593
 }
 
 
@@ -250,11 +258,11 @@ def plan(la, lb, lc, ld):
         for te in (1, 2):
             for nw in (1, 2, 4):
                 for rl, nparts in ((True, 1), (False, 1), (False, 2), (False, 3)):
-                    for nb in (1, 2, 3, 4, 6, 8):
+                    for nb in (1, 2, 3, 4, 6, 8, 12, 16):
                         p = Plan(la, lb, lc, ld, side, te, nw, nparts, rl, nb)
                         if p.parts is None or p.q == 0 or p.regs() > 270 or p.lds_bytes('fock') > 150 * 1024:
                             continue
-                        if nb > 1 and p.q * nb * p.nr > 3 * p.nt:
+                        if nb > 1 and p.q * nb > p.nt:
                             continue
                         c = p.cost()
                         if best is None or c < best[0]:
@@ -311,13 +319,14 @@ def emit(p, mode):
     E("I.qi = tid < NI * S && qi < tier.end ? qi : -1;")
     E("I.nsurv = 0;")
     E("I.pb0 = I.pk0 = I.npk = I.pbeg = I.pend = I.bp = I.kp = I.meta = 0;")
-    E("I.lnprec = A.ln_precision, I.qprec = A.precision, I.npbk = 0.0;")
+    E("I.lnprec = A.ln_precision, I.qprec = A.precision, I.npbk = I.rnpk = 0.0;")
     E.block("if (I.qi >= 0)")
     E("I.bp = A.bra_pair[qi], I.kp = A.ket_pair[qi], I.meta = A.meta[qi];")
     E("I.pb0 = A.pair_first[I.bp], I.pk0 = A.pair_first[I.kp];")
     E("const int npb = A.pair_np[I.bp];")
     E("I.npk = A.pair_np[I.kp];")
     E("I.npbk = (double)npb * (double)I.npk;")
+    E("I.rnpk = 1.0 / I.npk;")
     E("I.pend = npb * I.npk;")
     E("if (A.q_prange) I.pbeg = A.q_prange[qi].x, I.pend = A.q_prange[qi].y;")
     if mode == 'eri':
@@ -352,20 +361,33 @@ def emit(p, mode):
     if mode == 'eri':
         E("if (A.gpart_mode == 2) len = 0;  // the contracted values come from the pieces")
     E.block(f"for (int p0 = 0; p0 < len; p0 += {NB})")
-    # root stage
-    nroot = NB * Q * NR
-    rounds = -(-nroot // NT)
-    if rounds > 1:
-        E.block(f"for (int it = tid; it < {nroot}; it += {NT})")
-    else:
-        E("const int it = tid;")
-        E.block(f"if (it < {nroot})")
-    E(f"const int bq = it / {NR}, r = it - bq * {NR};")
-    E(f"const int b = bq / {Q}, q = bq - b * {Q};")
-    E(f"rys_prim<{NR}>(A, items[q], items[q].pbeg + p0 + b, r, sm + {rec} + bq * {REC}, sm + {uw} + it * 2, tab);")
+    E(f"const int nbat = min({NB}, len - p0);")
+
+    def lanes(n, per):  # a lane per item of the batch
+        if NB * per > NT:
+            E.block(f"for (int it = tid; it < {n}; it += {NT})")
+        else:
+            E("const int it = tid;")
+            E.block(f"if (it < {n})")
+    # primitive stage
+    E.block("")
+    lanes(f"nbat * {Q}", Q)
+    E(f"const int b = it / {Q}, q = it - b * {Q};")
+    E(f"rys_prim(A, items[q], items[q].pbeg + p0 + b, sm + {rec} + it * {REC});")
+    E.end()
     E.end()
     E(f"rys_sync<{NW}>();")
-    E(f"const int nbat = min({NB}, len - p0);")
+    # root stage
+    E.block("")
+    lanes(f"nbat * {Q * NR}", Q * NR)
+    E(f"const int bq = it / {NR}, r = it - bq * {NR};")
+    E(f"const double* const rc = sm + {rec} + bq * {REC};")
+    E("double u, w;")
+    E(f"rys_root<{NR}>(rc[13], tab, r, u, w);")
+    E(f"sm[{uw} + it * 2] = u, sm[{uw} + it * 2 + 1] = w * rc[14];")
+    E.end()
+    E.end()
+    E(f"rys_sync<{NW}>();")
     E("#pragma unroll 1")
     E.block("for (int b = 0; b < nbat; ++b)")
     # 2D stage
@@ -388,8 +410,9 @@ def emit(p, mode):
         E(f"const int q = qr / {NR}, node = b * {Q * NR} + qr;")
     E(f"const double* const rc = sm + {rec} + (b * {Q} + q) * {REC};")
     E(f"const double u = sm[{uw} + node * 2], w = sm[{uw} + node * 2 + 1];")
-    E("const double C00 = fma(u, rc[ax * 4 + 2], rc[ax * 4]), D00 = fma(u, rc[ax * 4 + 3], rc[ax * 4 + 1]);")
-    E("const double B00 = u * rc[16], B10 = fma(-u, rc[13], rc[12]), B01 = fma(-u, rc[15], rc[14]);")
+    E("const double ug = u * rc[9], up = u * rc[10], PQ = rc[ax * 3 + 2];")
+    E("const double C00 = fma(-ug, PQ, rc[ax * 3]), D00 = fma(up, PQ, rc[ax * 3 + 1]);")
+    E("const double B00 = up * rc[11], B10 = fma(-ug, rc[11], rc[11]), B01 = fma(-up, rc[12], rc[12]);")
     E("(void)C00; (void)D00; (void)B00; (void)B10; (void)B01;")
     E(f"double* const g = sm + {g0} + it * {p.gb};")
     E("const double g_0_0 = ax == 2 ? w : 1.0;")

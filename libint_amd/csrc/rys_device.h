@@ -59,16 +59,17 @@ __device__ __forceinline__ void rys_root(double T, const double* __restrict__ ta
   w = q;
 }
 
-// One primitive quartet as a Rys kernel's root stage leaves it in LDS: per
-// axis PA, QC, WP, WQ, then 1/2z, rho/2z^2, 1/2e, rho/2e^2, 1/2(z+e).
-#define L2G_RYS_REC 17
+// One primitive quartet as a Rys kernel's primitive stage leaves it in LDS:
+// per axis PA, QC, P - Q, then eta/(zeta+eta), zeta/(zeta+eta), 1/2zeta,
+// 1/2eta, the rule's argument T and the prefactor (0: screened out).
+#define L2G_RYS_REC 15
 
 // Shell quartet of a work item (LDS, one per quartet of the block).
 struct RysItem {
   int pb0, pk0, npk, pbeg, pend, bp, kp, meta;
   int qi;       // index in the work list, -1 past its end
   int nsurv;    // non-zero once a primitive quartet survived the screening
-  double lnprec, qprec, npbk;
+  double lnprec, qprec, npbk, rnpk;
 };
 
 // The work items of a block of Q slots.  The list is sorted by decreasing
@@ -119,20 +120,18 @@ __device__ __forceinline__ double rys_piece_sum(const double* __restrict__ g, lo
   return s;
 }
 
-// Primitive quartet p of an item (act false: a stand-in that contributes
-// nothing): screening as the per-lane kernels do it, the record (rec, by the
-// lane of root 0) and node and weight of root r.
-template <int NR>
-__device__ __forceinline__ void rys_prim(const L2gEriArgs& A, RysItem& I, int p, int r, double* rec, double* uw,
-                                         const double* __restrict__ tab) {
+// Primitive quartet p of an item: screening as the per-lane kernels do it,
+// and the record.  Past the item's end (act false) a stand-in with prefactor 0.
+__device__ __forceinline__ void rys_prim(const L2gEriArgs& A, RysItem& I, int p, double* rec) {
   const bool act = p < I.pend;
-  const int ib = act ? p / I.npk : 0;
+  // p / npk: the half keeps the product off the integers by more than its rounding error
+  const int ib = act ? (int)(((double)p + 0.5) * I.rnpk) : 0;
   const int gb = act ? I.pb0 + ib : 0, gk = act ? I.pk0 + (p - ib * I.npk) : 0;
   const double4 P = A.pp_P[gb], PA = A.pp_PA[gb], Q = A.pp_P[gk], QC = A.pp_PA[gk];
   const double2 xb = A.pp_aux[gb], xk = A.pp_aux[gk];
   const double rs = rsqrt(P.w + Q.w);
   const double oos = rs * rs;
-  const double pf = PA.w * QC.w * rs * A.scale;
+  double pf = PA.w * QC.w * rs * A.scale;
   bool ok = act && xb.x + xk.x > I.lnprec;
   if (A.method == L2G_SCREEN_ORIGINAL)
     ok = ok && !(fabs(pf) < I.qprec);
@@ -141,30 +140,22 @@ __device__ __forceinline__ void rys_prim(const L2gEriArgs& A, RysItem& I, int p,
   // contraction is off in the including files (copies of this code have to
   // round alike): the fused operations are written out
   const double PQx = P.x - Q.x, PQy = P.y - Q.y, PQz = P.z - Q.z;
-  const double goq = Q.w * oos, gop = P.w * oos;
+  double goq = Q.w * oos, gop = P.w * oos;
   const double rho = P.w * Q.w * oos;
-  double T = rho * fma(PQz, PQz, fma(PQy, PQy, PQx * PQx)), s = 1.0;
+  double T = rho * fma(PQz, PQz, fma(PQy, PQy, PQx * PQx));
   if (A.omega > 0) {  // erf(w r)/r: nodes s u(sT), weights sqrt(s) w(sT), s = w^2 / (w^2 + rho)
-    s = A.omega * A.omega / fma(A.omega, A.omega, rho);
+    const double s = A.omega * A.omega / fma(A.omega, A.omega, rho);
     T *= s;
+    goq *= s;  // the nodes enter as u goq and u gop only
+    gop *= s;
+    pf *= sqrt(s);
   }
-  double u, w;
-  rys_root<NR>(T, tab, r, u, w);
-  if (A.omega > 0) {
-    u *= s;
-    w *= sqrt(s);
-  }
-  uw[0] = u;
-  uw[1] = ok ? w * pf : 0.0;
-  if (r == 0) {
-    if (ok) I.nsurv = 1;
-    rec[0] = PA.x, rec[1] = QC.x, rec[2] = -goq * PQx, rec[3] = gop * PQx;
-    rec[4] = PA.y, rec[5] = QC.y, rec[6] = -goq * PQy, rec[7] = gop * PQy;
-    rec[8] = PA.z, rec[9] = QC.z, rec[10] = -goq * PQz, rec[11] = gop * PQz;
-    rec[12] = xb.y, rec[13] = xb.y * goq;
-    rec[14] = xk.y, rec[15] = xk.y * gop;
-    rec[16] = 0.5 * oos;
-  }
+  if (ok) I.nsurv = 1;
+  rec[0] = PA.x, rec[1] = QC.x, rec[2] = PQx;
+  rec[3] = PA.y, rec[4] = QC.y, rec[5] = PQy;
+  rec[6] = PA.z, rec[7] = QC.z, rec[8] = PQz;
+  rec[9] = goq, rec[10] = gop, rec[11] = xb.y, rec[12] = xk.y;
+  rec[13] = ok ? T : 0.0, rec[14] = ok ? pf : 0.0;
 }
 
 // Integrals of a canonical quartet with the pure flags of meta.
