@@ -745,20 +745,24 @@ def emit(p, mode):
     n = p.dims(False)
     ncomb = sum(n[i] * n[j] for i in range(4) for j in range(i + 1, 4))
     if mode == 'fock':
-        E("#pragma unroll 1")
-        E(f"for (int it = tid; it < qn * {ncomb}; it += {NT}) {{")
-        E.ind += 1
-        E(f"const int qp = it / {ncomb}, o = it - qp * {ncomb};")
-        E(f"if (items[qlo + qp].nsurv && o < dig[qp].off[6]) sm[qp * region + vofs + dig[qp].nv + o] = rys_density(A, dig[qp], o);")
-        E.end()
-        E(f"rys_sync<{NW}>();")
-        E("#pragma unroll 1")
-        E(f"for (int it = tid; it < qn * {ncomb}; it += {NT}) {{")
-        E.ind += 1
-        E(f"const int qp = it / {ncomb}, o = it - qp * {ncomb};")
-        E(f"if (items[qlo + qp].nsurv && o < dig[qp].off[6]) "
-          f"rys_digest(A, dig[qp], o, sm + qp * region + vofs, sm + qp * region + vofs + dig[qp].nv);")
-        E.end()
+        pure = ', '.join(map(str, p.dims(True)))
+        call = f"rys_digest_pure<{NT}, {NW}, {pure}>(A, items + qlo, dig, qn, sm + vofs, region);"
+        if not mask:
+            E(call)
+        else:
+            E.block("if (!cart)")
+            E(call)
+            E.end()
+            E.block("else")
+            for what in (f"sm[qp * region + vofs + dig[qp].nv + o] = rys_density(A, dig[qp], o);",
+                         f"rys_digest(A, dig[qp], o, sm + qp * region + vofs, sm + qp * region + vofs + dig[qp].nv);"):
+                E("#pragma unroll 1")
+                E.block(f"for (int it = tid; it < qn * {ncomb}; it += {NT})")
+                E(f"const int qp = it / {ncomb}, o = it - qp * {ncomb};")
+                E(f"if (items[qlo + qp].nsurv && o < dig[qp].off[6]) {what}")
+                E.end()
+                E(f"rys_sync<{NW}>();")
+            E.end()
     E.end()  # passes
     if mode == 'eri':
         E(f"rys_sync<{NW}>();")

@@ -348,9 +348,12 @@ struct l2g_basis_s {
   // caller's order would.  s and p shells keep the caller's order.
   bool second_is_centre(int i, int j) {
     if (i == j || l[i] != l[j] || l[i] < 2) return false;
+    // a single primitive pair (the Schwarz factors of primitives have 1e5
+    // of them) costs less to look at than to remember
+    const bool memo = nprim[i] * nprim[j] > 1;
     const uint64_t key = (uint64_t)(uint32_t)i << 32 | (uint32_t)j;
-    auto it = orient.find(key);
-    if (it != orient.end()) return it->second;
+    if (memo)
+      if (auto it = orient.find(key); it != orient.end()) return it->second;
     double AB2 = 0;
     for (int k = 0; k < 3; ++k) AB2 += (origin[3 * i + k] - origin[3 * j + k]) * (origin[3 * i + k] - origin[3 * j + k]);
     double s = 0, sa = 0, sb = 0;
@@ -368,8 +371,10 @@ struct l2g_basis_s {
         }
     }
     const bool r = l[i] >= 3 ? s > 0 : sb < 1e-3 * sa, back = l[i] >= 3 ? s < 0 : sa < 1e-3 * sb;
-    orient.emplace(key, r);
-    orient.emplace((uint64_t)(uint32_t)j << 32 | (uint32_t)i, back);
+    if (memo) {
+      orient.emplace(key, r);
+      orient.emplace((uint64_t)(uint32_t)j << 32 | (uint32_t)i, back);
+    }
     return r;
   }
   // canonical bra orientation of (i, j): l_i >= l_j, ties by second_is_centre

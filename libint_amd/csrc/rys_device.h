@@ -236,3 +236,64 @@ __device__ __forceinline__ void rys_digest(const L2gEriArgs& A, const RysDigest&
   double* m = b < 2 ? A.jg : A.kg;
   l2g_acc(&m[g.mo + g.fn(i, r, A.shg_gaussian) * g.N + g.fn(j, c, A.shg_gaussian)], g.deg * s, A.fx_hoff);
 }
+
+// The same for a block of quartets of solid harmonics (and s, p), whose
+// shell sizes are then the class's: block B of the density into LDS, and
+// block B's contributions.  A loop per block has no divergence and constant
+// strides; the general loops above spend 260 instructions an element on
+// decoding it.  Each sum runs in the general loop's order.
+template <int NT, int B, int N0, int N1, int N2, int N3>
+struct RysBlock {
+  static constexpr int n[4] = {N0, N1, N2, N3}, sv[4] = {N1 * N2 * N3, N2 * N3, N3, 1}, nv = N0 * N1 * N2 * N3;
+  static constexpr int bi[6] = {0, 2, 0, 0, 1, 1}, bj[6] = {1, 3, 2, 3, 2, 3};
+  static constexpr int first(int b) { return b == 0 ? 0 : first(b - 1) + n[bi[b - 1]] * n[bj[b - 1]]; }
+  static constexpr int i = bi[B], j = bj[B], size = n[i] * n[j];
+  static constexpr int pb = B < 2 ? 1 - B : 7 - B, pi = bi[pb], pj = bj[pb], nx = n[pi], ny = n[pj];
+
+  static __device__ __forceinline__ long long at(const L2gEriArgs& A, const RysDigest& g, int k) {
+    const int r = k / n[j], c = k - r * n[j];
+    const int fr = A.shg_gaussian ? g.fn(i, r, 1) : g.bf[i] + r, fc = A.shg_gaussian ? g.fn(j, c, 1) : g.bf[j] + c;
+    return g.mo + (long long)fr * (int)g.N + fc;
+  }
+  static __device__ __forceinline__ void density(const L2gEriArgs& A, const RysItem* items, const RysDigest* dig, int qn,
+                                                 double* V, int region) {
+    for (int it = threadIdx.x; it < qn * size; it += NT) {
+      const int q = it / size, k = it - q * size;
+      if (items[q].nsurv) V[q * region + nv + first(B) + k] = A.dens[at(A, dig[q], k)];
+    }
+  }
+  static __device__ __forceinline__ void digest(const L2gEriArgs& A, const RysItem* items, const RysDigest* dig, int qn,
+                                                const double* V, int region) {
+    for (int it = threadIdx.x; it < qn * size; it += NT) {
+      const int q = it / size, k = it - q * size;
+      if (!items[q].nsurv) continue;
+      const int r = k / n[j], c = k - r * n[j];
+      const double* v = V + q * region + r * sv[i] + c * sv[j];
+      const double* d = V + q * region + nv + first(pb);
+      double s = 0.0;
+#pragma unroll(nx * ny <= 25 ? nx : 1)
+      for (int x = 0; x < nx; ++x)
+#pragma unroll
+        for (int y = 0; y < ny; ++y) s = fma(d[x * ny + y], v[x * sv[pi] + y * sv[pj]], s);
+      l2g_acc(&(B < 2 ? A.jg : A.kg)[at(A, dig[q], k)], dig[q].deg * s, A.fx_hoff);
+    }
+  }
+};
+
+template <int NT, int NW, int N0, int N1, int N2, int N3>
+__device__ __forceinline__ void rys_digest_pure(const L2gEriArgs& A, const RysItem* items, const RysDigest* dig, int qn,
+                                                double* V, int region) {
+  RysBlock<NT, 0, N0, N1, N2, N3>::density(A, items, dig, qn, V, region);
+  RysBlock<NT, 1, N0, N1, N2, N3>::density(A, items, dig, qn, V, region);
+  RysBlock<NT, 2, N0, N1, N2, N3>::density(A, items, dig, qn, V, region);
+  RysBlock<NT, 3, N0, N1, N2, N3>::density(A, items, dig, qn, V, region);
+  RysBlock<NT, 4, N0, N1, N2, N3>::density(A, items, dig, qn, V, region);
+  RysBlock<NT, 5, N0, N1, N2, N3>::density(A, items, dig, qn, V, region);
+  rys_sync<NW>();
+  RysBlock<NT, 0, N0, N1, N2, N3>::digest(A, items, dig, qn, V, region);
+  RysBlock<NT, 1, N0, N1, N2, N3>::digest(A, items, dig, qn, V, region);
+  RysBlock<NT, 2, N0, N1, N2, N3>::digest(A, items, dig, qn, V, region);
+  RysBlock<NT, 3, N0, N1, N2, N3>::digest(A, items, dig, qn, V, region);
+  RysBlock<NT, 4, N0, N1, N2, N3>::digest(A, items, dig, qn, V, region);
+  RysBlock<NT, 5, N0, N1, N2, N3>::digest(A, items, dig, qn, V, region);
+}
