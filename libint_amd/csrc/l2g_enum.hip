@@ -29,6 +29,24 @@ __device__ __forceinline__ void decode_tri(long long t, long long& p1, long long
   p2 = t - a * (a + 1) / 2;
 }
 
+// Largest |D| of every shell block, and of all of them (dmax: bits of a
+// non-negative double, which order as integers)
+__global__ void __launch_bounds__(kEnumThreads) shell_norms(const double* __restrict__ D, long long N,
+                                                            const int* __restrict__ bf1st, int n,
+                                                            double* __restrict__ Dn,
+                                                            unsigned long long* __restrict__ dmax) {
+  const long long k = (long long)blockIdx.x * kEnumThreads + threadIdx.x;
+  double m = 0.0;
+  if (k < (long long)n * n) {
+    const int s1 = (int)(k / n), s2 = (int)(k - (long long)s1 * n);
+    for (int i = bf1st[s1]; i < bf1st[s1 + 1]; ++i)
+      for (int j = bf1st[s2]; j < bf1st[s2 + 1]; ++j) m = fmax(m, fabs(D[i * N + j]));
+    Dn[k] = m;
+  }
+  for (int o = 32; o > 0; o >>= 1) m = fmax(m, __shfl_xor(m, o));
+  if ((threadIdx.x & 63) == 0 && m > 0.0) atomicMax(dmax, (unsigned long long)__double_as_longlong(m));
+}
+
 struct Quartet {
   int s1, s2, s3, s4;
   double Dn1234;
@@ -125,27 +143,31 @@ __global__ void __launch_bounds__(kEnumThreads) enum_fill(const l2g_impl::FockEn
     }
 }
 
-template <class T>
-__global__ void gather_kernel(const T* __restrict__ in, const unsigned* __restrict__ perm, T* __restrict__ out,
-                              long long n) {
-  const long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i < n) out[i] = in[perm[i]];
+// the items in sorted order, one launch for their seven arrays
+__global__ void __launch_bounds__(kEnumThreads) gather_items(const l2g_impl::FockEnumOut in,
+                                                             const unsigned* __restrict__ perm,
+                                                             l2g_impl::FockEnumState::Items out, long long n) {
+  const long long k = (long long)blockIdx.x * kEnumThreads + threadIdx.x;
+  if (k >= n) return;
+  const unsigned i = perm[k];
+  const int bra = in.bra[i], ket = in.ket[i], meta = in.meta[i];
+  const double lnp = in.lnp[i], scale = in.scale[i];
+  const int4 bf = in.bf[i];
+  const int2 pr = in.pr[i];
+  out.bra[k] = bra, out.ket[k] = ket, out.meta[k] = meta, out.lnp[k] = lnp, out.scale[k] = scale, out.bf[k] = bf;
+  out.pr[k] = pr;
 }
 
-template <class T>
-void gather(const T* in, const unsigned* perm, T* out, long long n, hipStream_t s) {
-  if (n == 0) return;
-  const int block = 256;
-  hipLaunchKernelGGL(gather_kernel<T>, dim3((unsigned)((n + block - 1) / block)), dim3(block), 0, s, in, perm, out, n);
-  LAUNCHCHK("gather_kernel");
-}
+struct SplitChunks {  // largest piece per class
+  int c[l2g_impl::kEnumClasses];
+};
 
 // Primitive-range split of the sorted items: an item of class c whose
 // primitive loop is longer than chunk[c] becomes ceil(len / chunk[c])
 // consecutive pieces of near-equal length.
 __global__ void __launch_bounds__(kEnumThreads) split_count(long long n, const unsigned* __restrict__ key,
                                                                const int2* __restrict__ pr,
-                                                               const int* __restrict__ chunk,
+                                                               const SplitChunks chunk,
                                                                unsigned* __restrict__ pieces,
                                                                unsigned long long* __restrict__ cls_pieces) {
   __shared__ unsigned int hist[l2g_impl::kEnumClasses];
@@ -154,7 +176,7 @@ __global__ void __launch_bounds__(kEnumThreads) split_count(long long n, const u
   const long long i = (long long)blockIdx.x * kEnumThreads + threadIdx.x;
   if (i < n) {
     const int c = (int)(key[i] >> 13);
-    const int len = pr[i].y - pr[i].x, ch = chunk[c];
+    const int len = pr[i].y - pr[i].x, ch = chunk.c[c];
     const unsigned np = len > ch ? (unsigned)((len + ch - 1) / ch) : 1u;
     pieces[i] = np;
     atomicAdd(&hist[c], np);
@@ -173,14 +195,12 @@ __global__ void __launch_bounds__(kEnumThreads) split_fill(long long n, const un
   const unsigned np = pieces[i];
   const unsigned long long o = at[i];
   const int b = in.pr[i].x, len = in.pr[i].y - b;
+  const int bra = in.bra[i], ket = in.ket[i], meta = in.meta[i];
+  const double lnp = in.lnp[i], scale = in.scale[i];
+  const int4 bf = in.bf[i];
   for (unsigned k = 0; k < np; ++k) {
     const unsigned long long j = o + k;
-    out.bra[j] = in.bra[i];
-    out.ket[j] = in.ket[i];
-    out.meta[j] = in.meta[i];
-    out.lnp[j] = in.lnp[i];
-    out.scale[j] = in.scale[i];
-    out.bf[j] = in.bf[i];
+    out.bra[j] = bra, out.ket[j] = ket, out.meta[j] = meta, out.lnp[j] = lnp, out.scale[j] = scale, out.bf[j] = bf;
     out.pr[j] = int2{b + (int)((long long)len * k / np), b + (int)((long long)len * (k + 1) / np)};
   }
 }
@@ -189,31 +209,68 @@ __global__ void __launch_bounds__(kEnumThreads) split_fill(long long n, const un
 
 namespace l2g_impl {
 
+namespace {
+
+// Ranges of one allocation.
+struct Arena {
+  size_t bytes = 0;
+  char* base = nullptr;
+  size_t add(size_t b) {
+    const size_t at = bytes;
+    bytes += (b + 255) & ~size_t(255);
+    return at;
+  }
+  template <class T>
+  T* at(size_t o) const {
+    return reinterpret_cast<T*>(base + o);
+  }
+};
+
+// Workspaces up to this size stay with the builder from build to build (an
+// allocation and its release cost a small molecule's build 10 us each, and
+// there were 28); larger ones are given back.
+constexpr size_t kKeepBytes = size_t(64) << 20;
+
+void alloc_items(FockEnumState::Bufs& b, size_t n) {
+  b.bra.alloc(n * sizeof(int));
+  b.ket.alloc(n * sizeof(int));
+  b.meta.alloc(n * sizeof(int));
+  b.lnp.alloc(n * sizeof(double));
+  b.scale.alloc(n * sizeof(double));
+  b.bf.alloc(n * sizeof(int4));
+  b.pr.alloc(n * sizeof(int2));
+}
+
+unsigned blocks(long long n) { return (unsigned)((n + kEnumThreads - 1) / kEnumThreads); }
+
+}  // namespace
+
 void fock_split_device(FockEnumState& S, const std::vector<int>& chunk, hipStream_t st) {
   const long long n = S.n;
   S.cls_pieces.assign(kEnumClasses, 0ull);
   if (n == 0) return;
   if ((int)chunk.size() != kEnumClasses) throw L2gError(L2G_E_STATE, "split: one chunk per class expected");
   LAUNCHCHK("work before the item split");
-  DevBuf d_chunk, pieces, at, cls, tmp;
-  d_chunk.alloc(kEnumClasses * sizeof(int));
-  HIPCHK(hipMemcpyAsync(d_chunk.p, chunk.data(), kEnumClasses * sizeof(int), hipMemcpyHostToDevice, st));
-  pieces.alloc((size_t)n * sizeof(unsigned));
-  at.alloc((size_t)n * sizeof(unsigned long long));
-  cls.alloc(kEnumClasses * sizeof(unsigned long long));
-  HIPCHK(hipMemsetAsync(cls.p, 0, kEnumClasses * sizeof(unsigned long long), st));
-  const unsigned nb = (unsigned)((n + kEnumThreads - 1) / kEnumThreads);
-  hipLaunchKernelGGL(split_count, dim3(nb), dim3(kEnumThreads), 0, st, n, S.key.as<unsigned>(), S.pr.as<int2>(),
-                     d_chunk.as<int>(), pieces.as<unsigned>(), cls.as<unsigned long long>());
-  LAUNCHCHK("split_count");
+  SplitChunks sc;
+  std::copy(chunk.begin(), chunk.end(), sc.c);
+  Arena a;
+  const size_t o_pieces = a.add((size_t)n * sizeof(unsigned)), o_at = a.add((size_t)n * sizeof(unsigned long long)),
+               o_cls = a.add(kEnumClasses * sizeof(unsigned long long));
   size_t tmp_bytes = 0;
-  HIPCHK(hipcub::DeviceScan::ExclusiveSum(nullptr, tmp_bytes, pieces.as<unsigned>(), at.as<unsigned long long>(),
-                                          (int)n, st));
-  tmp.alloc(std::max<size_t>(tmp_bytes, 16));
-  HIPCHK(hipcub::DeviceScan::ExclusiveSum(tmp.p, tmp_bytes, pieces.as<unsigned>(), at.as<unsigned long long>(),
-                                          (int)n, st));
-  HIPCHK(hipMemcpyAsync(S.cls_pieces.data(), cls.p, kEnumClasses * sizeof(unsigned long long),
-                        hipMemcpyDeviceToHost, st));
+  HIPCHK(hipcub::DeviceScan::ExclusiveSum(nullptr, tmp_bytes, (unsigned*)nullptr, (unsigned long long*)nullptr, (int)n,
+                                          st));
+  const size_t o_tmp = a.add(std::max<size_t>(tmp_bytes, 16));
+  S.work.alloc(a.bytes);
+  a.base = S.work.as<char>();
+  unsigned* const pieces = a.at<unsigned>(o_pieces);
+  unsigned long long *const at = a.at<unsigned long long>(o_at), *const cls = a.at<unsigned long long>(o_cls);
+  HIPCHK(hipMemsetAsync(cls, 0, kEnumClasses * sizeof(unsigned long long), st));
+  hipLaunchKernelGGL(split_count, dim3(blocks(n)), dim3(kEnumThreads), 0, st, n, S.key.as<unsigned>(),
+                     S.cur.pr.as<int2>(), sc, pieces, cls);
+  LAUNCHCHK("split_count");
+  HIPCHK(hipcub::DeviceScan::ExclusiveSum(a.at<char>(o_tmp), tmp_bytes, pieces, at, (int)n, st));
+  HIPCHK(hipMemcpyAsync(S.cls_pieces.data(), cls, kEnumClasses * sizeof(unsigned long long), hipMemcpyDeviceToHost,
+                        st));
   HIPCHK(hipStreamSynchronize(st));
   unsigned long long total = 0;
   for (int c = 0; c < kEnumClasses; ++c) {
@@ -223,44 +280,51 @@ void fock_split_device(FockEnumState& S, const std::vector<int>& chunk, hipStrea
     total += S.cls_pieces[c];
   }
   if (total >= (1ull << 31)) throw L2gError(L2G_E_INVALID, "more than 2^31 work items in one Fock build");
-  if (total == (unsigned long long)n) return;  // nothing to split
-  FockEnumState::Items in = S.items();
-  DevBuf bra, ket, meta, lnp, scale, bf, pr;
-  bra.alloc(total * sizeof(int));
-  ket.alloc(total * sizeof(int));
-  meta.alloc(total * sizeof(int));
-  lnp.alloc(total * sizeof(double));
-  scale.alloc(total * sizeof(double));
-  bf.alloc(total * sizeof(int4));
-  pr.alloc(total * sizeof(int2));
-  FockEnumState::Items out{bra.as<int>(), ket.as<int>(), meta.as<int>(), lnp.as<double>(), scale.as<double>(),
-                           bf.as<int4>(), pr.as<int2>()};
-  hipLaunchKernelGGL(split_fill, dim3(nb), dim3(kEnumThreads), 0, st, n, pieces.as<unsigned>(),
-                     at.as<unsigned long long>(), in, out);
-  LAUNCHCHK("split_fill");
-  HIPCHK(hipStreamSynchronize(st));  // the inputs are freed on return
-  std::swap(S.bra, bra), std::swap(S.ket, ket), std::swap(S.meta, meta), std::swap(S.lnp, lnp);
-  std::swap(S.scale, scale), std::swap(S.bf, bf), std::swap(S.pr, pr);
-  S.n = (long long)total;
+  if (total != (unsigned long long)n) {  // else nothing to split
+    alloc_items(S.alt, total);
+    hipLaunchKernelGGL(split_fill, dim3(blocks(n)), dim3(kEnumThreads), 0, st, n, pieces, at, S.cur.items(),
+                       S.alt.items());
+    LAUNCHCHK("split_fill");
+    std::swap(S.cur, S.alt);
+    S.n = (long long)total;
+  }
+  if (S.work.bytes > kKeepBytes || S.alt.bytes() > kKeepBytes) {
+    HIPCHK(hipStreamSynchronize(st));
+    S.work = DevBuf();
+    S.alt = FockEnumState::Bufs();
+  }
 }
 
-void fock_count_device(const FockEnumArgs& E, FockEnumState& S, hipStream_t st) {
+void fock_count_device(const FockEnumArgs& E, const double* D, long long nbf, double* Dn, FockEnumState& S,
+                       hipStream_t st) {
   const long long np = E.npairs;
   S.total_t = np * (np + 1) / 2;
   S.block_count.clear();
   S.nblocks = 0;
   S.tchunk = 0;
-  if (S.total_t == 0) return;
-  S.nblocks = (int)std::min<long long>(8192, (S.total_t + kEnumThreads * 64 - 1) / (kEnumThreads * 64));
-  S.tchunk = (S.total_t + S.nblocks - 1) / S.nblocks;
-  S.counts.alloc((size_t)S.nblocks * sizeof(long long));
-  hipLaunchKernelGGL(enum_count, dim3(S.nblocks), dim3(kEnumThreads), 0, st, E, S.total_t, S.tchunk,
-                     S.counts.as<long long>());
-  LAUNCHCHK("enum_count");
-  S.block_count.resize(S.nblocks);
-  HIPCHK(hipMemcpyAsync(S.block_count.data(), S.counts.p, (size_t)S.nblocks * sizeof(long long),
+  S.dmax = 0.0;
+  // 4 quartets a thread in small molecules (64 left a 3-atom molecule one
+  // block: 77 us for its list, now 11), more where 8192 blocks are reached
+  S.nblocks = (int)std::min<long long>(8192, (S.total_t + kEnumThreads * 4 - 1) / (kEnumThreads * 4));
+  if (S.nblocks) S.tchunk = (S.total_t + S.nblocks - 1) / S.nblocks;
+  S.counts.alloc((size_t)(S.nblocks + 1) * sizeof(long long));
+  long long* const counts = S.counts.as<long long>();  // dmax, then a count per block
+  HIPCHK(hipMemsetAsync(counts, 0, sizeof(long long), st));
+  if (E.n) {
+    hipLaunchKernelGGL(shell_norms, dim3(blocks(E.n * E.n)), dim3(kEnumThreads), 0, st, D, nbf, E.bf1st, (int)E.n, Dn,
+                       reinterpret_cast<unsigned long long*>(counts));
+    LAUNCHCHK("shell_norms");
+  }
+  if (S.nblocks) {
+    hipLaunchKernelGGL(enum_count, dim3(S.nblocks), dim3(kEnumThreads), 0, st, E, S.total_t, S.tchunk, counts + 1);
+    LAUNCHCHK("enum_count");
+  }
+  S.block_count.resize(S.nblocks + 1);
+  HIPCHK(hipMemcpyAsync(S.block_count.data(), counts, (size_t)(S.nblocks + 1) * sizeof(long long),
                         hipMemcpyDeviceToHost, st));
   HIPCHK(hipStreamSynchronize(st));
+  std::memcpy(&S.dmax, S.block_count.data(), sizeof(double));
+  S.block_count.erase(S.block_count.begin());
 }
 
 void fock_fill_device(const FockEnumArgs& E, FockEnumState& S, int blk0, int blk1, hipStream_t st) {
@@ -282,70 +346,49 @@ void fock_fill_device(const FockEnumArgs& E, FockEnumState& S, int blk0, int blk
   HIPCHK(hipMemcpyAsync(S.base.p, base.data(), (size_t)nb * sizeof(long long), hipMemcpyHostToDevice, st));
   // unsorted items, then sorted
   const size_t sz = (size_t)n;
-  DevBuf u_bra, u_ket, u_meta, u_lnp, u_scale, u_bf, u_pr, u_key, u_idx, stats;
-  DevBuf& s_key = S.key;
-  u_bra.alloc(sz * sizeof(int));
-  u_ket.alloc(sz * sizeof(int));
-  u_meta.alloc(sz * sizeof(int));
-  u_lnp.alloc(sz * sizeof(double));
-  u_scale.alloc(sz * sizeof(double));
-  u_bf.alloc(sz * sizeof(int4));
-  u_pr.alloc(sz * sizeof(int2));
-  u_key.alloc(sz * sizeof(unsigned));
-  u_idx.alloc(sz * sizeof(unsigned));
-  s_key.alloc(sz * sizeof(unsigned));
-  stats.alloc(2 * kEnumClasses * sizeof(unsigned long long));
-  HIPCHK(hipMemsetAsync(stats.p, 0, 2 * kEnumClasses * sizeof(unsigned long long), st));
+  Arena a;
+  const size_t o_bra = a.add(sz * sizeof(int)), o_ket = a.add(sz * sizeof(int)), o_meta = a.add(sz * sizeof(int)),
+               o_lnp = a.add(sz * sizeof(double)), o_scale = a.add(sz * sizeof(double)),
+               o_bf = a.add(sz * sizeof(int4)), o_pr = a.add(sz * sizeof(int2)), o_key = a.add(sz * sizeof(unsigned)),
+               o_idx = a.add(sz * sizeof(unsigned)), o_perm = a.add(sz * sizeof(unsigned)),
+               o_stats = a.add(2 * kEnumClasses * sizeof(unsigned long long));
+  size_t tmp_bytes = 0;
+  HIPCHK(hipcub::DeviceRadixSort::SortPairs(nullptr, tmp_bytes, (unsigned*)nullptr, (unsigned*)nullptr,
+                                            (unsigned*)nullptr, (unsigned*)nullptr, (int)n, 0, kEnumKeyBits, st));
+  const size_t o_tmp = a.add(std::max<size_t>(tmp_bytes, 16));
+  S.work.alloc(a.bytes);
+  a.base = S.work.as<char>();
+  S.key.alloc(sz * sizeof(unsigned));
+  alloc_items(S.cur, sz);
   FockEnumOut O;
-  O.bra = u_bra.as<int>();
-  O.ket = u_ket.as<int>();
-  O.meta = u_meta.as<int>();
-  O.lnp = u_lnp.as<double>();
-  O.scale = u_scale.as<double>();
-  O.bf = u_bf.as<int4>();
-  O.pr = u_pr.as<int2>();
-  O.key = u_key.as<unsigned>();
-  O.idx = u_idx.as<unsigned>();
-  O.cls_count = stats.as<unsigned long long>();
-  O.cls_nprim = stats.as<unsigned long long>() + kEnumClasses;
+  O.bra = a.at<int>(o_bra);
+  O.ket = a.at<int>(o_ket);
+  O.meta = a.at<int>(o_meta);
+  O.lnp = a.at<double>(o_lnp);
+  O.scale = a.at<double>(o_scale);
+  O.bf = a.at<int4>(o_bf);
+  O.pr = a.at<int2>(o_pr);
+  O.key = a.at<unsigned>(o_key);
+  O.idx = a.at<unsigned>(o_idx);
+  O.cls_count = a.at<unsigned long long>(o_stats);
+  O.cls_nprim = O.cls_count + kEnumClasses;
+  HIPCHK(hipMemsetAsync(O.cls_count, 0, 2 * kEnumClasses * sizeof(unsigned long long), st));
   hipLaunchKernelGGL(enum_fill, dim3(nb), dim3(kEnumThreads), 0, st, E, S.total_t, S.tchunk, (long long)blk0,
                      S.base.as<long long>(), O);
   LAUNCHCHK("enum_fill");
   // sort the item indices by (class, decreasing depth)
-  S.perm.alloc(sz * sizeof(unsigned));
-  size_t tmp_bytes = 0;
-  HIPCHK(hipcub::DeviceRadixSort::SortPairs(nullptr, tmp_bytes, O.key, s_key.as<unsigned>(), O.idx,
-                                            S.perm.as<unsigned>(), (int)n, 0, kEnumKeyBits, st));
-  DevBuf tmp;
-  tmp.alloc(std::max<size_t>(tmp_bytes, 16));
-  HIPCHK(hipcub::DeviceRadixSort::SortPairs(tmp.p, tmp_bytes, O.key, s_key.as<unsigned>(), O.idx,
-                                            S.perm.as<unsigned>(), (int)n, 0, kEnumKeyBits, st));
-  const unsigned* perm = S.perm.as<unsigned>();
-  S.bra.alloc(sz * sizeof(int));
-  S.ket.alloc(sz * sizeof(int));
-  S.meta.alloc(sz * sizeof(int));
-  S.lnp.alloc(sz * sizeof(double));
-  S.scale.alloc(sz * sizeof(double));
-  S.bf.alloc(sz * sizeof(int4));
-  S.pr.alloc(sz * sizeof(int2));
-  gather(O.bra, perm, S.bra.as<int>(), n, st);
-  gather(O.ket, perm, S.ket.as<int>(), n, st);
-  gather(O.meta, perm, S.meta.as<int>(), n, st);
-  gather(O.lnp, perm, S.lnp.as<double>(), n, st);
-  gather(O.scale, perm, S.scale.as<double>(), n, st);
-  gather(O.bf, perm, S.bf.as<int4>(), n, st);
-  gather(O.pr, perm, S.pr.as<int2>(), n, st);
+  HIPCHK(hipcub::DeviceRadixSort::SortPairs(a.at<char>(o_tmp), tmp_bytes, O.key, S.key.as<unsigned>(), O.idx,
+                                            a.at<unsigned>(o_perm), (int)n, 0, kEnumKeyBits, st));
+  hipLaunchKernelGGL(gather_items, dim3(blocks(n)), dim3(kEnumThreads), 0, st, O, a.at<unsigned>(o_perm),
+                     S.cur.items(), n);
+  LAUNCHCHK("gather_items");
   std::vector<unsigned long long> h(2 * kEnumClasses);
-  HIPCHK(hipMemcpyAsync(h.data(), stats.p, 2 * kEnumClasses * sizeof(unsigned long long), hipMemcpyDeviceToHost,
+  HIPCHK(hipMemcpyAsync(h.data(), O.cls_count, 2 * kEnumClasses * sizeof(unsigned long long), hipMemcpyDeviceToHost,
                         st));
-  HIPCHK(hipStreamSynchronize(st));  // the temporaries are freed on return
+  HIPCHK(hipStreamSynchronize(st));
+  if (S.work.bytes > kKeepBytes) S.work = DevBuf();
   for (int c = 0; c < kEnumClasses; ++c) S.cls_count[c] = h[c], S.cls_nprim[c] = h[kEnumClasses + c];
   if (S.cls_count[kEnumClasses - 1]) throw L2gError(L2G_E_LMAX, "no Fock kernel for an angular momentum class");
-}
-
-void fock_enumerate_device(const FockEnumArgs& E, FockEnumState& S, hipStream_t st) {
-  fock_count_device(E, S, st);
-  fock_fill_device(E, S, 0, S.nblocks, st);
 }
 
 }  // namespace l2g_impl

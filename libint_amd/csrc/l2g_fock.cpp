@@ -730,30 +730,19 @@ int l2g_fock_schwarz(l2g_fock f, double* K) {
 
 namespace {
 
-// The count pass of a build: shell-block norms of D, then the screened
-// unique quartets counted on the GPU per enumeration block (f->enumst).
+// The count pass of a build, on the GPU: D into f->dens, its shell-block
+// norms (compute_shellblock_norm), and the screened unique quartets counted
+// per enumeration block (f->enumst).
 FockEnumArgs fock_count_pass(l2g_fock_s* f, const double* D, double precision) {
   const FockSetup& fs = f->setup;
   l2g_context_s* ctx = fs.B->ctx;
   HIPCHK(hipSetDevice(ctx->device));
-  const int n = fs.n, N = fs.nbf;
+  const int n = fs.n;
+  const size_t NN = (size_t)fs.nbf * fs.nbf;
   hipStream_t st = ctx->stream;
-  // shell-block infinity norms of D (compute_shellblock_norm)
-  std::vector<double> Dn((size_t)n * n, 0.0);
-  parallel_for(n, [&](int s1) {
-    for (int s2 = 0; s2 < n; ++s2) {
-      double m = 0;
-      for (int i = fs.bf1st[s1]; i < fs.bf1st[s1 + 1]; ++i)
-        for (int j = fs.bf1st[s2]; j < fs.bf1st[s2 + 1]; ++j) m = std::max(m, std::fabs(D[(size_t)i * N + j]));
-      Dn[(size_t)s1 * n + s2] = m;
-    }
-  });
-  double dmax = 0;
-  for (double v : Dn) dmax = std::max(dmax, v);
-  const double needed = dmax > 0 ? precision / dmax : precision;
-  if (needed < fs.max_engine_precision)
-    throw std::invalid_argument("requested Fock precision needs more engine precision than the shell-pair data hold");
-  upload(f->e_Dn, Dn, st);
+  f->dens.alloc(std::max<size_t>(NN, 1) * sizeof(double));
+  if (NN) HIPCHK(hipMemcpyAsync(f->dens.p, D, NN * sizeof(double), hipMemcpyHostToDevice, st));
+  f->e_Dn.alloc(std::max<size_t>((size_t)n * n, 1) * sizeof(double));
   // screened unique quartets on the GPU, sorted by class and depth
   FockEnumArgs E;
   E.ps1 = f->e_ps1.as<int>();
@@ -772,11 +761,14 @@ FockEnumArgs fock_count_pass(l2g_fock_s* f, const double* D, double precision) {
   E.clsmap = f->e_cls.as<int>();
   E.cls32map = f->e_cls32.as<int>();
   E.precision = precision;
-  E.needed = needed;
+  E.needed = 0.0;
   E.fp32_thr = f->fp32_threshold;
   E.hrr_factor = L2G_FP32_HRR_FACTOR;
   FockEnumState& es = f->enumst;
-  fock_count_device(E, es, st);  // synchronises; Dn may go
+  fock_count_device(E, f->dens.as<double>(), fs.nbf, f->e_Dn.as<double>(), es, st);
+  E.needed = es.dmax > 0 ? precision / es.dmax : precision;
+  if (E.needed < fs.max_engine_precision)
+    throw std::invalid_argument("requested Fock precision needs more engine precision than the shell-pair data hold");
   return E;
 }
 
@@ -815,14 +807,12 @@ int l2g_fock_build(l2g_fock f, const double* D, double precision, double* J, dou
     f->cls_nprim.assign(ncls, 0);
     f->cls_ms.assign(ncls, 0.0f);
     const size_t NN = (size_t)N * N;
-    f->dens.alloc(std::max<size_t>(NN, 1) * sizeof(double));
     // deterministic digest: a plane of low words, then one of high words
     const size_t planes = f->deterministic ? 2 : 1;
     const long long hoff = f->deterministic ? (long long)NN : 0;
     f->jg.alloc(std::max<size_t>(planes * NN, 1) * sizeof(double));
     f->kg.alloc(std::max<size_t>(planes * NN, 1) * sizeof(double));
     if (NN) {
-      HIPCHK(hipMemcpyAsync(f->dens.p, D, NN * sizeof(double), hipMemcpyHostToDevice, st));
       HIPCHK(hipMemsetAsync(f->jg.p, 0, planes * NN * sizeof(double), st));
       HIPCHK(hipMemsetAsync(f->kg.p, 0, planes * NN * sizeof(double), st));
     }
@@ -858,9 +848,9 @@ int l2g_fock_build(l2g_fock f, const double* D, double precision, double* J, dou
       // deep items cut by primitive range on the device (class-major order kept)
       fock_split_device(es, chunk, st);
       ItemsView big;
-      big.bra = es.bra.as<int>(), big.ket = es.ket.as<int>(), big.meta = es.meta.as<int>();
-      big.lnp = es.lnp.as<double>(), big.scale = es.scale.as<double>(), big.bf = es.bf.as<int4>();
-      big.pr = es.pr.as<int2>();
+      const FockEnumState::Items ei = es.cur.items();
+      big.bra = ei.bra, big.ket = ei.ket, big.meta = ei.meta, big.lnp = ei.lnp, big.scale = ei.scale, big.bf = ei.bf;
+      big.pr = ei.pr;
       big.first.assign(ncls, 0);
       big.count.assign(ncls, 0);
       int64_t o = 0;

@@ -500,22 +500,32 @@ struct FockEnumState {
   long long n = 0;  // items of the filled window (after fock_split_device: pieces)
   std::vector<unsigned long long> cls_count, cls_nprim;  // kEnumClasses classes
   std::vector<unsigned long long> cls_pieces;            // per class, after the split
-  DevBuf counts, base, perm, key, bra, ket, meta, lnp, scale, bf, pr;
+  double dmax = 0.0;  // largest |D| of the count pass
   struct Items {
     int *bra, *ket, *meta;
     double *lnp, *scale;
     int4* bf;
     int2* pr;
   };
-  Items items() {
-    return Items{bra.as<int>(), ket.as<int>(), meta.as<int>(), lnp.as<double>(), scale.as<double>(), bf.as<int4>(),
-                 pr.as<int2>()};
-  }
+  struct Bufs {
+    DevBuf bra, ket, meta, lnp, scale, bf, pr;
+    Items items() {
+      return Items{bra.as<int>(), ket.as<int>(), meta.as<int>(), lnp.as<double>(), scale.as<double>(), bf.as<int4>(),
+                   pr.as<int2>()};
+    }
+    size_t bytes() const {
+      return bra.bytes + ket.bytes + meta.bytes + lnp.bytes + scale.bytes + bf.bytes + pr.bytes;
+    }
+  };
+  Bufs cur, alt;  // the sorted items; the split's other side
+  DevBuf counts, base, key, work;
 };
-void fock_enumerate_device(const FockEnumArgs& E, FockEnumState& S, hipStream_t st);
-// the same in two steps: the count pass over the whole triangular range, then
-// the items of count-pass blocks [blk0, blk1) (a window), sorted
-void fock_count_device(const FockEnumArgs& E, FockEnumState& S, hipStream_t st);
+// Two steps: the shell-block norms Dn of the device density D (nbf x nbf) and
+// the count pass over the whole triangular range, then the items of
+// count-pass blocks [blk0, blk1) (a window), sorted.  E.needed enters the
+// second step only.
+void fock_count_device(const FockEnumArgs& E, const double* D, long long nbf, double* Dn, FockEnumState& S,
+                       hipStream_t st);
 void fock_fill_device(const FockEnumArgs& E, FockEnumState& S, int blk0, int blk1, hipStream_t st);
 // Splits the enumerated items by primitive range, chunk[c] primitives at most
 // per piece of class c (kEnumClasses entries); pieces stay class-major.

@@ -188,3 +188,20 @@ def test_fock_digest_shapes(ctx, pure, gauss):
     finally:
         ctx.set_solid_harmonics_ordering(la.SHG_STANDARD)
         oracle.set_shg_ordering(False)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("n", [1, 2, 9, 10])
+def test_fock_quartet_list_sizes(ctx, n):
+    """Quartet lists of 1, 6, 1035 and 1540: one enumeration block holds 1024;
+    two builds on one builder share its workspaces."""
+    rng = np.random.default_rng(n)
+    sh = [x for k in range(n) for x in shells(rng, (k % 3,), (1 + k % 2,), True)]
+    say(f"case: Fock build of {n} shells")
+    fock_check(ctx, sh, n)
+    arrays = la.BasisArrays.from_shells(sh)
+    fb = la.FockBuilder(la.Basis(ctx, arrays))
+    N = int(arrays.sizes().sum())
+    one = [fb.build(s * np.eye(N), 1e-12) for s in (1.0, 1e-3, 1.0)]
+    for x, y in zip(one[0], one[2]):
+        assert np.abs(x - y).max() <= 1e-9
