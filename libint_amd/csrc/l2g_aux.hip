@@ -150,6 +150,49 @@ void launch_deriv1_combine(const double* raw, const long long* raw_off, const lo
   LAUNCHCHK("l2g_deriv1_combine_kernel");
 }
 
+namespace {
+
+__global__ void __launch_bounds__(64) schwarz_reduce_kernel(const long long* __restrict__ off,
+                                                            const double* __restrict__ vals, int norm,
+                                                            const int* __restrict__ first,
+                                                            const double* __restrict__ gpart, long long stride, int ne,
+                                                            const long long* __restrict__ idx,
+                                                            double* __restrict__ out, double* __restrict__ out2) {
+  const int i = blockIdx.x;
+  double m = 0.0, q = 0.0, h = 0.0;
+  for (long long k = off[i] + threadIdx.x; k < off[i + 1]; k += 64) {
+    const double v = vals[k];
+    m = fmax(m, fabs(v));
+    q = fma(v, v, q);
+  }
+  if (out2)
+    for (int e = threadIdx.x; e < ne; e += 64) {
+      double s = 0.0;
+      for (int x = first[i]; x < first[i + 1]; ++x) s += gpart[x * stride + (long long)e * ne + e];
+      h = fmax(h, fabs(s));
+    }
+  for (int o = 32; o > 0; o >>= 1) {
+    m = fmax(m, __shfl_xor(m, o));
+    q += __shfl_xor(q, o);
+    h = fmax(h, __shfl_xor(h, o));
+  }
+  if (threadIdx.x == 0) {
+    out[idx[i]] = norm ? sqrt(sqrt(q)) : sqrt(m);
+    if (out2) out2[idx[i]] = sqrt(h);
+  }
+}
+
+}  // namespace
+
+void launch_schwarz_reduce(int n, const long long* off, const double* vals, int norm, const int* first,
+                           const double* gpart, long long stride, int ne, const long long* idx, double* out,
+                           double* out2, hipStream_t s) {
+  if (n <= 0) return;
+  hipLaunchKernelGGL(schwarz_reduce_kernel, dim3((unsigned)n), dim3(64), 0, s, off, vals, norm, first, gpart, stride,
+                     ne, idx, out, out2);
+  LAUNCHCHK("schwarz_reduce_kernel");
+}
+
 void launch_fock_finish(double* jg, double* kg, double* g, long long N, long long hoff, hipStream_t s) {
   if (N <= 0) return;
   const long long n = N * N;

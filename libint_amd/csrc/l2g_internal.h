@@ -403,6 +403,14 @@ namespace l2g_impl {
 void schwarz_impl(l2g_basis B, int64_t npairs, const int32_t* pairs, double precision, int norm, double* K,
                   double* S);
 
+// l2g_aux.hip: Schwarz factors of n pairs from their (p|p) blocks
+// vals[off[i], off[i + 1]) (norm 0: sqrt(max|v|), 1: the Frobenius norm's
+// root) to out[idx[i]], and with out2 sqrt(max |[e0|e0]|) from the pieces
+// [first[i], first[i + 1]) of their ne x ne contracted values.
+void launch_schwarz_reduce(int n, const long long* off, const double* vals, int norm, const int* first,
+                           const double* gpart, long long stride, int ne, const long long* idx, double* out,
+                           double* out2, hipStream_t s);
+
 // l2g_aux.hip: in-place Fock symmetrisation of one N x N block (J into jg,
 // K into kg, G = 2J - K into g)
 // hoff: 0 for FP64 accumulators; else the fixed-point accumulators' offset
