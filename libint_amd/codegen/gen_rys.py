@@ -330,9 +330,11 @@ def emit(p, mode):
     E("I.pend = npb * I.npk;")
     E("if (A.q_prange) I.pbeg = A.q_prange[qi].x, I.pend = A.q_prange[qi].y;")
     if mode == 'eri':
+        E("I.pbeg <<= A.erfc, I.pend <<= A.erfc;")
+    if mode == 'eri':
         E.block("if (S > 1)")
         E("const int b = I.pbeg, n = I.pend - b, k = tid % S;")
-        E("I.pbeg = b + n * k / S, I.pend = b + n * (k + 1) / S;")
+        E("I.pbeg = b + (int)((long long)n * k / S), I.pend = b + (int)((long long)n * (k + 1) / S);")
         E.end()
     if mode == 'fock':
         E("I.lnprec = A.q_lnprec[qi];")

@@ -104,6 +104,7 @@ struct L2gEriArgs {
   int coop;          // Schwarz kernels: one wave per pair, its lanes splitting the primitive loop
   int win;           // per-lane ERI and Fock kernels: work items of a wave's window (0: 64)
   double omega;      // > 0: erf-attenuated Coulomb erf(omega r)/r (0: Coulomb)
+  int erfc;          // Rys ERI kernels, with omega > 0: 1 = erfc(omega r)/r in one pass, else 0
   int store_sub;     // ERI kernels: subtract from the output instead of storing
   double* __restrict__ out;
   double* __restrict__ ybuf;

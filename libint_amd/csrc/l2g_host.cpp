@@ -891,7 +891,8 @@ int l2g_eri_plan_execute(l2g_eri_plan p, double* d_out) {
     // runs on the Coulomb kernels.
     // Passes (attenuation, subtract): Coulomb; erf = one attenuated pass
     // (omega = 0 gives exact zeros as Coulomb minus Coulomb); erfc =
-    // Coulomb minus the erf pass, both per class on the class's stream
+    // Coulomb minus the erf pass, both per class on the class's stream, or
+    // one pass over both on a Rys kernel (rys_prim)
     std::vector<std::pair<double, int>> passes;
     if (p->oper == 0) passes = {{0.0, 0}};
     else if (p->oper == 1) passes = p->omega > 0 ? std::vector<std::pair<double, int>>{{p->omega, 0}}
@@ -901,7 +902,11 @@ int l2g_eri_plan_execute(l2g_eri_plan p, double* d_out) {
     auto launch_classes = [&] {
     for (auto& c : p->classes) {
     for (size_t ps = 0; ps < passes.size(); ++ps) {
-      A.omega = passes[ps].first;
+      const bool erfc = c.rys >= 0 && p->oper == 2 && p->omega > 0;
+      if (erfc && ps) continue;
+      const bool last = erfc || ps + 1 == passes.size();
+      A.omega = erfc ? p->omega : passes[ps].first;
+      A.erfc = erfc;
       A.store_sub = passes[ps].second;
       hipStream_t cs = sides && c.slot.side >= 0 ? ctx->side[c.slot.side] : ctx->stream;
       A.ybuf = p->ybuf.as<double>() + c.slot.yoff;
@@ -936,7 +941,7 @@ int l2g_eri_plan_execute(l2g_eri_plan p, double* d_out) {
         if (!c.npieces) P.rys_deep[0] = c.rys_deep[0], P.rys_deep[1] = c.rys_deep[1];
         ci.launch(P, 0, 0, cs);
         LAUNCHCHK(std::string("Rys ERI kernel of class ") + std::to_string(c.rys));
-        if (!capture && ps + 1 == passes.size()) HIPCHK(hipEventRecord(c.ev1, cs));
+        if (!capture && last) HIPCHK(hipEventRecord(c.ev1, cs));
         continue;
       }
       int erf_idx = -1;  // the class's erf-attenuated register kernel, for an attenuated pass
@@ -984,7 +989,7 @@ int l2g_eri_plan_execute(l2g_eri_plan p, double* d_out) {
         ci.launch(A, c.slot.grid, p->block, cs);
         LAUNCHCHK(std::string("ERI kernel of class ") + std::to_string(c.cls));
       }
-      if (!capture && ps + 1 == passes.size()) HIPCHK(hipEventRecord(c.ev1, cs));
+      if (!capture && last) HIPCHK(hipEventRecord(c.ev1, cs));
     }
     }
     };

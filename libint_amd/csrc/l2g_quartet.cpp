@@ -226,6 +226,10 @@ void quartet_compute_impl(l2g_context_s* ctx, const QuartetBuffers& qb, const in
                                          : std::vector<std::pair<double, int>>{{0.0, 0}, {0.0, 1}};
   else passes = omega > 0 ? std::vector<std::pair<double, int>>{{0.0, 0}, {omega, 1}}
                           : std::vector<std::pair<double, int>>{{0.0, 0}};
+  if (rys >= 0 && oper == 2 && omega > 0) {  // erfc in one pass
+    passes = {{omega, 0}};
+    A.erfc = 1;
+  }
   for (const auto& ps : passes) {
     A.omega = ps.first;
     A.store_sub = ps.second;

@@ -122,8 +122,12 @@ __device__ __forceinline__ double rys_piece_sum(const double* __restrict__ g, lo
 
 // Primitive quartet p of an item: screening as the per-lane kernels do it,
 // and the record.  Past the item's end (act false) a stand-in with prefactor 0.
+// erfc(w r)/r takes each primitive quartet twice, p even with 1/r and p odd
+// with -erf(w r)/r: the sums are never larger than the values, and one launch
+// does both operators.
 __device__ __forceinline__ void rys_prim(const L2gEriArgs& A, RysItem& I, int p, double* rec) {
-  const bool act = p < I.pend;
+  const bool act = p < I.pend, erf = A.omega > 0 && (!A.erfc || (p & 1));
+  p >>= A.erfc;
   // p / npk: the half keeps the product off the integers by more than its rounding error
   const int ib = act ? (int)(((double)p + 0.5) * I.rnpk) : 0;
   const int gb = act ? I.pb0 + ib : 0, gk = act ? I.pk0 + (p - ib * I.npk) : 0;
@@ -143,12 +147,12 @@ __device__ __forceinline__ void rys_prim(const L2gEriArgs& A, RysItem& I, int p,
   double goq = Q.w * oos, gop = P.w * oos;
   const double rho = P.w * Q.w * oos;
   double T = rho * fma(PQz, PQz, fma(PQy, PQy, PQx * PQx));
-  if (A.omega > 0) {  // erf(w r)/r: nodes s u(sT), weights sqrt(s) w(sT), s = w^2 / (w^2 + rho)
+  if (erf) {  // erf(w r)/r: nodes s u(sT), weights sqrt(s) w(sT), s = w^2 / (w^2 + rho)
     const double s = A.omega * A.omega / fma(A.omega, A.omega, rho);
     T *= s;
     goq *= s;  // the nodes enter as u goq and u gop only
     gop *= s;
-    pf *= sqrt(s);
+    pf *= A.erfc ? -sqrt(s) : sqrt(s);
   }
   if (ok) I.nsurv = 1;
   rec[0] = PA.x, rec[1] = QC.x, rec[2] = PQx;
