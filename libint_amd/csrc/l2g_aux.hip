@@ -50,11 +50,27 @@ __device__ __forceinline__ int l2g_cart_index(int l, int a, int b) { return (l -
 // out[d * total + out_off[q] + f], f row-major over the four shells' output
 // functions in caller order (the layout of Engine::results()[d] for
 // deriv_order = 1, include/libint2/engine.h:779-781).  A block per quartet
-// takes the 12 derivatives one at a time: the Cartesian block (two loads
-// per element) into LDS, then one centre's solid-harmonic rows after the
-// other between two LDS buffers, then the store.  Shells up to l = 2 (the
-// raised ones up to 3): at most 6^4 Cartesian elements.
+// takes as many of the 12 derivatives at a time as its buffers hold, all of
+// them for most classes: the Cartesian blocks (two loads per element) into
+// LDS, then one centre's solid-harmonic rows after the other between two LDS
+// buffers, then the store.  Bound by the barriers' and loads' latency: one
+// derivative at a time (60 barriers a quartet, integer divisions for every
+// index) took 450 us for 20,000 s/p/d quartets, this 190.  Shells up to l = 2
+// (the raised ones up to 3): at most 6^4 Cartesian elements.
 constexpr int kDerivMaxCart = 1296;
+
+// x / n and the remainder for x < 2^21: the half keeps the product further
+// from the integers than its rounding error
+struct FastDiv {
+  int n;
+  float r;
+  __device__ __forceinline__ explicit FastDiv(int n_) : n(n_), r(1.0f / (float)n_) {}
+  __device__ __forceinline__ int div(int& x) const {  // x: the remainder
+    const int q = (int)(((float)x + 0.5f) * r);
+    x -= q * n;
+    return q;
+  }
+};
 
 __global__ void __launch_bounds__(256) l2g_deriv1_combine_kernel(const double* __restrict__ raw,
                                                                  const long long* __restrict__ raw_off,
@@ -63,78 +79,85 @@ __global__ void __launch_bounds__(256) l2g_deriv1_combine_kernel(const double* _
                                                                  long long total, double* __restrict__ out,
                                                                  l2g_impl::L2gDerivTab tab) {
   __shared__ double buf[2][kDerivMaxCart];
+  __shared__ long long ro[8];
+  __shared__ double coef[3 * 7 * 4];  // rows of l = 0 .. 2, from the argument once: a load per use is far slower
+  __shared__ signed char cidx[3 * 7 * 4], nnz[3 * 7];
   const long long q = blockIdx.x;
   if (q >= nq) return;
   const int info = qinfo[q];
-  int l[4], pure[4], nc[4];
-  for (int k = 0; k < 4; ++k) {
-    l[k] = (info >> (4 * k)) & 15;
-    pure[k] = (info >> (16 + k)) & 1;
-    nc[k] = (l[k] + 1) * (l[k] + 2) / 2;
+  if (threadIdx.x < 3 * 7 * 4) {
+    const int i = threadIdx.x / 28, m = threadIdx.x / 4 % 7, a = threadIdx.x & 3;
+    coef[threadIdx.x] = tab.coef[i][m][a];
+    cidx[threadIdx.x] = tab.cidx[i][m][a];
+    if (a == 0) nnz[threadIdx.x / 4] = tab.nnz[i][m];
+  } else if (threadIdx.x >= 128 && threadIdx.x < 136) {
+    ro[threadIdx.x - 128] = raw_off[(threadIdx.x - 128) * nq + q];
   }
+  __syncthreads();
+  auto lof = [&](int k) { return (info >> (4 * k)) & 15; };
+  int nc[4];
+#pragma unroll
+  for (int k = 0; k < 4; ++k) nc[k] = (lof(k) + 1) * (lof(k) + 2) / 2;
   const int ncart = nc[0] * nc[1] * nc[2] * nc[3];
   const long long obase = out_off[q];
-  for (int d = 0; d < 12; ++d) {
-    const int k = d / 3, ax = d - 3 * k;
-    const double* rb = raw + raw_off[(long long)k * nq + q];
-    const double* lb = raw + raw_off[(long long)(4 + k) * nq + q];
-    int dp[4], dm[4];
-    for (int j = 0; j < 4; ++j) dp[j] = dm[j] = nc[j];
-    dp[k] = (l[k] + 2) * (l[k] + 3) / 2;
-    dm[k] = l[k] * (l[k] + 1) / 2;
-    // Cartesian derivative block
-    for (int idx = threadIdx.x; idx < ncart; idx += blockDim.x) {
-      int c[4], f = idx;
-      for (int j = 3; j >= 0; --j) {
-        c[j] = f % nc[j];
-        f /= nc[j];
-      }
-      int r = 0;
-      while ((r + 1) * (r + 2) / 2 <= c[k]) ++r;
-      int e[3];
-      e[2] = c[k] - r * (r + 1) / 2;
-      e[1] = r - e[2];
-      e[0] = l[k] - r;
-      int cu[4] = {c[0], c[1], c[2], c[3]};
-      ++e[ax];
-      cu[k] = l2g_cart_index(l[k] + 1, e[0], e[1]);
-      --e[ax];
-      double v = rb[((long long)(cu[0] * dp[1] + cu[1]) * dp[2] + cu[2]) * dp[3] + cu[3]];
-      if (e[ax] > 0) {
-        const int nx = e[ax];
-        --e[ax];
-        cu[k] = l2g_cart_index(l[k] - 1, e[0], e[1]);
-        v -= nx * lb[((long long)(cu[0] * dm[1] + cu[1]) * dm[2] + cu[2]) * dm[3] + cu[3]];
-      }
-      buf[0][idx] = v;
+  const FastDiv dcart(ncart), d1(nc[1]), d2(nc[2]), d3(nc[3]);
+  // as many derivatives at a time as the buffers hold
+  const int most = min(12, kDerivMaxCart / ncart);
+  for (int d0 = 0; d0 < 12; d0 += most) {
+    const int nd = min(most, 12 - d0);
+    // Cartesian derivative blocks
+    for (int it = threadIdx.x; it < nd * ncart; it += blockDim.x) {
+      int f = it;
+      const int d = d0 + dcart.div(f), k = d / 3, ax = d - 3 * k;
+      int c3 = f;
+      int c2 = d3.div(c3), c1 = d2.div(c2);
+      const int c0 = d1.div(c1);
+      const int lk = lof(k), ck = k == 0 ? c0 : k == 1 ? c1 : k == 2 ? c2 : c3;
+      const int r = (ck >= 1) + (ck >= 3) + (ck >= 6);
+      const int ez = ck - r * (r + 1) / 2, ey = r - ez, ex = lk - r;
+      const int dp = (lk + 2) * (lk + 3) / 2, dm = lk * (lk + 1) / 2;
+      auto at = [&](int dk, int u) {  // element with component u (of dk) on centre k
+        const int a0 = k == 0 ? u : c0, a1 = k == 1 ? u : c1, a2 = k == 2 ? u : c2, a3 = k == 3 ? u : c3;
+        return ((a0 * (k == 1 ? dk : nc[1]) + a1) * (k == 2 ? dk : nc[2]) + a2) * (k == 3 ? dk : nc[3]) + a3;
+      };
+      double v = raw[ro[k] + at(dp, l2g_cart_index(lk + 1, ex + (ax == 0), ey + (ax == 1)))];
+      const int nx = ax == 0 ? ex : ax == 1 ? ey : ez;
+      if (nx > 0) v -= nx * raw[ro[4 + k] + at(dm, l2g_cart_index(lk - 1, ex - (ax == 0), ey - (ax == 1)))];
+      buf[0][it] = v;
     }
     __syncthreads();
     // solid-harmonic rows, one pure centre at a time
     int dims[4] = {nc[0], nc[1], nc[2], nc[3]};
     int cur = 0;
+#pragma unroll
     for (int j = 0; j < 4; ++j) {
-      if (!pure[j]) continue;
-      const int nout_j = 2 * l[j] + 1;
-      int inner = 1;
-      for (int t = j + 1; t < 4; ++t) inner *= dims[t];
-      int outer = 1;
-      for (int t = 0; t < j; ++t) outer *= dims[t];
-      const int n_new = outer * nout_j * inner;
-      for (int idx = threadIdx.x; idx < n_new; idx += blockDim.x) {
-        const int i_in = idx % inner, rest = idx / inner;
-        const int m = rest % nout_j, o = rest / nout_j;
+      if (!((info >> (16 + j)) & 1)) continue;
+      const int lj = lof(j), nout_j = 2 * lj + 1;
+      int inner = 1, outer = nd;
+#pragma unroll
+      for (int t = 0; t < 4; ++t) (t > j ? inner : outer) *= t == j ? 1 : dims[t];
+      const FastDiv di(inner), dm(nout_j);
+      for (int it = threadIdx.x; it < outer * nout_j * inner; it += blockDim.x) {
+        int i_in = it;
+        int m = di.div(i_in);
+        const int o = dm.div(m);
         double s = 0.0;
-        for (int a = 0; a < tab.nnz[l[j]][m]; ++a)
-          s += tab.coef[l[j]][m][a] * buf[cur][(o * dims[j] + tab.cidx[l[j]][m][a]) * inner + i_in];
-        buf[cur ^ 1][idx] = s;
+        const int row = lj * 7 + m, n = nnz[row];
+        for (int a = 0; a < n; ++a)
+          s += coef[4 * row + a] * buf[cur][(o * dims[j] + cidx[4 * row + a]) * inner + i_in];
+        buf[cur ^ 1][it] = s;
       }
       dims[j] = nout_j;
       cur ^= 1;
       __syncthreads();
     }
     const int nout = dims[0] * dims[1] * dims[2] * dims[3];
-    double* dst = out + (long long)d * total + obase;
-    for (int idx = threadIdx.x; idx < nout; idx += blockDim.x) dst[idx] = buf[cur][idx];
+    const FastDiv dn(nout);
+    for (int it = threadIdx.x; it < nd * nout; it += blockDim.x) {
+      int i = it;
+      const int d = dn.div(i);
+      out[(long long)(d0 + d) * total + obase + i] = buf[cur][it];
+    }
     __syncthreads();
   }
 }
