@@ -257,6 +257,12 @@ int64_t fock_lanes(const l2g_context_s* ctx, int c, int64_t m) {
   const int per = fock_info(c).lanes;
   return per ? m * per : l2g_window_lanes(m, ctx->ncu);
 }
+// expected work of m items with nprim primitive quartets in all: lane
+// operations, a digest about as long as ten primitive quartets
+double fock_cost(int c, int64_t m, int64_t nprim) {
+  const double per = fock_is_generic(c) ? 10.0 * fock_gclass(c).nvals : (double)fock_info(c).nodes;
+  return per * ((double)nprim + 10.0 * (double)m);
+}
 int fock_ybuf(int c) { return fock_is_generic(c) ? 0 : fock_info(c).ybuf_doubles; }
 
 // The screened unique quartets of one Fock build, by kernel class.
@@ -537,34 +543,24 @@ struct ItemsDev {
   }
 };
 
-// Launches every non-empty class of `items` with the common arguments A;
-// grid and scratch as sized by the caller.
-// With `ev` (2 events per class), records the class's launch between
-// ev[2c] and ev[2c+1].
-// Launches every class of an item set.  With slots (plan_slots over the
-// classes), each class gets its own grid and scratch region, and the classes
-// too small to fill the chip run on the side streams beside each other;
-// without, every class runs in order on st with the scratch in A.
-void fock_launch_all(l2g_context_s* ctx, L2gEriArgs A, const ItemsView& items, bool with_req, int grid, int block,
-                     hipStream_t st, hipEvent_t* ev = nullptr, const std::vector<ClassSlot>* slots = nullptr) {
+// Launches the classes of an item set in the order `launch`, each with its
+// grid, scratch region and stream (plan_slots).  With `ev` (2 events per
+// class), records the class's launch between ev[2c] and ev[2c+1].
+void fock_launch_all(l2g_context_s* ctx, L2gEriArgs A, const ItemsView& items, bool with_req, int block,
+                     hipStream_t st, hipEvent_t* ev, const std::vector<ClassSlot>& slots,
+                     const std::vector<int>& launch) {
   double* const ybase = A.ybuf;
   bool sides = false;
-  if (slots)
-    for (size_t c = 0; c < items.count.size(); ++c) sides |= items.count[c] > 0 && (*slots)[c].side >= 0;
+  for (int c : launch) sides |= slots[(size_t)c].side >= 0;
   if (sides) fork_sides(*ctx);
   try {
-  for (size_t c = 0; c < items.count.size(); ++c) {
+  for (int c : launch) {
     const int64_t m = items.count[c], o = items.first[c];
-    if (m == 0) continue;
-    hipStream_t cs = st;
-    int g = (int)std::min<int64_t>(grid, (m + block - 1) / block);
-    if (slots) {
-      const ClassSlot& sl = (*slots)[c];
-      if (sides && sl.side >= 0) cs = ctx->side[sl.side];
-      A.ybuf = ybase + sl.yoff;
-      A.ystride = sl.ystride;
-      g = sl.grid;
-    }
+    const ClassSlot& sl = slots[(size_t)c];
+    hipStream_t cs = sl.side >= 0 ? ctx->side[sl.side] : st;
+    A.ybuf = ybase + sl.yoff;
+    A.ystride = sl.ystride;
+    const int g = sl.grid;
     if (ev) HIPCHK(hipEventRecord(ev[2 * c], cs));
     A.bra_pair = items.bra + o;
     A.ket_pair = items.ket + o;
@@ -576,11 +572,11 @@ void fock_launch_all(l2g_context_s* ctx, L2gEriArgs A, const ItemsView& items, b
     A.q_prange = items.pr + o;
     A.n = (int)m;
     A.win = l2g_lane_window(m, ctx->ncu);
-    if (fock_is_generic((int)c)) {
-      launch_generic(kGenericFock, A, fock_gclass((int)c), ctx->gprog.as<int4>(), ctx->gidx.as<int>(),
+    if (fock_is_generic(c)) {
+      launch_generic(kGenericFock, A, fock_gclass(c), ctx->gprog.as<int4>(), ctx->gidx.as<int>(),
                      (int)std::min<int64_t>((int64_t)ctx->ncu * 8, m), cs);
     } else {
-      fock_info((int)c).launch(A, g, block, cs);
+      fock_info(c).launch(A, g, block, cs);
       LAUNCHCHK(std::string("Fock kernel of class ") + std::to_string(c) + " (grid " + std::to_string(g) +
                 ", block " + std::to_string(block) + ", items " + std::to_string(m) + ")");
     }
@@ -821,7 +817,6 @@ int l2g_fock_build(l2g_fock f, const double* D, double precision, double* J, dou
       for (auto& e : f->ev) HIPCHK(hipEventCreate(&e));
     }
     const int block = 128;
-    const int grid = (int)ctx->ncu * 8;
     // The quartet list is produced and digested in windows of consecutive
     // count-pass blocks holding at most window_items quartets each (one
     // block may exceed it alone), so that a large molecule's list (1e10
@@ -862,9 +857,11 @@ int l2g_fock_build(l2g_fock f, const double* D, double precision, double* J, dou
       }
       int64_t ymax = 0;
       std::vector<int64_t> lanes(ncls, 0), yd(ncls, 0);
+      std::vector<double> cost(ncls, 0.0);
       for (int c = 0; c < ncls; ++c) {
         const int64_t m = big.count[c];
         if (m == 0) continue;
+        cost[c] = fock_cost(c, m, (int64_t)es.cls_nprim[c]);
         // the generic kernel runs a block per item, no lane scratch, a few
         // blocks per CU: up to 4 items per CU count as small (side streams)
         lanes[c] = fock_is_generic(c) ? m * 64 : fock_lanes(ctx, c, m);
@@ -872,8 +869,9 @@ int l2g_fock_build(l2g_fock f, const double* D, double precision, double* J, dou
         ymax = std::max<int64_t>(ymax, yd[c]);
       }
       std::vector<ClassSlot> slots;
+      std::vector<int> launch;
       const int64_t ytotal = plan_slots(slots, lanes, yd, ctx->ncu, block, l2g_context_s::kSide,
-                                        ymax * (int64_t)ctx->ncu * 8 * block + (int64_t(1) << 29));
+                                        ymax * (int64_t)ctx->ncu * 8 * block + (int64_t(1) << 29), launch, true, &cost);
       f->ybuf.alloc(std::max<int64_t>(ytotal, 1) * sizeof(double));
       const int64_t ystride = 0;  // per class, from its slot
       const PairDev& p = f->pairs;
@@ -883,7 +881,7 @@ int l2g_fock_build(l2g_fock f, const double* D, double precision, double* J, dou
                                f->ybuf.as<double>(), ystride, hoff);
       hipEvent_t e0 = f->ev[2 * ncls], e1 = f->ev[2 * ncls + 1];
       HIPCHK(hipEventRecord(e0, st));
-      fock_launch_all(ctx, A, big, false, grid, block, st, f->ev.data(), &slots);
+      fock_launch_all(ctx, A, big, false, block, st, f->ev.data(), slots, launch);
       HIPCHK(hipEventRecord(e1, st));
       // the window's items and scratch are reused by the next window
       hipError_t e = hipStreamSynchronize(st);
@@ -1350,10 +1348,11 @@ void run_round(l2g_server_s* S, const std::vector<ServerRequest*>& act) {
     lanes[c] = fock_is_generic((int)c) ? rv.count[c] * 64 : fock_lanes(ctx, (int)c, rv.count[c]);
     yd[c] = fock_ybuf((int)c);
   }
+  std::vector<int> launch;
   std::vector<ClassSlot> slots;  // within the server's scratch (sized for the full grid)
   (void)plan_slots(slots, lanes, yd, ctx->ncu, S->block, l2g_context_s::kSide,
-                   (int64_t)(S->ybuf.bytes / sizeof(double)));
-  fock_launch_all(ctx, A, rv, true, S->grid, S->block, st, nullptr, &slots);
+                   (int64_t)(S->ybuf.bytes / sizeof(double)), launch, true);
+  fock_launch_all(ctx, A, rv, true, S->block, st, nullptr, slots, launch);
   HIPCHK(hipEventRecord(S->rev[b], st));
   // requests whose last quartets are in this round: finish on the device and
   // copy J, K, G to their pinned host buffers

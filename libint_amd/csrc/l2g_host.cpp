@@ -118,6 +118,7 @@ struct l2g_eri_plan_s {
   int64_t ymax = 0;  // largest scratch doubles per lane over the classes
   int block = 128;
   bool wave_split = true;  // classes of few deep quartets run a wave per quartet
+  std::vector<int> launch;  // classes in launch order (plan_slots)
   int oper = 0;             // 0 Coulomb, 1 erf-attenuated, 2 erfc-attenuated
   double omega = 0;
   // hipGraph mode: the class launches are captured once per output buffer
@@ -781,7 +782,7 @@ void plan_layout(l2g_eri_plan_s* p, l2g_context_s* ctx) {
   // 0.0025), plus 100 ns per quartet
   for (const auto& c : p->classes) {
     if (c.rys >= 0) {  // lane operations per primitive quartet, at 2 waves per SIMD on a part of the chip
-      cost.push_back((double)c.nprimq * l2g_gen_rys[c.rys].nodes * 1e-4 + 3.0 * (double)c.count);
+      cost.push_back((double)c.nprimq * l2g_gen_rys[c.rys].nodes * 4e-4 + 3.0 * (double)c.count);
       continue;
     }
     const double vals = c.generic ? (double)l2g_gen_generic[c.cls].nvals
@@ -792,7 +793,7 @@ void plan_layout(l2g_eri_plan_s* p, l2g_context_s* ctx) {
   std::vector<ClassSlot> slots;
   // side regions up to 4 GiB of scratch beyond the shared one
   const int64_t total = plan_slots(slots, lanes, yd, ctx->ncu, p->block, l2g_context_s::kSide,
-                                   p->ymax * (int64_t)ctx->ncu * 8 * p->block + (int64_t(1) << 29), &cost);
+                                   p->ymax * (int64_t)ctx->ncu * 8 * p->block + (int64_t(1) << 29), p->launch, false, &cost);
   for (size_t i = 0; i < p->classes.size(); ++i) p->classes[i].slot = slots[i];
   p->ybuf.alloc(std::max<int64_t>(total, 1) * sizeof(double));
 }
@@ -900,7 +901,8 @@ int l2g_eri_plan_execute(l2g_eri_plan p, double* d_out) {
     else passes = p->omega > 0 ? std::vector<std::pair<double, int>>{{0.0, 0}, {p->omega, 1}}
                                : std::vector<std::pair<double, int>>{{0.0, 0}};
     auto launch_classes = [&] {
-    for (auto& c : p->classes) {
+    for (int ic : p->launch) {
+    ClassWork& c = p->classes[(size_t)ic];
     for (size_t ps = 0; ps < passes.size(); ++ps) {
       const bool erfc = c.rys >= 0 && p->oper == 2 && p->omega > 0;
       if (erfc && ps) continue;

@@ -275,7 +275,7 @@ struct RysBlock {
       const double* v = V + q * region + r * sv[i] + c * sv[j];
       const double* d = V + q * region + nv + first(pb);
       double s = 0.0;
-#pragma unroll(nx * ny <= 25 ? nx : 1)
+#pragma unroll nx * ny <= 25 ? nx : 1
       for (int x = 0; x < nx; ++x)
 #pragma unroll
         for (int y = 0; y < ny; ++y) s = fma(d[x * ny + y], v[x * sv[pi] + y * sv[pj]], s);
