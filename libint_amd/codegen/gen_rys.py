@@ -16,8 +16,12 @@ of ceil(ne / 2) (or ne) lanes instead of one lane that has to walk its targets
 in groups and recompute shared recursion for each.  A block of 1, 2 or 4 waves
 holds as many quartets as fit.  Per batch of NB primitive quartets:
 
-  1. root stage: a lane per (primitive, quartet, node) evaluates prefactors,
-     screening, node and weight from the table (codegen/rys_table.py);
+  0. primitive stage: a lane per (primitive, quartet) evaluates prefactors and
+     screening and leaves a record of 15 doubles in LDS (evaluated by every
+     lane of the root stage instead, the light classes spent 40 % of their
+     instructions on it: (pp|dp) 0.067 -> 0.053 ns a primitive quartet);
+  1. root stage: a lane per (primitive, quartet, node) evaluates node and
+     weight from the table (codegen/rys_table.py);
   2. 2D stage: a lane per (quartet, node, axis) runs the two-index recurrence
      and leaves its (na+1)(nc+1) values in LDS;
   3. product stage: a lane reads the rows of its components per axis and does
@@ -34,9 +38,9 @@ Per primitive quartet (dd|dd) takes about 500 x 16 lane operations in the
 product stage where the Obara-Saika kernels evaluate 4123 recursion nodes of
 two to five operations with half of the live values in accumulation registers.
 Measured per class on an MI355X, K = 6 shells (77 primitive quartets a quartet
-on average): 34,000 (dd|dd) quartets 55.6 -> 2.0 ms, 40,000 (dp|dp) 11.0 ->
-0.71 ms, 40,000 (pp|pp) 2.35 -> 0.37 ms, 2,200 (fd|fd) 3.9 -> 0.60 ms, 1,000
-(ff|ff) 17 -> 2.4 ms; what bounds the heavy ones is the FP64 VALU: of the 820
+on average), when the kernels came: 34,000 (dd|dd) quartets 55.6 -> 2.0 ms,
+40,000 (dp|dp) 11.0 -> 0.71 ms, 40,000 (pp|pp) 2.35 -> 0.37 ms, 2,200 (fd|fd)
+3.9 -> 0.60 ms, 1,000 (ff|ff) 17 -> 2.4 ms; what bounds the heavy ones is the FP64 VALU: of the 820
 instructions a wave issues per primitive quartet of (dd|dd) 60 % are the
 product stage's multiplies and adds.
 The contracted block then goes through LDS: a lane per bra component for the
@@ -779,10 +783,8 @@ def emit(p, mode):
 
 
 def use(la, lb, lc, ld):
-    """Whether a class runs on its Rys kernel: every class but (ss|..), whose
-    one bra component leaves a tile of one lane a quartet (measured 0.2 to 0.8
-    times the speed of the per-lane kernels on 2000 to 40000 quartets, against
-    0.8 to 28 times for the others)."""
+    """Whether a class runs on its Rys kernel: every class does (0.8 to 28 times
+    the speed of the per-lane kernels on 2000 to 40000 quartets)."""
     return True
 
 

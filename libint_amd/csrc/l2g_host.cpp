@@ -287,7 +287,6 @@ int l2g_init(int device, l2g_context* out) {
     };
     fill(ctx->fock_of, l2g_gen_fock, l2g_gen_nfock);
     fill(ctx->class32_of, l2g_gen_classes32, l2g_gen_nclasses32);
-    fill(ctx->classerf_of, l2g_gen_classes_erf, l2g_gen_nclasses_erf);
     fill(ctx->fock32_of, l2g_gen_fock32, l2g_gen_nfock32);
     fill(ctx->rys_of, l2g_gen_rys, l2g_gen_nrys);
     for (auto& a : ctx->schwarz_of)
@@ -621,18 +620,15 @@ static int plan_create_impl(l2g_basis B, int64_t nq, const int32_t* quartets, do
 
 namespace {
 
-// Launch layout of a plan.  A class with a Rys kernel runs on it, a tile of
+// Launch layout of a plan.  An FP64 class runs on its Rys kernel, a tile of
 // lanes per quartet; with wave_split (the default) a class whose deepest
 // quartets would outlast the rest has its primitive loops cut into pieces
-// (plan_pieces).  The other classes run on their per-lane kernels: a
-// persistent grid with enough blocks to fill every CU several times over, and
-// the lane-private scratch for it; of these, a class of few quartets (fewer
-// than a quarter of the chip's lanes at one wave per SIMD) with deep
-// primitive loops runs, with wave_split, a wave per quartet whose lanes split
-// the loop (summing each contraction as 64 serial partial sums and a fixed
-// butterfly, another order than libint's serial loop, no less accurate).
-// Without wave_split, a class of few deep quartets (averaging at least 64
-// primitive quartets) and total angular momentum 7 or more runs on the
+// (plan_pieces).  FP32 classes run on their per-lane kernels: a persistent
+// grid with enough blocks to fill every CU several times over, and the
+// lane-private scratch for it; deep quartets share their wave
+// (l2g_lane_tier).  Without wave_split, a class of few deep quartets (fewer
+// than a quarter of the chip's lanes at one wave per SIMD, averaging at least
+// 64 primitive quartets) and total angular momentum 7 or more runs on the
 // generic kernel, a block per quartet whose threads split the targets.
 #ifndef L2G_GENERIC_MIN_DEPTH
 #define L2G_GENERIC_MIN_DEPTH 64
@@ -885,11 +881,8 @@ int l2g_eri_plan_execute(l2g_eri_plan p, double* d_out) {
     bool sides = false;
     for (auto& c : p->classes) sides |= c.slot.side >= 0;
     sides &= !capture;
-    // attenuated passes run on the class's erf-attenuated register kernel
-    // (a separate instantiation, so the Coulomb kernels' primitive loop
-    // carries no operator branch) where one is built, else on the generic
-    // kernel, whose core-integral step takes omega; the Coulomb pass of erfc
-    // runs on the Coulomb kernels.
+    // attenuated passes run on the class's Rys kernel, or on the generic
+    // kernel, whose core-integral step takes omega too
     // Passes (attenuation, subtract): Coulomb; erf = one attenuated pass
     // (omega = 0 gives exact zeros as Coulomb minus Coulomb); erfc =
     // Coulomb minus the erf pass, both per class on the class's stream, or
@@ -946,17 +939,7 @@ int l2g_eri_plan_execute(l2g_eri_plan p, double* d_out) {
         if (!capture && last) HIPCHK(hipEventRecord(c.ev1, cs));
         continue;
       }
-      int erf_idx = -1;  // the class's erf-attenuated register kernel, for an attenuated pass
-      if (A.omega > 0 && !c.generic && !c.fp32) {
-        const L2gClassInfo& ci = l2g_gen_classes[c.cls];
-        erf_idx = ctx->classerf_of[ci.la][ci.lb][ci.lc][ci.ld];
-      }
-      if (erf_idx >= 0) {
-        const L2gClassInfo& ci = l2g_gen_classes_erf[erf_idx];
-        A.win = l2g_lane_window(c.count, ctx->ncu);
-        ci.launch(A, c.slot.grid, p->block, cs);
-        LAUNCHCHK(std::string("erf ERI kernel of class ") + std::to_string(c.cls));
-      } else if (c.generic || A.omega > 0) {  // the attenuated pass of erf / erfc
+      if (c.generic || A.omega > 0) {  // the attenuated pass of erf / erfc
         // one block per quartet, persistent over the class
         if (c.gidx < 0) throw L2gError(L2G_E_LMAX, "no generic-kernel program for this class");
         const L2gGenericClass& gc = l2g_gen_generic[c.gidx];

@@ -28,9 +28,6 @@ extern const L2gClassInfo l2g_gen_classes32[];
 extern const int l2g_gen_nclasses32;
 extern const L2gClassInfo l2g_gen_fock32[];
 extern const int l2g_gen_nfock32;
-// erf-attenuated ERI variants (same plans and scratch layout as l2g_gen_classes)
-extern const L2gClassInfo l2g_gen_classes_erf[];
-extern const int l2g_gen_nclasses_erf;
 // Rys kernels of the ERI batches (codegen/gen_rys.py) and their node table
 extern const L2gClassInfo l2g_gen_rys[];
 extern const int l2g_gen_nrys;
@@ -290,7 +287,6 @@ struct l2g_context_s {
   int class_of[8][8][8][8];  // index into l2g_gen_classes
   int fock_of[8][8][8][8];   // index into l2g_gen_fock (its own order)
   int class32_of[8][8][8][8];  // index into l2g_gen_classes32
-  int classerf_of[8][8][8][8]; // index into l2g_gen_classes_erf
   int rys_of[8][8][8][8];      // index into l2g_gen_rys
   int fock32_of[8][8][8][8];   // index into l2g_gen_fock32
   int schwarz_of[8][8];
@@ -355,14 +351,19 @@ struct l2g_basis_s {
   // caller's order would.  s and p shells keep the caller's order.
   bool second_is_centre(int i, int j) {
     if (i == j || l[i] != l[j] || l[i] < 2) return false;
-    // a single primitive pair (the Schwarz factors of primitives have 1e5
-    // of them) costs less to look at than to remember
-    const bool memo = nprim[i] * nprim[j] > 1;
-    const uint64_t key = (uint64_t)(uint32_t)i << 32 | (uint32_t)j;
-    if (memo)
-      if (auto it = orient.find(key); it != orient.end()) return it->second;
     double AB2 = 0;
     for (int k = 0; k < 3; ++k) AB2 += (origin[3 * i + k] - origin[3 * j + k]) * (origin[3 * i + k] - origin[3 * j + k]);
+    if (nprim[i] * nprim[j] == 1) {  // the Schwarz factors of primitives have 1e5 such pairs: the same by exponents alone
+      const double a1 = alpha[off[i]], a2 = alpha[off[j]], x = a2 / (a1 + a2), y = a1 / (a1 + a2);
+      if (!(AB2 > 0)) return false;
+      if (l[i] >= 3) return a2 > a1;
+      double ta = 1.0, tb = 1.0;
+      for (int k = 0; k < l[i]; ++k) ta *= x * (1.0 + x), tb *= y * (1.0 + y);
+      return tb < 1e-3 * ta;
+    }
+    const uint64_t key = (uint64_t)(uint32_t)i << 32 | (uint32_t)j;
+    auto it = orient.find(key);
+    if (it != orient.end()) return it->second;
     double s = 0, sa = 0, sb = 0;
     if (AB2 > 0) {
       const double ab = std::sqrt(AB2);
@@ -378,10 +379,8 @@ struct l2g_basis_s {
         }
     }
     const bool r = l[i] >= 3 ? s > 0 : sb < 1e-3 * sa, back = l[i] >= 3 ? s < 0 : sa < 1e-3 * sb;
-    if (memo) {
-      orient.emplace(key, r);
-      orient.emplace((uint64_t)(uint32_t)j << 32 | (uint32_t)i, back);
-    }
+    orient.emplace(key, r);
+    orient.emplace((uint64_t)(uint32_t)j << 32 | (uint32_t)i, back);
     return r;
   }
   // canonical bra orientation of (i, j): l_i >= l_j, ties by second_is_centre

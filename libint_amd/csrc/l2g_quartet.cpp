@@ -34,12 +34,9 @@ namespace l2g_impl {
 
 int64_t quartet_ylane(int max_l) {
   int64_t y = 0;
-  for (const L2gClassInfo* tab : {l2g_gen_classes, l2g_gen_classes_erf}) {
-    const int n = tab == l2g_gen_classes ? l2g_gen_nclasses : l2g_gen_nclasses_erf;
-    for (int i = 0; i < n; ++i) {
-      const L2gClassInfo& c = tab[i];
-      if (std::max(std::max(c.la, c.lb), std::max(c.lc, c.ld)) <= max_l) y = std::max<int64_t>(y, c.ybuf_doubles);
-    }
+  for (int i = 0; i < l2g_gen_nclasses; ++i) {
+    const L2gClassInfo& c = l2g_gen_classes[i];
+    if (std::max(std::max(c.la, c.lb), std::max(c.lc, c.ld)) <= max_l) y = std::max<int64_t>(y, c.ybuf_doubles);
   }
   return y;
 }
@@ -233,16 +230,11 @@ void quartet_compute_impl(l2g_context_s* ctx, const QuartetBuffers& qb, const in
   for (const auto& ps : passes) {
     A.omega = ps.first;
     A.store_sub = ps.second;
-    int erf_idx = -1;
-    if (A.omega > 0 && cls >= 0) erf_idx = ctx->classerf_of[l[b1]][l[b2]][l[k1]][l[k2]];
     if (rys >= 0) {
       const int tier = rys_tier_of((long long)pb.np[0] * pb.np[1]);
       if (tier < 2) A.rys_deep[tier] = 1;
       l2g_gen_rys[rys].launch(A, 1, kQuartetBlock, st);
       LAUNCHCHK("Rys ERI kernel (quartet engine)");
-    } else if (erf_idx >= 0) {
-      l2g_gen_classes_erf[erf_idx].launch(A, 1, kQuartetBlock, st);
-      LAUNCHCHK("erf ERI kernel (quartet engine)");
     } else if (cls < 0 || A.omega > 0) {
       if (gcls < 0) throw L2gError(L2G_E_LMAX, "no generic-kernel program for this class");
       launch_generic(kGenericEri, A, l2g_gen_generic[gcls], ctx->gprog.as<int4>(), ctx->gidx.as<int>(), 1, st);
