@@ -223,7 +223,7 @@ def eri_f_leg(la, molecule, flop_model, ctx, nquartets, reps=3, seed=21):
     cube, s4p3d2f1, K~U{1..8}): a seeded sample of quartets with
     K_ab K_cd >= 1e-12 over every class up to (ff|ff), FP64 and mixed
     (FP32 where K_ab K_cd < 1e-6 and S_ab S_cd < 16e-6, l <= the FP32 kernels'
-    l), and FP64 with the wave split off (a lane per quartet, or the generic
+    l), and FP64 with the wave split off (no pieces; the generic
     kernel for few deep high-l classes); quartets/s and model TFLOP/s of the
     whole batch, and the classes that take the most time."""
     mol = molecule.make_molecule(3)
@@ -614,7 +614,7 @@ def main():
             "unit": "TFLOP/s",
             "frac": achieved / FP64_PEAK_TFLOPS,
             "traffic": measured_traffic(len(q)),
-            "kernel": "l2g_eri_2222",
+            "kernel": "l2g_rys_eri_2222",
             "kernel_ms": kms,
             "model_flops_per_launch": flops,
             "model_flops_per_launch_derived": flops_derived,

@@ -205,3 +205,49 @@ def test_fock_quartet_list_sizes(ctx, n):
     one = [fb.build(s * np.eye(N), 1e-12) for s in (1.0, 1e-3, 1.0)]
     for x, y in zip(one[0], one[2]):
         assert np.abs(x - y).max() <= 1e-9
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("c", [(1, 0, 2, 1), (2, 1, 2, 1)])
+def test_fp32_lane_tiers(ctx, c):
+    """The per-lane FP32 kernels share a quartet between 1, 4, 16 or 64 lanes
+    from 16, 64 and 512 primitive quartets on.  n additions in FP32 round by
+    at most n eps of the pre-HRR size S_ab S_cd; a lost or doubled primitive
+    of 513 would be off by 2e-3 of the value."""
+    rng = np.random.default_rng(5 + sum(c))
+    ks = [(5, 3, 1, 1), (16, 1, 1, 1), (17, 1, 1, 1), (9, 7, 1, 1), (8, 1, 8, 1), (13, 1, 5, 1), (73, 1, 7, 1),
+          (16, 2, 16, 1), (27, 1, 19, 1)]
+    sh = [x for k in ks for x in shells(rng, c, k, True)]
+    b = la.Basis(ctx, la.BasisArrays.from_shells(sh))
+    q = np.arange(len(sh), dtype=np.int32).reshape(-1, 4)
+    say(f"case: FP32 {c} primitive counts {[int(np.prod(k)) for k in ks]}")
+    ctx.set_fp32_policy(la.FP32_ALWAYS)
+    try:
+        m = la.EriPlan(b, q, fp32_threshold=1e6)
+        assert all(s["fp32"] for s in m.stats())
+    finally:
+        ctx.set_fp32_policy(la.FP32_MEASURED)
+    m.execute()
+    g, _ = m.download()
+    o, off, _ = oracle.eri_quartets(b.arrays, q)
+    _, S = la.precision_bounds(b, np.concatenate([q[:, :2], q[:, 2:]]))
+    ends = np.append(off[1:], o.size)
+    for k in range(len(q)):
+        bar = (np.prod(ks[k]) + 16) * 1.2e-7 * S[k] * S[k + len(q)]
+        assert np.abs(g[off[k]:ends[k]] - o[off[k]:ends[k]]).max() <= bar, ks[k]
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("n", [1, 7, 8, 9, 16, 17])
+def test_one_body_items_around_a_wave(ctx, n):
+    """8 primitive pairs of two shells and n charges: 8 n items for 64 lanes."""
+    from oracle import onebody
+    rng = np.random.default_rng(n)
+    sh = shells(rng, (2,), (2,), False) + shells(rng, (1,), (4,), False)
+    charges = [(float(z), rng.normal(0, 1.2, 3)) for z in rng.uniform(1, 8, n)]
+    say(f"case: one-body integrals, {n} charges")
+    got = la.one_body(la.Basis(ctx, la.BasisArrays.from_shells(sh)), charges)
+    ref = onebody.one_body([(s.l, s.alpha, s.coeff, s.O) for s in sh], charges)
+    for g, o in zip(got, ref):
+        d = np.abs(g - o)
+        assert not ((d > 1e-12) & (d > 1e-10 * np.abs(o))).any()
