@@ -306,17 +306,21 @@ void sort_by_depth(FockItems& it) {
 // more HRR, transform and digest per range.
 // Longest primitive range of one work item of class cls, for m items with
 // `total` primitive quartets in all, on a chip of `lanes` lanes (one wave
-// per SIMD): half of the class's share per item in flight, but not below the
-// length from which one more HRR and digest is small against the loop.  The
+// per SIMD): a multiple of the class's share per item in flight, but not below
+// the length from which one more HRR and digest is small against the loop.  The
 // generic kernel runs one item per block; only its classes with few items
 // are split, to about 2e6 recursion values per piece.
 int split_chunk(int cls, int64_t m, int64_t total, int lanes) {
   if (m == 0) return INT_MAX;
   if (fock_is_generic(cls))
     return m < 4096 ? std::max(16, 2000000 / std::max(1, fock_gclass(cls).nvals)) : INT_MAX;
-  if (const int per = fock_info(cls).lanes) {  // a tile of lanes per item, at 2 waves per SIMD
+  if (const int per = fock_info(cls).lanes) {
+    // a tile of lanes per item, at 2 waves per SIMD: twice the class's
+    // share per item in flight, as four streams of classes share the chip
+    // (5 atoms with f, K to 8: 24.2 ms at half the share, 21.8 at it, 20.3 at
+    // twice, 22.1 at four times; 5 atoms s/p/d 3.05, 2.62, 2.43, 2.67)
     const int64_t slots = std::max<int64_t>(1, 2ll * lanes / per);
-    return (int)std::min<int64_t>(INT_MAX, std::max<int64_t>(32, (total + 2 * slots - 1) / (2 * slots)));
+    return (int)std::min<int64_t>(INT_MAX, std::max<int64_t>(40, 2 * total / slots));
   }
   // the per-lane kernels share an item of 512 or more between the lanes of a
   // wave (l2g_lane_tier)
