@@ -271,35 +271,6 @@ struct FockWork {
   int64_t nq = 0, nq32 = 0, nprim = 0;
 };
 
-// Reorders the items of one class by decreasing primitive-loop length, so
-// that neighbouring lanes run equal-length loops.  Stable counting sort.
-void sort_by_depth(FockItems& it) {
-  const size_t m = it.size();
-  if (m < 2) return;
-  int wmax = 0;
-  std::vector<int> w(m);
-  for (size_t i = 0; i < m; ++i) {
-    w[i] = it.pr[i].y - it.pr[i].x;
-    wmax = std::max(wmax, w[i]);
-  }
-  std::vector<size_t> cnt((size_t)wmax + 2, 0);
-  for (size_t i = 0; i < m; ++i) ++cnt[(size_t)(wmax - w[i]) + 1];
-  for (size_t k = 1; k < cnt.size(); ++k) cnt[k] += cnt[k - 1];
-  std::vector<size_t> ord(m);
-  for (size_t i = 0; i < m; ++i) ord[cnt[(size_t)(wmax - w[i])]++] = i;
-  FockItems s;
-  s.bra.resize(m), s.ket.resize(m), s.meta.resize(m), s.lnp.resize(m), s.scale.resize(m), s.bf.resize(m),
-      s.pr.resize(m);
-  if (!it.req.empty()) s.req.resize(m);
-  for (size_t k = 0; k < m; ++k) {
-    const size_t i = ord[k];
-    s.bra[k] = it.bra[i], s.ket[k] = it.ket[i], s.meta[k] = it.meta[i];
-    s.lnp[k] = it.lnp[i], s.scale[k] = it.scale[i], s.bf[k] = it.bf[i], s.pr[k] = it.pr[i];
-    if (!it.req.empty()) s.req[k] = it.req[i];
-  }
-  it = std::move(s);
-}
-
 // Deep items are split by primitive-quartet range: an item whose loop is
 // longer than the class's chunk becomes several items.  The digest is linear
 // in the integrals, so each range is digested on its own; the cost is one
@@ -328,33 +299,46 @@ int split_chunk(int cls, int64_t m, int64_t total, int lanes) {
   return (int)std::min<int64_t>(INT_MAX, std::max<int64_t>(1024, share));
 }
 
-void split_deep(FockItems& it, int cls, int lanes) {
-  const size_t m = it.size();
-  int64_t total = 0;
-  for (size_t i = 0; i < m; ++i) total += it.pr[i].y - it.pr[i].x;
-  const int chunk = split_chunk(cls, (int64_t)m, total, lanes);
-  if (chunk == INT_MAX) return;
-  size_t extra = 0;
-  for (size_t i = 0; i < m; ++i) {
-    const int len = it.pr[i].y - it.pr[i].x;
-    if (len > chunk) extra += (size_t)((len + chunk - 1) / chunk) - 1;
+// One class's items of all parts, deep ones cut into ranges, by decreasing
+// primitive-loop length (neighbouring tiles then run equal-length loops; a
+// stable counting sort).  Written straight to their places: the lists of a
+// request of 12 atoms with f hold 600 MB, and every pass over them counts
+// against its admission.
+template <class Part>
+void gather_class(std::vector<Part>& parts, int cls, int lanes, FockItems& out) {
+  int64_t m = 0, total = 0;
+  for (auto& w : parts) {
+    m += (int64_t)w.cls[cls].size();
+    for (const int2& r : w.cls[cls].pr) total += r.y - r.x;
   }
-  if (extra == 0) return;
-  FockItems s;
-  s.bra.reserve(m + extra), s.ket.reserve(m + extra), s.meta.reserve(m + extra), s.lnp.reserve(m + extra),
-      s.scale.reserve(m + extra), s.bf.reserve(m + extra), s.pr.reserve(m + extra);
-  if (!it.req.empty()) s.req.reserve(m + extra);
-  for (size_t i = 0; i < m; ++i) {
-    const int b = it.pr[i].x, e = it.pr[i].y, len = e - b;
-    const int nch = len > chunk ? (len + chunk - 1) / chunk : 1;
-    for (int k = 0; k < nch; ++k) {
-      s.bra.push_back(it.bra[i]), s.ket.push_back(it.ket[i]), s.meta.push_back(it.meta[i]);
-      s.lnp.push_back(it.lnp[i]), s.scale.push_back(it.scale[i]), s.bf.push_back(it.bf[i]);
-      if (!it.req.empty()) s.req.push_back(it.req[i]);
-      s.pr.push_back(int2{b + (int)((int64_t)len * k / nch), b + (int)((int64_t)len * (k + 1) / nch)});
-    }
+  if (m == 0) return;
+  const int chunk = split_chunk(cls, m, total, lanes);
+  // the ranges [k len / nch, (k + 1) len / nch) of an item
+  auto each = [&](const int2& r, auto&& f) {
+    const int len = r.y - r.x, nch = len > chunk ? (len - 1) / chunk + 1 : 1;
+    for (int k = 0; k < nch; ++k)
+      f(int2{r.x + (int)((int64_t)len * k / nch), r.x + (int)((int64_t)len * (k + 1) / nch)});
+  };
+  int wmax = 0;
+  for (auto& w : parts)
+    for (const int2& r : w.cls[cls].pr) wmax = std::max(wmax, std::min(r.y - r.x, chunk));
+  std::vector<size_t> at((size_t)wmax + 2, 0);
+  for (auto& w : parts)
+    for (const int2& r : w.cls[cls].pr) each(r, [&](int2 x) { ++at[(size_t)(wmax - (x.y - x.x)) + 1]; });
+  for (size_t k = 1; k < at.size(); ++k) at[k] += at[k - 1];
+  const size_t n = at.back();
+  out.bra.resize(n), out.ket.resize(n), out.meta.resize(n), out.lnp.resize(n), out.scale.resize(n), out.bf.resize(n),
+      out.pr.resize(n);
+  for (auto& w : parts) {
+    FockItems& it = w.cls[cls];
+    for (size_t i = 0; i < it.size(); ++i)
+      each(it.pr[i], [&](int2 x) {
+        const size_t k = at[(size_t)(wmax - (x.y - x.x))]++;
+        out.bra[k] = it.bra[i], out.ket[k] = it.ket[i], out.meta[k] = it.meta[i];
+        out.lnp[k] = it.lnp[i], out.scale[k] = it.scale[i], out.bf[k] = it.bf[i], out.pr[k] = x;
+      });
+    it = FockItems();
   }
-  it = std::move(s);
 }
 
 // Screened, permutationally-unique shell quartets of compute_2body_fock
@@ -449,15 +433,7 @@ void fock_enumerate(const FockSetup& f, const double* D, double precision, doubl
     out.nprim += w.nprim;
   }
   parallel_for(ncls, [&](int c) {
-    size_t tot = 0;
-    for (auto& w : part) tot += w.cls[c].size();
-    if (tot == 0) return;
-    FockItems& o = out.cls[c];
-    o.bra.reserve(tot), o.ket.reserve(tot), o.meta.reserve(tot), o.lnp.reserve(tot), o.scale.reserve(tot),
-        o.bf.reserve(tot);
-    for (auto& w : part) o.append(w.cls[c]);
-    split_deep(o, c, f.B->ctx->ncu * 256);
-    sort_by_depth(o);
+    gather_class(part, c, f.B->ctx->ncu * 256, out.cls[c]);
   });
 }
 
