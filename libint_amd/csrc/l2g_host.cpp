@@ -147,7 +147,13 @@ struct l2g_eri_plan_s {
 };
 
 namespace {
-void plan_layout(l2g_eri_plan_s* p, l2g_context_s* ctx);  // launch layout, defined below
+// a plan's work-item arrays on the host, in launch order
+struct WorkLists {
+  std::vector<int> bra, ket, meta;
+  std::vector<long long> qidx;
+};
+// launch layout, defined below; without `lists` the arrays are read back where needed
+void plan_layout(l2g_eri_plan_s* p, l2g_context_s* ctx, const WorkLists* lists);
 }  // namespace
 
 
@@ -543,8 +549,9 @@ static int plan_create_impl(l2g_basis B, int64_t nq, const int32_t* quartets, do
       }
     }
     // flatten: classes in table order, each sorted by contraction depth
-    std::vector<int> bra, ket, meta;
-    std::vector<long long> off, qidx;
+    WorkLists wl;
+    std::vector<int>&bra = wl.bra, &ket = wl.ket, &meta = wl.meta;
+    std::vector<long long> off, &qidx = wl.qidx;
     bra.reserve(nq);
     ket.reserve(nq);
     meta.reserve(nq);
@@ -608,7 +615,7 @@ static int plan_create_impl(l2g_basis B, int64_t nq, const int32_t* quartets, do
     upload(plan->ppAux, pb.aux, st);
     upload(plan->ppNs, pb.ns, st);
     plan->ymax = ymax;
-    plan_layout(plan.get(), ctx);
+    plan_layout(plan.get(), ctx, &wl);
     HIPCHK(hipStreamSynchronize(st));
     ++ctx->live;
     basis_retain(B);
@@ -663,13 +670,11 @@ int class_l(const ClassWork& c) {
 // 8, takes 3.0 ms at 48, 2.4 at 32, 2.05 at 24, 2.4 at 20, 3.1 at 16: shorter
 // pieces leave more partial sums than loops saved.
 constexpr int64_t kRysPiece = 24, kRysSerial = 96;
-void plan_pieces(l2g_eri_plan_s* p, l2g_context_s* ctx) {
+void plan_pieces(l2g_eri_plan_s* p, l2g_context_s* ctx, const WorkLists* lists) {
   std::vector<int> pb, pk, pm, pf;
   std::vector<long long> pq;
   std::vector<int2> pr;
-  std::vector<int> hb((size_t)p->nq), hk((size_t)p->nq), hm((size_t)p->nq);
-  std::vector<long long> hq((size_t)p->nq);
-  bool have = false;
+  WorkLists back;
   int64_t gtotal = 0;
   for (auto& c : p->classes) {
     c.npieces = 0;
@@ -689,12 +694,16 @@ void plan_pieces(l2g_eri_plan_s* p, l2g_context_s* ctx) {
       chunk += chunk & 1;  // even: the two-primitive pass stays full
       if (wmax <= chunk) continue;
     }
-    if (!have) {  // the plan's work-item arrays, read back once
-      HIPCHK(hipMemcpy(hb.data(), p->bra.p, hb.size() * sizeof(int), hipMemcpyDeviceToHost));
-      HIPCHK(hipMemcpy(hk.data(), p->ket.p, hk.size() * sizeof(int), hipMemcpyDeviceToHost));
-      HIPCHK(hipMemcpy(hm.data(), p->meta.p, hm.size() * sizeof(int), hipMemcpyDeviceToHost));
-      HIPCHK(hipMemcpy(hq.data(), p->qidx.p, hq.size() * sizeof(long long), hipMemcpyDeviceToHost));
-      have = true;
+    if (!lists) {  // read back once
+      const size_t n = (size_t)p->nq;
+      back.bra.resize(n), back.ket.resize(n), back.meta.resize(n), back.qidx.resize(n);
+      // the context's stream does not wait for hipMemcpy, nor hipMemcpy for it
+      HIPCHK(hipStreamSynchronize(ctx->stream));
+      HIPCHK(hipMemcpy(back.bra.data(), p->bra.p, n * sizeof(int), hipMemcpyDeviceToHost));
+      HIPCHK(hipMemcpy(back.ket.data(), p->ket.p, n * sizeof(int), hipMemcpyDeviceToHost));
+      HIPCHK(hipMemcpy(back.meta.data(), p->meta.p, n * sizeof(int), hipMemcpyDeviceToHost));
+      HIPCHK(hipMemcpy(back.qidx.data(), p->qidx.p, n * sizeof(long long), hipMemcpyDeviceToHost));
+      lists = &back;
     }
     if (c.rys >= 0) {
       const L2gClassInfo& ci = l2g_gen_rys[c.rys];
@@ -715,10 +724,10 @@ void plan_pieces(l2g_eri_plan_s* p, l2g_context_s* ctx) {
       pf.push_back((int)((int64_t)pb.size() - c.piece_off));
       const int w = p->itemw[(size_t)i];
       for (int a = 0; a < w || a == 0; a += (int)chunk) {
-        pb.push_back(hb[(size_t)i]);
-        pk.push_back(hk[(size_t)i]);
-        pm.push_back(hm[(size_t)i]);
-        pq.push_back(hq[(size_t)i]);
+        pb.push_back(lists->bra[(size_t)i]);
+        pk.push_back(lists->ket[(size_t)i]);
+        pm.push_back(lists->meta[(size_t)i]);
+        pq.push_back(lists->qidx[(size_t)i]);
         pr.push_back(make_int2(a, (int)std::min<int64_t>(w, a + chunk)));
       }
     }
@@ -739,7 +748,7 @@ void plan_pieces(l2g_eri_plan_s* p, l2g_context_s* ctx) {
   HIPCHK(hipStreamSynchronize(st));
 }
 
-void plan_layout(l2g_eri_plan_s* p, l2g_context_s* ctx) {
+void plan_layout(l2g_eri_plan_s* p, l2g_context_s* ctx, const WorkLists* lists) {
   p->block = 128;
   std::vector<int64_t> lanes, yd;
   std::vector<double> cost;
@@ -767,7 +776,7 @@ void plan_layout(l2g_eri_plan_s* p, l2g_context_s* ctx) {
     lanes.push_back(c.generic ? c.count * 64 : l2g_window_lanes(c.count, ctx->ncu));
     yd.push_back(c.generic ? 0 : (c.fp32 ? l2g_gen_classes32 : l2g_gen_classes)[c.cls].ybuf_doubles);
   }
-  plan_pieces(p, ctx);
+  plan_pieces(p, ctx, lists);
   for (size_t i = 0; i < p->classes.size(); ++i)
     if (const ClassWork& c = p->classes[i]; c.npieces)
       lanes[i] = c.npieces * (c.rys >= 0 ? l2g_gen_rys[c.rys].lanes : 64);
@@ -1049,7 +1058,7 @@ int l2g_eri_plan_set_wave_split(l2g_eri_plan p, int on) {
     if (on < 0 || on > 2) throw std::invalid_argument("wave split mode must be 0, 1 or 2");
     p->wave_split = on != 0;
     p->drop_graph();
-    plan_layout(p, ctx);
+    plan_layout(p, ctx, nullptr);
   });
 }
 
