@@ -670,54 +670,77 @@ int class_l(const ClassWork& c) {
 // 8, takes 3.0 ms at 48, 2.4 at 32, 2.05 at 24, 2.4 at 20, 3.1 at 16: shorter
 // pieces leave more partial sums than loops saved.
 constexpr int64_t kRysPiece = 24, kRysSerial = 96;
-void plan_pieces(l2g_eri_plan_s* p, l2g_context_s* ctx, const WorkLists* lists) {
+void plan_pieces(l2g_eri_plan_s* p, l2g_context_s* ctx, const WorkLists* lists, bool cut_rys = true) {
+  for (DevBuf* d : {&p->gp_bra, &p->gp_ket, &p->gp_meta, &p->gp_qidx, &p->gp_range, &p->gp_first, &p->gpart})
+    *d = DevBuf();
+  // which classes, in pieces of what length
+  std::vector<int64_t> chunks(p->classes.size(), 0);
+  std::vector<size_t> cand;
+  std::vector<PieceCandidate> room;
+  bool any = false;
+  for (size_t k = 0; k < p->classes.size(); ++k) {
+    ClassWork& c = p->classes[k];
+    c.npieces = 0;
+    if (c.rys >= 0 ? !p->wave_split || !cut_rys : !c.generic || c.count > (int64_t)ctx->ncu * 16) continue;
+    int wmax = 0;
+    for (int64_t i = c.first; i < c.first + c.count; ++i) wmax = std::max(wmax, p->itemw[(size_t)i]);
+    if (c.rys < 0) {
+      int64_t chunk = std::max<int64_t>(32, (c.nprimq + 4 * ctx->ncu - 1) / (4 * ctx->ncu));
+      chunk += chunk & 1;  // even: the two-primitive pass stays full
+      if (wmax <= chunk) continue;
+      const L2gGenericClass& g = l2g_gen_generic[c.cls];
+      c.gstride = (int64_t)g.ne * g.accs + 1;
+      chunks[k] = chunk;
+      any = true;
+      continue;
+    }
+    const L2gClassInfo& ci = l2g_gen_rys[c.rys];
+    const int64_t slots = (int64_t)ctx->ncu * 512 / ci.lanes;  // quartets at 2 waves per SIMD
+    const int64_t chunk = std::max<int64_t>(kRysPiece, (c.nprimq + slots - 1) / slots);
+    // the longest serial loop: the deepest quartet's, shared by up to 16 slots
+    const int64_t serial = wmax / std::min<int64_t>(wmax >= L2G_RYS_DEEP0 ? 16 : wmax >= L2G_RYS_DEEP1 ? 4 : 1,
+                                                    std::max(1, 64 / ci.lanes));
+    if (serial <= std::max<int64_t>(2 * chunk, kRysSerial)) continue;
+    auto nc = [](int l1, int l2) {
+      int n = 0;
+      for (int l = l1; l <= l1 + l2; ++l) n += ncart(l);
+      return n;
+    };
+    c.gstride = (int64_t)nc(ci.la, ci.lb) * nc(ci.lc, ci.ld) + 1;
+    const int64_t doubles = (c.count + c.nprimq / chunk) * c.gstride;
+    if (doubles > (int64_t(1) << 27)) continue;  // 1 GiB of pieces
+    chunks[k] = chunk;
+    cand.push_back(k);
+    room.push_back({doubles, (double)(serial - chunk) * ci.nodes});
+  }
+  const std::vector<char> cut = choose_pieces(room, kPlanPieceDoubles);
+  for (size_t i = 0; i < cand.size(); ++i) {
+    if (!cut[i]) chunks[cand[i]] = 0;
+    any |= cut[i] != 0;
+  }
+  if (!any) return;
+  WorkLists back;
+  if (!lists) {  // read back once
+    const size_t n = (size_t)p->nq;
+    back.bra.resize(n), back.ket.resize(n), back.meta.resize(n), back.qidx.resize(n);
+    // the context's stream does not wait for hipMemcpy, nor hipMemcpy for it
+    HIPCHK(hipStreamSynchronize(ctx->stream));
+    HIPCHK(hipMemcpy(back.bra.data(), p->bra.p, n * sizeof(int), hipMemcpyDeviceToHost));
+    HIPCHK(hipMemcpy(back.ket.data(), p->ket.p, n * sizeof(int), hipMemcpyDeviceToHost));
+    HIPCHK(hipMemcpy(back.meta.data(), p->meta.p, n * sizeof(int), hipMemcpyDeviceToHost));
+    HIPCHK(hipMemcpy(back.qidx.data(), p->qidx.p, n * sizeof(long long), hipMemcpyDeviceToHost));
+    lists = &back;
+  }
   std::vector<int> pb, pk, pm, pf;
   std::vector<long long> pq;
   std::vector<int2> pr;
-  WorkLists back;
   int64_t gtotal = 0;
-  for (auto& c : p->classes) {
-    c.npieces = 0;
-    if (c.rys >= 0 ? !p->wave_split : !c.generic || c.count > (int64_t)ctx->ncu * 16) continue;
-    int wmax = 0;
-    for (int64_t i = c.first; i < c.first + c.count; ++i) wmax = std::max(wmax, p->itemw[(size_t)i]);
-    int64_t chunk;
-    if (c.rys >= 0) {
-      const int64_t slots = (int64_t)ctx->ncu * 512 / l2g_gen_rys[c.rys].lanes;  // quartets at 2 waves per SIMD
-      chunk = std::max<int64_t>(kRysPiece, (c.nprimq + slots - 1) / slots);
-      // the longest serial loop: the deepest quartet's, shared by up to 16 slots
-      const int64_t serial = wmax / std::min<int64_t>(wmax >= L2G_RYS_DEEP0 ? 16 : wmax >= L2G_RYS_DEEP1 ? 4 : 1,
-                                                      std::max(1, 64 / l2g_gen_rys[c.rys].lanes));
-      if (serial <= std::max<int64_t>(2 * chunk, kRysSerial)) continue;
-    } else {
-      chunk = std::max<int64_t>(32, (c.nprimq + 4 * ctx->ncu - 1) / (4 * ctx->ncu));
-      chunk += chunk & 1;  // even: the two-primitive pass stays full
-      if (wmax <= chunk) continue;
-    }
-    if (!lists) {  // read back once
-      const size_t n = (size_t)p->nq;
-      back.bra.resize(n), back.ket.resize(n), back.meta.resize(n), back.qidx.resize(n);
-      // the context's stream does not wait for hipMemcpy, nor hipMemcpy for it
-      HIPCHK(hipStreamSynchronize(ctx->stream));
-      HIPCHK(hipMemcpy(back.bra.data(), p->bra.p, n * sizeof(int), hipMemcpyDeviceToHost));
-      HIPCHK(hipMemcpy(back.ket.data(), p->ket.p, n * sizeof(int), hipMemcpyDeviceToHost));
-      HIPCHK(hipMemcpy(back.meta.data(), p->meta.p, n * sizeof(int), hipMemcpyDeviceToHost));
-      HIPCHK(hipMemcpy(back.qidx.data(), p->qidx.p, n * sizeof(long long), hipMemcpyDeviceToHost));
-      lists = &back;
-    }
-    if (c.rys >= 0) {
-      const L2gClassInfo& ci = l2g_gen_rys[c.rys];
-      auto nc = [](int l1, int l2) {
-        int n = 0;
-        for (int l = l1; l <= l1 + l2; ++l) n += ncart(l);
-        return n;
-      };
-      c.gstride = (int64_t)nc(ci.la, ci.lb) * nc(ci.lc, ci.ld) + 1;
-      if ((c.count + c.nprimq / chunk) * c.gstride > (int64_t(1) << 27)) continue;  // 1 GiB of pieces
-    } else {
-      const L2gGenericClass& g = l2g_gen_generic[c.cls];
-      c.gstride = (int64_t)g.ne * g.accs + 1;
-    }
+  bool rys = false;
+  for (size_t k = 0; k < p->classes.size(); ++k) {
+    const int64_t chunk = chunks[k];
+    if (!chunk) continue;
+    ClassWork& c = p->classes[k];
+    rys |= c.rys >= 0;
     c.piece_off = (int64_t)pb.size();
     c.pfirst_off = (int64_t)pf.size();
     for (int64_t i = c.first; i < c.first + c.count; ++i) {
@@ -736,15 +759,23 @@ void plan_pieces(l2g_eri_plan_s* p, l2g_context_s* ctx, const WorkLists* lists) 
     c.gpart_off = gtotal;
     gtotal += c.npieces * c.gstride;
   }
-  if (pb.empty()) return;
   hipStream_t st = ctx->stream;
-  upload(p->gp_bra, pb, st);
-  upload(p->gp_ket, pk, st);
-  upload(p->gp_meta, pm, st);
-  upload(p->gp_qidx, pq, st);
-  upload(p->gp_range, pr, st);
-  upload(p->gp_first, pf, st);
-  p->gpart.alloc(gtotal * sizeof(double));
+  try {
+    p->gpart.alloc(gtotal * sizeof(double));
+    upload(p->gp_bra, pb, st);
+    upload(p->gp_ket, pk, st);
+    upload(p->gp_meta, pm, st);
+    upload(p->gp_qidx, pq, st);
+    upload(p->gp_range, pr, st);
+    upload(p->gp_first, pf, st);
+  } catch (const L2gError& e) {
+    // beside a caller's own memory the pieces may not fit: the Rys classes then run unsplit
+    if (e.code != L2G_E_OOM || !rys) throw;
+    (void)hipGetLastError();
+    HIPCHK(hipStreamSynchronize(st));
+    plan_pieces(p, ctx, lists, false);
+    return;
+  }
   HIPCHK(hipStreamSynchronize(st));
 }
 

@@ -17,6 +17,7 @@
 
 #include "../../include/l2g.h"
 #include "eri_device.h"
+#include "launch_rules.h"
 
 extern const L2gClassInfo l2g_gen_classes[];
 extern const int l2g_gen_nclasses;
