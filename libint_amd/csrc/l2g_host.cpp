@@ -1206,12 +1206,9 @@ namespace {
 // Schwarz factors of n pairs of a class on its Rys kernel: the contracted
 // [e0|e0] values of (p|p) in pieces of kSchwarzPiece primitive quartets, the
 // finish launch into a scratch block per pair, and a reduction over each.  In
-// windows of up to kSchwarzDoubles values.  1275 pairs of a 5-atom molecule
+// windows of up to kSchwarzDoubles values (a pair alone never takes more).  1275 pairs of a 5-atom molecule
 // with f shells, K to 8: 78 -> 13.6 ms against a block per pair on the generic
 // kernel.
-constexpr int kSchwarzPiece = 64;
-constexpr int64_t kSchwarzDoubles = int64_t(1) << 25;
-
 void schwarz_rys(l2g_context_s* ctx, const L2gEriArgs& A0, const L2gClassInfo& ci, const std::vector<int>& pid,
                  const std::vector<int>& meta, const std::vector<int>& np, hipStream_t st) {
   int ne = 0;
@@ -1224,7 +1221,7 @@ void schwarz_rys(l2g_context_s* ctx, const L2gEriArgs& A0, const L2gClassInfo& c
     std::vector<long long> off{0};
     for (; i1 < pid.size(); ++i1) {
       const int64_t w = (int64_t)np[pid[i1]] * np[pid[i1]];
-      const int64_t pieces = std::max<int64_t>(1, (w + kSchwarzPiece - 1) / kSchwarzPiece);
+      const int64_t pieces = schwarz_pieces(w, stride);
       const int64_t n1 = nfun(ci.la, (meta[i1] >> 3) & 1), n2 = nfun(ci.lb, (meta[i1] >> 4) & 1);
       if (i1 > i0 && ((first.back() + pieces) * stride > kSchwarzDoubles ||
                       off.back() + n1 * n2 * n1 * n2 > kSchwarzDoubles))

@@ -32,4 +32,12 @@ inline std::vector<char> choose_pieces(const std::vector<PieceCandidate>& c, int
   return cut;
 }
 
+// Pieces of a shell pair's (p|p) loop of w primitive quartets for its Schwarz
+// factor: 64 each, longer where one pair's would not fit a window of
+// kSchwarzDoubles (a piece leaves `stride` of them).
+constexpr int64_t kSchwarzPiece = 64, kSchwarzDoubles = int64_t(1) << 25;
+inline int64_t schwarz_pieces(int64_t w, int64_t stride) {
+  return std::max<int64_t>(1, std::min((w + kSchwarzPiece - 1) / kSchwarzPiece, kSchwarzDoubles / stride));
+}
+
 }  // namespace l2g_impl

@@ -15,5 +15,9 @@ int main(int argc, char** argv) {
     for (char x : choose_pieces(c, cap ? cap : kPlanPieceDoubles)) std::printf("%d ", x);
     return 0;
   }
+  if (argc == 4 && !std::strcmp(argv[1], "schwarz")) {
+    std::printf("%lld %lld", (long long)schwarz_pieces(std::atoll(argv[2]), std::atoll(argv[3])), (long long)kSchwarzDoubles);
+    return 0;
+  }
   return 1;
 }

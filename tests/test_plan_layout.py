@@ -107,6 +107,28 @@ def test_classes_beyond_the_piece_scratch_run_unsplit(ctx):
     assert agree(v, w)
 
 
+@pytest.mark.parametrize("stride", [10 * 10 + 1, 74 * 74 + 1])  # (fs|fs), (ff|ff)
+@pytest.mark.parametrize("w", [1, 64, 65, 4096, 2500 ** 2, 46000 ** 2])
+def test_a_deep_pair_fits_the_schwarz_window(rules, w, stride):
+    pieces, cap = rules("schwarz", w, stride)
+    assert 1 <= pieces <= max(1, w) and pieces * stride <= cap
+    assert pieces == -(-w // 64) or (pieces + 1) * stride > cap
+
+
+@pytest.mark.gpu
+def test_schwarz_of_a_deep_f_pair(ctx):
+    """A pair of 30-primitive f shells, 810,000 primitive quartets: more than
+    the 6126 pieces that fit the window at 64 each.  Against the (p|p)
+    integrals of an ERI batch, at the integral bar on K^2."""
+    rng = np.random.default_rng(8)
+    sh = shells(rng, (3, 3), (30, 30))
+    b = la.Basis(ctx, la.BasisArrays.from_shells(sh))
+    say("case: Schwarz factor of an (f|f) pair of 900 primitive pairs")
+    K = la.schwarz(b, np.array([[0, 1]], np.int32), 0.0)
+    v, _, _ = la.compute_quartets(b, np.array([[0, 1, 0, 1]], np.int32), precision=0.0)
+    assert agree(K ** 2, np.array([np.abs(v).max()]))
+
+
 @pytest.mark.gpu
 def test_pieces_of_a_long_list(ctx):
     """100,000 quartets, one of 4096 primitive quartets, laid out right after
