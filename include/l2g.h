@@ -190,8 +190,8 @@ int l2g_eri_plan_device_output(l2g_eri_plan plan, double** d_out);
  * (HIP events on the context stream).  The code adds 10000 for an FP32
  * kernel, 20000 for the generic kernel and for the classes beyond the node
  * limit of the per-lane kernels ((df|ff), (ff|ff)), and 100000 where the
- * primitive loops of the class's quartets are split over lanes or blocks
- * (l2g_eri_plan_set_wave_split). */
+ * layout by batch gives the class another kernel, other groups of lanes or
+ * pieces than it has with that layout off (l2g_eri_plan_set_wave_split). */
 int l2g_eri_plan_stats(l2g_eri_plan plan, int cap, int* nclasses, int* class_code, int64_t* nquartets,
                        int64_t* nprim_quartets, float* ms);
 
@@ -217,23 +217,30 @@ int l2g_eri_plan_set_graph(l2g_eri_plan plan, int on);
 #define L2G_OPER_ERFC_COULOMB 2
 int l2g_eri_plan_set_operator(l2g_eri_plan plan, int oper, double omega);
 
-/* Split of deep primitive loops (default on).  Classes with a Rys kernel (all
- * but (ss|..)) whose deepest quartets would outlast the rest of their launch
- * are cut into pieces of their primitive loops, evaluated by separate blocks
- * and summed per quartet in piece order; (ss|..) classes of few quartets
- * (fewer than a quarter of the chip's lanes at one wave per SIMD) averaging
- * at least 16 primitive quartets run a wave per quartet, its contraction
- * summed as 64 serial partial sums joined by a fixed butterfly.  Both are
- * another order than libint's serial primitive loop
+/* Layout by batch (on by default; on = 2 is accepted as 1).  On: the kernel of
+ * a class and the way its quartets' primitive loops are shared follow from
+ * the whole batch.  Light classes run on 1, 4, 16 or 64 lanes per quartet
+ * where that is faster than the tiles of their quadrature kernel; classes on
+ * the latter whose deepest quartets would outlast the rest of their launch are
+ * cut into pieces of their primitive loops, evaluated by separate blocks and
+ * summed per quartet in piece order (at most 2 GiB of partial sums a plan).
+ * Each is another order than libint's serial primitive loop
  * (engine.impl.h:1306-1766): well-conditioned integrals agree with it to
  * rounding, ill-conditioned ones (large cancelling terms) stay within the
  * error the reference's own FP64 algorithm makes against the exact integral.
- * on = 2 is accepted as 1.  Off: classes of few quartets averaging at least
- * 64 primitive quartets with a total angular momentum of 7 and more run on
- * the generic kernel (a block per quartet), the rest unsplit.  Whether a
- * class is split depends on how many quartets of it the plan holds, so the
- * same quartet in plans of another composition can differ in its last bits;
- * with the split off an unsplit quartet's values depend on the quartet only.
+ * The same quartet in plans of another composition can differ in its last
+ * bits.
+ * Off: both follow from the class and the quartet's own number of primitive
+ * quartets (the lanes of the lightest classes, up to (ps|ps) and (fs|ps); the
+ * quadrature kernel of the others, on which quartets of 32 and of 128
+ * primitive quartets share up to 4 and 16 slots of a block), so a quartet has
+ * the same bits in every plan and from l2g_quartet_compute.  The exception:
+ * classes of total angular momentum 7 and more with few quartets (fewer than
+ * a quarter of the chip's lanes at one wave per SIMD) run on the generic
+ * kernel, another algorithm, when they average at least 64 primitive
+ * quartets.  No pieces: deep quartets take longer than with the layout by
+ * batch, and so do large batches of the classes that it moves to lanes (up to
+ * four times).
  * No counterpart in the reference. */
 int l2g_eri_plan_set_wave_split(l2g_eri_plan plan, int on);
 

@@ -352,6 +352,9 @@ AX = 'xyz'
 # arithmetic type of the recursion, HRR and transforms of the kernel being
 # emitted ('double', or 'float' for the reduced-precision variants)
 _R = 'double'
+# attenuated variant: the core integrals s^(m+1/2) F_m(sT), s = w^2/(w^2+rho), of erf(w r)/r, or with A.erfc
+# F_m(T) minus them
+_ATT = False
 # HRR and transforms with every fused multiply-add written out (for code whose
 # copies have to round alike; contraction is off there)
 _FUSED = False
@@ -576,8 +579,12 @@ def _emit_stage2(E, sfx, gb, gk, count):
     E(f"const double PQx{sfx} = Pg{sfx}.x - Qg{sfx}.x, PQy{sfx} = Pg{sfx}.y - Qg{sfx}.y, "
       f"PQz{sfx} = Pg{sfx}.z - Qg{sfx}.z;")
     E(f"pfac{sfx} = ok{sfx} ? pf{sfx} : 0.0;")
-    E(f"boys_fetch(gp{sfx} * gq{sfx} * oos{sfx} * (PQx{sfx} * PQx{sfx} + PQy{sfx} * PQy{sfx} + "
-      f"PQz{sfx} * PQz{sfx}), boysL, bq{sfx});")
+    T = f"gp{sfx} * gq{sfx} * oos{sfx} * (PQx{sfx} * PQx{sfx} + PQy{sfx} * PQy{sfx} + PQz{sfx} * PQz{sfx})"
+    if _ATT:  # the screening keeps the Coulomb prefactor, as the reference does
+        E(f"T{sfx} = {T};")
+        E(f"sw{sfx} = A.omega * A.omega / (A.omega * A.omega + gp{sfx} * gq{sfx} * oos{sfx});")
+        T = f"sw{sfx} * T{sfx}"
+    E(f"boys_fetch({T}, boysL, bq{sfx});")
 
 
 def emit_prim_loop(E, plan, graph, gi, accs):
@@ -596,6 +603,8 @@ def emit_prim_loop(E, plan, graph, gi, accs):
     E(f"double4 Qg = A.pp_P[{ka}], QCk = A.pp_PA[{ka}];")
     E(f"double2 xk = A.pp_aux[{ka}];")
     E("double pfac;")
+    if _ATT:
+        E("double sw, T;")
     E("L2gBoysArg bq;")
     E.block("")
     _emit_stage2(E, "", ga, ka, "" if gi == 0 else None)
@@ -610,9 +619,26 @@ def emit_prim_loop(E, plan, graph, gi, accs):
     E(f"const double4 Qgn = A.pp_P[{kan}], QCkn = A.pp_PA[{kan}];")
     E(f"const double2 xkn = A.pp_aux[{kan}];")
     E("double pfacn;")
+    if _ATT:
+        E("double swn, Tn;")
     E("L2gBoysArg bqn;")
     E(f"double F[{plan.L + 1}];")
-    E(f"boys_eval<{plan.L}>(bq, pfac, F);")
+    if _ATT:
+        E(f"boys_eval<{plan.L}>(bq, pfac * sqrt(sw), F);")
+        if plan.L > 0:
+            E.block("")
+            E("double sm = sw;")
+            E(f"for (int m = 1; m <= {plan.L}; ++m, sm *= sw) F[m] *= sm;")
+            E.end()
+        E.block("if (A.erfc)")
+        E("L2gBoysArg b1;")
+        E("boys_fetch(T, boysL, b1);")
+        E(f"double F1[{plan.L + 1}];")
+        E(f"boys_eval<{plan.L}>(b1, pfac, F1);")
+        E(f"for (int m = 0; m <= {plan.L}; ++m) F[m] = F1[m] - F[m];")
+        E.end()
+    else:
+        E(f"boys_eval<{plan.L}>(bq, pfac, F);")
     if _R == 'double':
         E("const double* Fv = F;")
     else:
@@ -645,11 +671,13 @@ def emit_prim_loop(E, plan, graph, gi, accs):
     emit_vrr_group(E, plan, graph, gi, accs, mid=mid)
     E("Pg = Pgn; PAk = PAkn; xb = xbn; Qg = Qgn; QCk = QCkn; xk = xkn;")
     E("pfac = pfacn; bq = bqn; ib = ibn; ik = ikn;")
+    if _ATT:
+        E("sw = swn; T = Tn;")
     E.end()  # p loop
     E.end()  # npq > 0
 
 
-def emit_class(plan: ClassPlan, block=128, mode='eri', waves=0, real='double'):
+def emit_class(plan: ClassPlan, block=128, mode='eri', waves=0, real='double', att=False):
     la, lb, lc, ld = plan.la, plan.lb, plan.lc, plan.ld
     graph = VrrGraph()
     ne, nf = len(plan.ecomps), len(plan.fcomps)
@@ -659,9 +687,9 @@ def emit_class(plan: ClassPlan, block=128, mode='eri', waves=0, real='double'):
       f"{G} target group(s)")
     E(f"// group sizes (bra components x ket targets): {[(len(g), len(f)) for g, f in plan.groups]}")
     E(f"// group graph nodes: {plan.group_nodes}; estimated peak live doubles: {plan.group_peak}")
-    global _R
-    _R = real
-    kname = f"l2g_{mode}{'32' if real == 'float' else ''}_{plan.name}"
+    global _R, _ATT
+    _R, _ATT = real, att
+    kname = f"l2g_{'att' if att else mode}{'32' if real == 'float' else ''}_{plan.name}"
     attr = f" __attribute__((amdgpu_waves_per_eu({waves}, {waves})))" if waves else ""
     if mode == 'fock':
         E("// Fock variant: digests each integral of the unique quartet into the")
@@ -685,6 +713,16 @@ def emit_class(plan: ClassPlan, block=128, mode='eri', waves=0, real='double'):
         E("const bool coop = A.coop != 0;")
         E("const int pst = 1;")
         E.block("for (int qi = coop ? (tid >> 6) : tid; qi < A.n; qi += coop ? (nthr >> 6) : nthr)")
+    elif mode == 'eri':
+        E("// the list's items in their tiers (A.lane_tier): on 64, 16, 4 or 1 lanes that")
+        E("// take their primitive quartets in turn; the accumulators are summed over the group")
+        E("const L2gLaneUnits lu(A);")
+        E.block("for (int u = tid >> 6; u < lu.n; u += nthr >> 6)")
+        E("int glog, first, end;")
+        E("lu.unit(A, u, glog, first, end);")
+        E("const int pst = 1 << glog, gl = lane & (pst - 1);")
+        E("const int qi = first + (lane >> glog);")
+        E("if (qi >= end) continue;")
     else:
         E("// a wave walks windows of A.win items of the list, runs of items of the same")
         E("// tier (l2g_lane_tier) at a time: each on 1, 4, 16 or 64 lanes that take its")
@@ -932,7 +970,7 @@ def emit_class(plan: ClassPlan, block=128, mode='eri', waves=0, real='double'):
     E.end()  # quartet loop
     E.ind -= 1
     E("}")
-    _R = 'double'
+    _R, _ATT = 'double', False
     return kname, E.text(), in_regs
 
 
@@ -976,14 +1014,18 @@ def generate(outdir, lmax=2, budget=160, nfiles=8, waves=0, only=None, budgets=N
     # reduced-precision variants hold twice as many values per register
     plans32 = [plan_class(p.la, p.lb, p.lc, p.ld, budget=2 * cfg((p.la, p.lb, p.lc, p.ld))[0]) for p in plans
                if max(p.la, p.lb, p.lc, p.ld) <= fp32_lmax] if 'fp32' in modes else []
-    # classes on the Rys kernels (gen_rys.py) have no other FP64 ERI or Fock kernel
+    # classes on the Rys kernels (gen_rys.py) have no other FP64 Fock kernel, and an ERI kernel here where batches of
+    # them are faster on it
     sys.path.insert(0, os.path.dirname(os.path.abspath(__file__)))
     import gen_rys
     ryscls = [c for c in classes if gen_rys.use(*c)] if 'rys' in modes else []
     jobs = []  # (plan, mode, real)
     for p in plans:
-        if (p.la, p.lb, p.lc, p.ld) not in ryscls:
+        c = (p.la, p.lb, p.lc, p.ld)
+        if c not in ryscls:
             jobs += [(p, m, 'double') for m in ('eri', 'fock') if m in modes]
+        elif gen_rys.lane_cost(*c) and 'eri' in modes:
+            jobs += [(p, m, 'double') for m in ('eri', 'att')]
         if 'schwarz' in modes and (p.la, p.lb) == (p.lc, p.ld):
             jobs.append((p, 'schwarz', 'double'))
     for p in plans32:
@@ -1000,7 +1042,7 @@ def generate(outdir, lmax=2, budget=160, nfiles=8, waves=0, only=None, budgets=N
         files[j].append(i)
         load[j] += w
     tables = {('eri', 'double'): [], ('schwarz', 'double'): [], ('fock', 'double'): [],
-              ('eri', 'float'): [], ('fock', 'float'): []}
+              ('eri', 'float'): [], ('fock', 'float'): [], ('att', 'double'): []}
     written = []
     for fi, idxs in enumerate(files):
         fn = os.path.join(outdir, f"eri_gen_{fi}.hip")
@@ -1009,7 +1051,8 @@ def generate(outdir, lmax=2, budget=160, nfiles=8, waves=0, only=None, budgets=N
         for i in sorted(idxs):
             p, mode, real = jobs[i]
             wv = cfg((p.la, p.lb, p.lc, p.ld))[1]
-            kname, code, in_regs = emit_class(p, mode=mode, waves=wv, real=real)
+            kname, code, in_regs = emit_class(p, mode='eri' if mode == 'att' else mode, waves=wv, real=real,
+                                              att=mode == 'att')
             parts.append(code)
             parts.append(f"void {kname}_launch(const L2gEriArgs& A, int grid, int block, hipStream_t s) {{")
             parts.append(f"  hipLaunchKernelGGL({kname}, dim3(grid), dim3(block), 0, s, A);")
@@ -1021,11 +1064,14 @@ def generate(outdir, lmax=2, budget=160, nfiles=8, waves=0, only=None, budgets=N
             with open(fn, 'w') as f:
                 f.write(new)
         written.append(fn)
+    for k in (('eri', 'double'), ('att', 'double')):  # the same order in both
+        tables[k].sort(key=lambda x: x[0].name)
     table, stable, ftable = tables[('eri', 'double')], tables[('schwarz', 'double')], tables[('fock', 'double')]
     table32, ftable32 = tables[('eri', 'float')], tables[('fock', 'float')]
     lines = ['// generated by libint_amd/codegen/gen_eri.py — do not edit',
              '#include "eri_device.h"', '']
-    for p, k, _ in table + stable + ftable + table32 + ftable32:
+    atable = tables[('att', 'double')]
+    for p, k, _ in table + stable + ftable + table32 + ftable32 + atable:
         lines.append(f"void {k}_launch(const L2gEriArgs& A, int grid, int block, hipStream_t s);")
     lines.append('')
     rys = {m: gen_rys.generate(ryscls, m) for m in ('eri', 'fock') if m in modes}
@@ -1049,27 +1095,30 @@ def generate(outdir, lmax=2, budget=160, nfiles=8, waves=0, only=None, budgets=N
     lines.append(f"extern const int l2g_gen_lmax = {lmax};")
     for name, tab in (("l2g_gen_classes", table), ("l2g_gen_schwarz", stable), ("l2g_gen_fock", ftable),
                       ("l2g_gen_classes32", table32), ("l2g_gen_fock32", ftable32),
-                      ("l2g_gen_rys", [])):
+                      ("l2g_gen_classes_att", atable), ("l2g_gen_rys", [])):
         lines.append(f"extern const L2gClassInfo {name}[] = {{")
         for p, k, in_regs in tab:
             ybuf = 0 if in_regs else len(p.ecomps) * ncart(p.lc) * ncart(p.ld) + \
                 (len(p.ecomps) * len(p.fcomps) if p.split_rows else 0)
-            if not in_regs and name in ("l2g_gen_classes", "l2g_gen_classes32"):
+            if not in_regs and name in ("l2g_gen_classes", "l2g_gen_classes32", "l2g_gen_classes_att"):
                 ybuf += ncart(p.la) * ncart(p.lb) * ncart(p.lc) * ncart(p.ld)  # staged output
             pays = cfg((p.la, p.lb, p.lc, p.ld))[2] if name in ("l2g_gen_classes32", "l2g_gen_fock32") else 0
+            cost = gen_rys.lane_cost(p.la, p.lb, p.lc, p.ld) if name == "l2g_gen_classes" and ryscls else None
             lines.append(f"  {{{p.la}, {p.lb}, {p.lc}, {p.ld}, {len(p.groups)}, {ybuf}, "
-                         f"{sum(p.group_nodes)}, {pays}, 0, 0, &{k}_launch}},")
+                         f"{sum(p.group_nodes)}, {pays}, 0, 0, {{{', '.join(map(str, cost or (0,)))}}}, &{k}_launch}},")
         rest = rys.get({'l2g_gen_fock': 'fock', 'l2g_gen_rys': 'eri'}.get(name), [])
         for p, n, _ in rest:
             over = int(not any((x.la, x.lb, x.lc, x.ld) == p.l for x in plans))
-            lines.append(f"  {{{', '.join(map(str, p.l))}, 1, 0, {int(p.cost())}, 0, {over}, {p.nt // p.q}, &{n}_launch}},")
+            lines.append(f"  {{{', '.join(map(str, p.l))}, 1, 0, {int(p.cost())}, 0, {over}, {p.nt // p.q}, {{0}}, "
+                         f"&{n}_launch}},")
         if not tab and not rest:
-            lines.append("  {0, 0, 0, 0, 0, 0, 0, 0, 0, 0, nullptr},")
+            lines.append("  {0, 0, 0, 0, 0, 0, 0, 0, 0, 0, {0}, nullptr},")
         lines.append("};")
     lines.append(f"extern const int l2g_gen_nclasses = {len(table)};")
     lines.append(f"extern const int l2g_gen_nschwarz = {len(stable)};")
     lines.append(f"extern const int l2g_gen_nfock = {len(ftable) + len(rys.get('fock', []))};")
     lines.append(f"extern const int l2g_gen_nrys = {len(rys.get('eri', []))};")
+    lines.append(f"extern const int l2g_gen_nclasses_att = {len(atable)};")
     lines.append(f"extern const int l2g_gen_nclasses32 = {len(table32)};")
     lines.append(f"extern const int l2g_gen_nfock32 = {len(ftable32)};")
     fn = os.path.join(outdir, "eri_table.cpp")

@@ -788,6 +788,50 @@ def use(la, lb, lc, ld):
     return True
 
 
+# Classes whose ERI batches have a per-lane kernel (gen_eri.py) besides their Rys kernel (launch_rules.h, LaneCost):
+# nanoseconds per quartet and per primitive quartet on the per-lane kernel, the same on the Rys kernel (150,000 quartets
+# of 1 and of 256 primitive quartets on one MI355X), and by how many microseconds a launch of few quartets takes longer
+# on the per-lane kernel, of 1 and of many primitive quartets (300 quartets).  The tiles of a Rys kernel spend more on
+# prologue, 2D integrals and epilogue than on the products in these classes: 150,000 (ps|ps) quartets of 256 primitive
+# quartets took 0.55 ms a lane per quartet, take 1.11 on tiles and 0.35 on the per-lane kernel; of 20,000 quartets with
+# K <= 6 820, 137 and 61 us.  The classes left out are slower there at 1 to 256 primitive quartets, or by less than a
+# tenth faster.
+LANE_COST = {
+    '0000': (0.027, 0.0045, 0.035, 0.0103, -14, -30),
+    '0010': (0.033, 0.0065, 0.126, 0.0145, -5, -7),
+    '0011': (0.075, 0.0075, 0.214, 0.0216, -3, -2),
+    '0020': (0.044, 0.0076, 0.202, 0.0209, -3, -1),
+    '0021': (0.124, 0.0113, 0.346, 0.0274, 0, 5),
+    '0022': (0.145, 0.0178, 0.463, 0.0403, 2, 13),
+    '0030': (0.054, 0.0104, 0.188, 0.0249, -21, -53),
+    '0031': (0.155, 0.0179, 0.415, 0.0415, 2, 11),
+    '0032': (0.553, 0.0246, 0.482, 0.0462, -26, -69),
+    '0033': (0.789, 0.0401, 3.812, 0.0934, 20, 68),
+    '1010': (0.068, 0.0082, 0.144, 0.0275, -5, -15),
+    '1011': (0.307, 0.0162, 0.181, 0.0381, -3, -11),
+    '1020': (0.113, 0.0132, 0.181, 0.0370, -7, -14),
+    '1021': (0.588, 0.0282, 0.230, 0.0541, 9, -1),  # through 16 and 256
+    '1022': (1.053, 0.0471, 0.428, 0.0877, 19, 24),
+    '1030': (0.124, 0.0251, 0.188, 0.0629, -5, -22),
+    '1031': (0.842, 0.0487, 0.329, 0.0800, 14, 17),
+    '1033': (3.344, 0.2538, 4.991, 0.1776, 96, 440),
+    '1111': (0.833, 0.0282, 0.364, 0.0564, 16, 54),
+    '1120': (0.445, 0.0286, 0.294, 0.0601, 10, 30),
+    '1130': (0.607, 0.0612, 0.395, 0.0718, 18, 100),
+    '2011': (0.497, 0.0245, 0.303, 0.0586, 11, 11),
+    '2020': (0.147, 0.0233, 0.275, 0.0589, -2, 20),
+    '2021': (0.943, 0.0567, 0.377, 0.0853, 22, 71),
+    '2030': (0.404, 0.0527, 0.361, 0.0721, 11, 69),
+    '2033': (6.405, 0.4845, 10.957, 0.3229, 164, 1014),
+    '3021': (1.517, 0.1116, 0.558, 0.1339, 46, 192),
+    '3030': (0.550, 0.1090, 0.522, 0.1882, 20, 142),
+}
+
+
+def lane_cost(la, lb, lc, ld):
+    return LANE_COST.get(f"{la}{lb}{lc}{ld}")
+
+
 def generate(classes, mode):
     """[(plan, kernel name, source)] of the classes."""
     return [(p, *emit(p, mode)) for p in (plan(*c) for c in classes)]

@@ -102,7 +102,9 @@ struct L2gEriArgs {
   int uniform_cart;
   int schwarz_norm;  // Schwarz kernels: 0 = max-abs norm, 1 = Frobenius norm
   int coop;          // Schwarz kernels: one wave per pair, its lanes splitting the primitive loop
-  int win;           // per-lane ERI and Fock kernels: work items of a wave's window (0: 64)
+  int win;           // per-lane Fock kernels: work items of a wave's window (0: 64)
+  // per-lane ERI kernels: items of the list on 64, 16, 4 lanes and one lane each, in this order
+  int lane_tier[4];
   double omega;      // > 0: erf-attenuated Coulomb erf(omega r)/r (0: Coulomb)
   int erfc;          // Rys ERI kernels, with omega > 0: 1 = erfc(omega r)/r in one pass, else 0
   int store_sub;     // ERI kernels: subtract from the output instead of storing
@@ -139,7 +141,32 @@ struct L2gEriArgs {
   const int* __restrict__ gpart_first;
 };
 
-// Lanes per item of the per-lane kernels, by its primitive quartets: 1, from
+// The wave-sized units of a per-lane ERI launch: 1, 4, 16 or 64 items each.
+// (Windows of 64 items of the sorted list instead left the deepest items
+// together in the first waves: 150,000 (ps|ps) quartets of K <= 6 took 1070 us,
+// now 233; (pp|pp) in FP64 4220, now 868.)
+struct L2gLaneUnits {
+  int e0, e1, e2, n;  // ends of the tiers' units
+  __device__ __forceinline__ explicit L2gLaneUnits(const L2gEriArgs& A)
+      : e0(A.lane_tier[0]), e1(e0 + (A.lane_tier[1] + 3) / 4), e2(e1 + (A.lane_tier[2] + 15) / 16),
+        n(e2 + (A.lane_tier[3] + 63) / 64) {}
+  // unit u: log2 of the lanes per item, the first item and the end of its tier
+  __device__ __forceinline__ void unit(const L2gEriArgs& A, int u, int& glog, int& first, int& end) const {
+    const int t0 = A.lane_tier[0], t1 = t0 + A.lane_tier[1], t2 = t1 + A.lane_tier[2];
+    if (u < e0) {
+      glog = 6, first = u, end = t0;
+    } else if (u < e1) {
+      glog = 4, first = t0 + (u - e0) * 4, end = t1;
+    } else if (u < e2) {
+      glog = 2, first = t1 + (u - e1) * 16, end = t2;
+    } else {
+      glog = 0, first = t2 + (u - e2) * 64, end = t2 + A.lane_tier[3];
+    }
+    glog = __builtin_amdgcn_readfirstlane(glog);
+  }
+};
+
+// Lanes per item of the per-lane Fock kernels, by its primitive quartets: 1, from
 // 16 on 4, from 64 on 16, from 512 on 64.  A lane walks its part serially,
 // each step waiting on a gather of pair data, and the lanes of a group read
 // neighbouring records; summing the group's accumulators (log2 of its size
@@ -209,6 +236,7 @@ struct L2gClassInfo {
   int fp32_pays;     // FP32 variants: measured faster than the class's FP64 kernel
   int over_limit;    // Rys kernels: the class is beyond the node limit of the per-lane kernels
   int lanes;         // Rys kernels: lanes per work item (0: a lane per item, with lane scratch)
+  float cost[6];     // per-lane ERI kernels of classes that have a Rys kernel too: LaneCost (launch_rules.h)
   L2gLaunchFn launch;
 };
 

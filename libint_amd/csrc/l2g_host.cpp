@@ -89,6 +89,9 @@ struct ClassWork {
   int rys = -1;       // index into l2g_gen_rys where the class runs on its Rys kernel
   int rys_cls = -1;   // the class's Rys kernel, whether it runs on it or not
   int rys_deep[2] = {0, 0};  // items in its tiers of deep quartets (rys_tier_of)
+  bool lane = false;         // on its per-lane kernel
+  LaneTiers tiers;           // lanes per item there
+  bool batch_layout = false;  // the kernel or the tiers depend on the batch (not with the split off)
   int gidx = -1;      // the class's program in the generic kernel's tables
   int64_t first, count;
   ClassSlot slot;     // grid, scratch region and stream of the launch
@@ -117,7 +120,7 @@ struct l2g_eri_plan_s {
   DevBuf gp_bra, gp_ket, gp_meta, gp_qidx, gp_range, gp_first, gpart;  // generic-class pieces
   int64_t ymax = 0;  // largest scratch doubles per lane over the classes
   int block = 128;
-  bool wave_split = true;  // classes of few deep quartets run a wave per quartet
+  bool wave_split = true;  // layouts by batch, deep loops cut into pieces (l2g_eri_plan_set_wave_split)
   std::vector<int> launch;  // classes in launch order (plan_slots)
   int oper = 0;             // 0 Coulomb, 1 erf-attenuated, 2 erfc-attenuated
   double omega = 0;
@@ -628,12 +631,14 @@ static int plan_create_impl(l2g_basis B, int64_t nq, const int32_t* quartets, do
 namespace {
 
 // Launch layout of a plan.  An FP64 class runs on its Rys kernel, a tile of
-// lanes per quartet; with wave_split (the default) a class whose deepest
-// quartets would outlast the rest has its primitive loops cut into pieces
-// (plan_pieces).  FP32 classes run on their per-lane kernels: a persistent
-// grid with enough blocks to fill every CU several times over, and the
-// lane-private scratch for it; deep quartets share their wave
-// (l2g_lane_tier).  Without wave_split, a class of few deep quartets (fewer
+// lanes per quartet, or where that is faster on its per-lane kernel
+// (lane_faster).  With wave_split (the default) a class on its Rys kernel
+// whose deepest quartets would outlast the rest has its primitive loops cut
+// into pieces (plan_pieces).  The per-lane kernels, FP32's among them, take a
+// persistent grid with enough blocks to fill every CU several times over, and
+// the lane-private scratch for it; deep quartets share their wave
+// (lane_tiers).  Without wave_split a class's kernel and lanes do not depend
+// on the batch, but for this: a class of few deep quartets (fewer
 // than a quarter of the chip's lanes at one wave per SIMD, averaging at least
 // 64 primitive quartets) and total angular momentum 7 or more runs on the
 // generic kernel, a block per quartet whose threads split the targets.
@@ -779,6 +784,17 @@ void plan_pieces(l2g_eri_plan_s* p, l2g_context_s* ctx, const WorkLists* lists, 
   HIPCHK(hipStreamSynchronize(st));
 }
 
+// A class's items on its per-lane kernel: all or none, and their lanes.
+bool on_lanes(const l2g_context_s* ctx, const ClassWork& c, const int* w, bool by_batch, LaneTiers& t) {
+  const L2gClassInfo& ci = (c.fp32 ? l2g_gen_classes32 : l2g_gen_classes)[c.spec_cls];
+  if (c.rys_cls >= 0) {
+    const LaneCost k = lane_cost(ci);
+    if (!(by_batch ? lane_faster(k, c.count, c.nprimq, w[0]) : lane_always(k))) return false;
+  }
+  t = lane_tiers(w, c.count, lane_length(class_targets(ci), c.nprimq, (int64_t)ctx->ncu * 256, by_batch));
+  return true;
+}
+
 void plan_layout(l2g_eri_plan_s* p, l2g_context_s* ctx, const WorkLists* lists) {
   p->block = 128;
   std::vector<int64_t> lanes, yd;
@@ -790,22 +806,24 @@ void plan_layout(l2g_eri_plan_s* p, l2g_context_s* ctx, const WorkLists* lists) 
     const bool deep_generic = !p->wave_split && !c.fp32 && c.gidx >= 0 && few &&
                               c.nprimq >= L2G_GENERIC_MIN_DEPTH * c.count && class_l(c) >= L2G_GENERIC_MIN_L;
     c.rys = deep_generic ? -1 : c.rys_cls;
-    if (c.rys >= 0) {
-      c.generic = false;
-      lanes.push_back(c.count * l2g_gen_rys[c.rys].lanes);
-      yd.push_back(0);
-      continue;
-    }
+    c.lane = c.batch_layout = false;
     if (deep_generic) {
       c.generic = true;
       c.cls = c.gidx;
+    } else if (!c.native_generic) {
+      const int* const w = p->itemw.data() + c.first;
+      LaneTiers off;
+      c.lane = on_lanes(ctx, c, w, p->wave_split, c.tiers);
+      if (c.lane) c.rys = -1;
+      c.batch_layout = on_lanes(ctx, c, w, false, off) != c.lane || (c.lane && !(off == c.tiers));
     }
+    if (c.rys >= 0) c.generic = false;
     // the generic kernel runs a block per quartet, no lane scratch, a few
     // blocks per CU (LDS bound): up to 4 quartets per CU leave the chip
     // underfilled, so such classes count as small and run beside each other
     // on the side streams
-    lanes.push_back(c.generic ? c.count * 64 : l2g_window_lanes(c.count, ctx->ncu));
-    yd.push_back(c.generic ? 0 : (c.fp32 ? l2g_gen_classes32 : l2g_gen_classes)[c.cls].ybuf_doubles);
+    lanes.push_back(c.generic ? c.count * 64 : c.lane ? 64 * c.tiers.units() : c.count * l2g_gen_rys[c.rys].lanes);
+    yd.push_back(c.lane ? (c.fp32 ? l2g_gen_classes32 : l2g_gen_classes)[c.cls].ybuf_doubles : 0);
   }
   plan_pieces(p, ctx, lists);
   for (size_t i = 0; i < p->classes.size(); ++i)
@@ -819,6 +837,11 @@ void plan_layout(l2g_eri_plan_s* p, l2g_context_s* ctx, const WorkLists* lists) 
   for (const auto& c : p->classes) {
     if (c.rys >= 0) {  // lane operations per primitive quartet, at 2 waves per SIMD on a part of the chip
       cost.push_back((double)c.nprimq * l2g_gen_rys[c.rys].nodes * 4e-4 + 3.0 * (double)c.count);
+      continue;
+    }
+    if (c.lane && !c.fp32 && c.rys_cls >= 0) {  // on the scale of the former (its cost a primitive quartet: 15 to 35 rys_p)
+      const LaneCost k = lane_cost(l2g_gen_classes[c.cls]);
+      cost.push_back(25.0 * (k.lane_q * (double)c.count + k.lane_p * (double)c.nprimq));
       continue;
     }
     const double vals = c.generic ? (double)l2g_gen_generic[c.cls].nvals
@@ -921,12 +944,13 @@ int l2g_eri_plan_execute(l2g_eri_plan p, double* d_out) {
     bool sides = false;
     for (auto& c : p->classes) sides |= c.slot.side >= 0;
     sides &= !capture;
-    // attenuated passes run on the class's Rys kernel, or on the generic
-    // kernel, whose core-integral step takes omega too
+    // attenuated passes run on the class's Rys kernel, on the attenuated
+    // variant of its per-lane kernel, or on the generic kernel, whose
+    // core-integral step takes omega too
     // Passes (attenuation, subtract): Coulomb; erf = one attenuated pass
     // (omega = 0 gives exact zeros as Coulomb minus Coulomb); erfc =
     // Coulomb minus the erf pass, both per class on the class's stream, or
-    // one pass over both on a Rys kernel (rys_prim)
+    // one pass over both on a Rys or per-lane kernel
     std::vector<std::pair<double, int>> passes;
     if (p->oper == 0) passes = {{0.0, 0}};
     else if (p->oper == 1) passes = p->omega > 0 ? std::vector<std::pair<double, int>>{{p->omega, 0}}
@@ -937,7 +961,7 @@ int l2g_eri_plan_execute(l2g_eri_plan p, double* d_out) {
     for (int ic : p->launch) {
     ClassWork& c = p->classes[(size_t)ic];
     for (size_t ps = 0; ps < passes.size(); ++ps) {
-      const bool erfc = c.rys >= 0 && p->oper == 2 && p->omega > 0;
+      const bool erfc = !c.generic && !c.fp32 && p->oper == 2 && p->omega > 0;
       if (erfc && ps) continue;
       const bool last = erfc || ps + 1 == passes.size();
       A.omega = erfc ? p->omega : passes[ps].first;
@@ -953,7 +977,14 @@ int l2g_eri_plan_execute(l2g_eri_plan p, double* d_out) {
       A.qidx = p->qidx.as<long long>() + c.first;
       A.n = (int)c.count;
       if (!capture && ps == 0) HIPCHK(hipEventRecord(c.ev0, cs));
-      if (c.rys >= 0) {
+      // (the FP32 kernels have no attenuated form)
+      if (c.lane && (A.omega == 0 || !c.fp32)) {
+        std::copy(c.tiers.n, c.tiers.n + 4, A.lane_tier);
+        // exactly the slot's grid: the scratch region holds grid * block lanes
+        (c.fp32 ? l2g_gen_classes32 : A.omega > 0 ? l2g_gen_classes_att : l2g_gen_classes)[c.cls].launch(
+            A, c.slot.grid, p->block, cs);
+        LAUNCHCHK(std::string("ERI kernel of class ") + std::to_string(c.cls));
+      } else if (c.rys >= 0) {
         const L2gClassInfo& ci = l2g_gen_rys[c.rys];
         L2gEriArgs P = A;
         if (c.npieces) {  // pieces of the primitive loops, then the sum per quartet
@@ -972,14 +1003,12 @@ int l2g_eri_plan_execute(l2g_eri_plan p, double* d_out) {
           P.gpart = p->gpart.as<double>() + c.gpart_off;
           P.gpart_stride = c.gstride;
           P.gpart_first = p->gp_first.as<int>() + c.pfirst_off;
+        } else {
+          P.rys_deep[0] = c.rys_deep[0], P.rys_deep[1] = c.rys_deep[1];
         }
-        if (!c.npieces) P.rys_deep[0] = c.rys_deep[0], P.rys_deep[1] = c.rys_deep[1];
         ci.launch(P, 0, 0, cs);
         LAUNCHCHK(std::string("Rys ERI kernel of class ") + std::to_string(c.rys));
-        if (!capture && last) HIPCHK(hipEventRecord(c.ev1, cs));
-        continue;
-      }
-      if (c.generic || A.omega > 0) {  // the attenuated pass of erf / erfc
+      } else {  // the generic kernel's classes; the attenuated pass of erf / erfc in FP32
         // one block per quartet, persistent over the class
         if (c.gidx < 0) throw L2gError(L2G_E_LMAX, "no generic-kernel program for this class");
         const L2gGenericClass& gc = l2g_gen_generic[c.gidx];
@@ -1007,12 +1036,6 @@ int l2g_eri_plan_execute(l2g_eri_plan p, double* d_out) {
           const int grid = (int)std::min<int64_t>((int64_t)ctx->ncu * 8, c.count);
           launch_generic(kGenericEri, A, gc, ctx->gprog.as<int4>(), ctx->gidx.as<int>(), grid, cs);
         }
-      } else {
-        const L2gClassInfo& ci = (c.fp32 ? l2g_gen_classes32 : l2g_gen_classes)[c.cls];
-        A.win = l2g_lane_window(c.count, ctx->ncu);
-        // exactly the slot's grid: the scratch region holds grid * block lanes
-        ci.launch(A, c.slot.grid, p->block, cs);
-        LAUNCHCHK(std::string("ERI kernel of class ") + std::to_string(c.cls));
       }
       if (!capture && last) HIPCHK(hipEventRecord(c.ev1, cs));
     }
@@ -1153,7 +1176,7 @@ int l2g_eri_plan_stats(l2g_eri_plan p, int cap, int* ncls, int* code, int64_t* n
       const bool generic = c.rys >= 0 ? l2g_gen_rys[c.rys].over_limit != 0 : c.generic;
       if (code)
         code[i] = la * 1000 + lb * 100 + lc * 10 + ld + (c.fp32 ? 10000 : 0) + (generic ? 20000 : 0) +
-                  (c.rys >= 0 && c.npieces ? 100000 : 0);
+                  ((c.rys >= 0 && c.npieces) || c.batch_layout ? 100000 : 0);
       if (nquart) nquart[i] = c.count;
       if (nprimq) nprimq[i] = c.nprimq;
       if (ms) {

@@ -29,6 +29,21 @@ extern const L2gClassInfo l2g_gen_classes32[];
 extern const int l2g_gen_nclasses32;
 extern const L2gClassInfo l2g_gen_fock32[];
 extern const int l2g_gen_nfock32;
+// attenuated (erf, erfc) variants of l2g_gen_classes, in its order
+extern const L2gClassInfo l2g_gen_classes_att[];
+extern const int l2g_gen_nclasses_att;
+inline l2g_impl::LaneCost lane_cost(const L2gClassInfo& c) {
+  return {c.cost[0], c.cost[1], c.cost[2], c.cost[3], c.cost[4], c.cost[5]};
+}
+// contracted [e0|f0] targets of a class
+inline int class_targets(const L2gClassInfo& c) {
+  auto comps = [](int l1, int l2) {
+    int n = 0;
+    for (int l = l1; l <= l1 + l2; ++l) n += (l + 1) * (l + 2) / 2;
+    return n;
+  };
+  return comps(c.la, c.lb) * comps(c.lc, c.ld);
+}
 // Rys kernels of the ERI batches (codegen/gen_rys.py) and their node table
 extern const L2gClassInfo l2g_gen_rys[];
 extern const int l2g_gen_nrys;

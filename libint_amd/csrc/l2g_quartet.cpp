@@ -36,6 +36,7 @@ int64_t quartet_ylane(int max_l) {
   int64_t y = 0;
   for (int i = 0; i < l2g_gen_nclasses; ++i) {
     const L2gClassInfo& c = l2g_gen_classes[i];
+    if (!lane_always(lane_cost(c))) continue;  // the others run on their Rys kernel
     if (std::max(std::max(c.la, c.lb), std::max(c.lc, c.ld)) <= max_l) y = std::max<int64_t>(y, c.ybuf_doubles);
   }
   return y;
@@ -164,6 +165,7 @@ void quartet_compute_impl(l2g_context_s* ctx, const QuartetBuffers& qb, const in
   const int64_t n = (int64_t)nfun(l[0], pure[0]) * nfun(l[1], pure[1]) * nfun(l[2], pure[2]) * nfun(l[3], pure[3]);
   const int cls = ctx->force_generic ? -1 : ctx->class_of[l[b1]][l[b2]][l[k1]][l[k2]];
   const int rys = ctx->force_generic ? -1 : ctx->rys_of[l[b1]][l[b2]][l[k1]][l[k2]];
+  const bool lane = cls >= 0 && lane_always(lane_cost(l2g_gen_classes[cls]));
   const int gcls = ctx->generic_of[l[b1]][l[b2]][l[k1]][l[k2]];
   if (cls < 0 && gcls < 0) throw L2gError(L2G_E_LMAX, "no kernel for this angular momentum class");
   // stage the inputs
@@ -223,24 +225,27 @@ void quartet_compute_impl(l2g_context_s* ctx, const QuartetBuffers& qb, const in
                                          : std::vector<std::pair<double, int>>{{0.0, 0}, {0.0, 1}};
   else passes = omega > 0 ? std::vector<std::pair<double, int>>{{0.0, 0}, {omega, 1}}
                           : std::vector<std::pair<double, int>>{{0.0, 0}};
-  if (rys >= 0 && oper == 2 && omega > 0) {  // erfc in one pass
+  if ((lane || rys >= 0) && oper == 2 && omega > 0) {  // erfc in one pass
     passes = {{omega, 0}};
     A.erfc = 1;
   }
   for (const auto& ps : passes) {
     A.omega = ps.first;
     A.store_sub = ps.second;
-    if (rys >= 0) {
+    if (lane) {
+      const int w = pb.np[0] * pb.np[1];
+      const LaneTiers t = lane_tiers(&w, 1, lane_length(class_targets(l2g_gen_classes[cls]), w, 1, false));
+      std::copy(t.n, t.n + 4, A.lane_tier);
+      (A.omega > 0 ? l2g_gen_classes_att : l2g_gen_classes)[cls].launch(A, 1, kQuartetBlock, st);
+      LAUNCHCHK("ERI kernel (quartet engine)");
+    } else if (rys >= 0) {
       const int tier = rys_tier_of((long long)pb.np[0] * pb.np[1]);
       if (tier < 2) A.rys_deep[tier] = 1;
       l2g_gen_rys[rys].launch(A, 1, kQuartetBlock, st);
       LAUNCHCHK("Rys ERI kernel (quartet engine)");
-    } else if (cls < 0 || A.omega > 0) {
+    } else {
       if (gcls < 0) throw L2gError(L2G_E_LMAX, "no generic-kernel program for this class");
       launch_generic(kGenericEri, A, l2g_gen_generic[gcls], ctx->gprog.as<int4>(), ctx->gidx.as<int>(), 1, st);
-    } else {
-      l2g_gen_classes[cls].launch(A, 1, kQuartetBlock, st);
-      LAUNCHCHK("ERI kernel (quartet engine)");
     }
   }
   HIPCHK(hipMemcpyAsync(qb.hout, dout, (size_t)(n + 1) * sizeof(double), hipMemcpyDeviceToHost, st));

@@ -10,6 +10,9 @@ import numpy as np
 import pytest
 
 import libint_amd as la
+import oracle
+sys.path.insert(0, os.path.join(os.path.dirname(la.__file__), "codegen"))
+import gen_rys  # noqa: E402
 
 ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
 CSRC = os.path.join(ROOT, "libint_amd", "csrc")
@@ -145,3 +148,97 @@ def test_pieces_of_a_long_list(ctx):
     v, nz = plan.download()
     w, nw = values(plan, False)
     assert agree(v, w) and np.array_equal(nz, nw)
+
+
+def test_lanes_per_item(rules):
+    """Tiers from len, 4 len and 32 len primitive quartets on; units of 64, 16, 4 and 1 items."""
+    assert rules("tiers", 8, 256, 255, 32, 31, 8, 7, 1) == [1, 2, 2, 2, 4]
+    assert rules("tiers", 16, *[511] * 5, *[16] * 17, *[15] * 65) == [0, 5, 17, 65, 2 + 2 + 2]
+    assert rules("tiers", 8, *[1] * 64) == [0, 0, 0, 64, 1]
+    assert rules("tiers", 8, 100000) == [1, 0, 0, 0, 1]
+    # by the class alone, and where the batch fills the chip anyway
+    assert [rules("length", t, 10 ** 9, 65536, 0)[0] for t in (1, 24, 25, 32, 33, 444)] == [8, 8, 8, 8, 16, 16]
+    assert [rules("length", t, 2 * 65536 * 100, 65536, 1)[0] for t in (24, 25, 33)] == [8, 100, 100]
+    assert rules("length", 81, 2 * 65536 * 15, 65536, 1) == [16]
+
+
+def route(rules, c, n, nprim, wmax):
+    return bool(rules("faster", *(gen_rys.LANE_COST.get(c) or (0,) * 6), n, nprim, wmax)[0])
+
+
+@pytest.mark.parametrize("c, n, w, lane", [
+    # (class, quartets, primitive quartets each, per-lane kernel): on the sides of the crossings that were measured
+    ("1010", 1, 1, True), ("1010", 150000, 1296, True), ("0032", 1, 1, True),
+    ("1111", 150000, 1, False), ("1111", 300, 256, False), ("1111", 20000, 256, True), ("1111", 150000, 256, True),
+    ("0033", 300, 1, False), ("0033", 20000, 1, True), ("0033", 300, 256, False), ("0033", 60000, 16, True),
+    ("1033", 150000, 1, True), ("1033", 150000, 16, False), ("3030", 60000, 256, True), ("3030", 3000, 16, False),
+    ("2222", 150000, 1, False), ("2222", 150000, 256, False), ("2121", 10 ** 6, 256, False),  # Rys kernel only
+])
+def test_which_kernel_a_class_runs_on(rules, c, n, w, lane):
+    assert route(rules, c, n, n * w, w) == lane
+
+
+LANE_CLASSES = sorted(gen_rys.LANE_COST)
+
+
+def lane_case(c, pure, seed):
+    """200 quartets of a class in mixed caller orders: primitive quartets on both sides of the tiers (8, 32, 256 and 16,
+    64, 512), solid harmonics or Cartesians."""
+    l = [int(x) for x in c]
+    rng = np.random.default_rng(seed)
+    ks = [(1, 1, 1, 1), (7, 1, 1, 1), (2, 2, 2, 1), (3, 1, 5, 1), (4, 2, 2, 1), (31, 1, 1, 1), (4, 2, 4, 1), (9, 1, 7, 1),
+          (4, 4, 2, 2), (15, 1, 17, 1), (4, 4, 4, 4), (7, 1, 73, 1), (8, 4, 4, 4)]
+    if sum(l) > 6:
+        ks = ks[:8]
+    sh = [x for k in ks for x in shells(rng, l, k, pure)]
+    q = np.array([[4 * (n % len(ks)) + x for x in range(4)] for n in range(200)], np.int32)
+    q[1::3] = q[1::3][:, [1, 0, 2, 3]]
+    # (pp|ds) and (ds|pp) are classes of their own
+    q[2::3] = q[2::3][:, [1, 0, 3, 2] if l[0] + l[1] == l[2] + l[3] else [2, 3, 1, 0]]
+    return la.BasisArrays.from_shells(sh), q[rng.permutation(200)]
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("c", LANE_CLASSES)
+@pytest.mark.parametrize("pure", [True, False])
+def test_per_lane_kernels(ctx, rules, c, pure):
+    """Every class that has a per-lane kernel, in a batch that runs on it (the 200 quartets repeated until the rule takes
+    it there), each operator, against the oracle: the values of every repeat."""
+    arrays, q = lane_case(c, pure, 3 + sum(map(int, c)))
+    b = la.Basis(ctx, arrays)
+    if c in ("1033", "2033"):  # these only in large batches of shallow quartets
+        q = q[(q < 4).all(1)]
+    w = arrays.nprim[q].prod(1)
+    reps = next(r for r in (1, 50, 150, 400, 1000, 3000) if route(rules, c, r * len(q), r * int(w.sum()), int(w.max())))
+    say(f"case: per-lane kernel of ({c}), pure {pure}, {len(q)} quartets {reps} times")
+    plan = la.EriPlan(b, np.tile(q, (reps, 1)))
+    # reported where the kernel is not the one of the split turned off
+    assert reps == 1 or [s["wave"] for s in plan.stats()] == [True]
+    for oper, omega in ((la.COULOMB, 0.0), (la.ERF_COULOMB, 0.6), (la.ERFC_COULOMB, 0.6), (la.ERFC_COULOMB, 0.0)):
+        plan.set_operator(oper, omega)
+        plan.execute()
+        g, nz = plan.download()
+        o, _, onz = oracle.eri_quartets(arrays, q, **(dict(oper=oper, omega=omega) if oper else {}))
+        g = g.reshape(reps, -1)
+        assert np.array_equal(nz.reshape(reps, -1), np.tile(onz, (reps, 1)))
+        assert all(agree(x, o) for x in (g[0], g[reps // 2], g[-1])), (oper, omega)
+        if reps > 1:
+            assert agree(g, g[0])
+    plan._release()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("c", [c for c in LANE_CLASSES if gen_rys.LANE_COST[c][4] <= 1 and gen_rys.LANE_COST[c][5] <= 1])
+def test_light_classes_have_the_same_bits_in_every_batch(ctx, c):
+    """With the split off: a quartet alone, among others and from the quartet engine."""
+    arrays, q = lane_case(c, True, 11)
+    b = la.Basis(ctx, arrays)
+    say(f"case: bits of ({c}) quartets")
+    plan = la.EriPlan(b, np.tile(q, (40, 1)))
+    v, _ = values(plan, False)
+    v = v.reshape(40, -1)
+    assert (v == v[0]).all()
+    off = np.append(la.EriPlan(b, q).offsets(), v.shape[1])
+    for k in range(0, 200, 9):
+        one = la.EriPlan(b, q[k:k + 1])
+        assert np.array_equal(values(one, False)[0], v[0][off[k]:off[k + 1]]), k
