@@ -238,7 +238,8 @@ int l2g_eri_plan_set_operator(l2g_eri_plan plan, int oper, double omega);
  * classes of total angular momentum 7 and more with few quartets (fewer than
  * a quarter of the chip's lanes at one wave per SIMD) run on the generic
  * kernel, another algorithm, when they average at least 64 primitive
- * quartets.  No pieces: deep quartets take longer than with the layout by
+ * quartets, (df|ff) and (ff|ff) also when one quartet is far deeper than the
+ * rest together.  No pieces: deep quartets take longer than with the layout by
  * batch, and so do large batches of the classes that it moves to lanes (up to
  * four times).
  * No counterpart in the reference. */

@@ -641,7 +641,8 @@ namespace {
 // on the batch, but for this: a class of few deep quartets (fewer
 // than a quarter of the chip's lanes at one wave per SIMD, averaging at least
 // 64 primitive quartets) and total angular momentum 7 or more runs on the
-// generic kernel, a block per quartet whose threads split the targets.
+// generic kernel, a block per quartet whose threads split the targets, and so
+// does a class beyond the node limit with a far deeper quartet (unsplit_generic).
 #ifndef L2G_GENERIC_MIN_DEPTH
 #define L2G_GENERIC_MIN_DEPTH 64
 #endif
@@ -803,8 +804,11 @@ void plan_layout(l2g_eri_plan_s* p, l2g_context_s* ctx, const WorkLists* lists) 
     c.generic = c.native_generic;
     c.cls = c.spec_cls;
     const bool few = c.count * 4 <= (int64_t)ctx->ncu * 256;
-    const bool deep_generic = !p->wave_split && !c.fp32 && c.gidx >= 0 && few &&
-                              c.nprimq >= L2G_GENERIC_MIN_DEPTH * c.count && class_l(c) >= L2G_GENERIC_MIN_L;
+    const bool deep_generic =
+        !p->wave_split && !c.fp32 && c.gidx >= 0 &&
+        ((few && c.nprimq >= L2G_GENERIC_MIN_DEPTH * c.count && class_l(c) >= L2G_GENERIC_MIN_L) ||
+         (c.rys_cls >= 0 && l2g_gen_rys[c.rys_cls].over_limit &&
+          unsplit_generic(c.count, c.nprimq, p->itemw[(size_t)c.first], ctx->ncu)));
     c.rys = deep_generic ? -1 : c.rys_cls;
     c.lane = c.batch_layout = false;
     if (deep_generic) {

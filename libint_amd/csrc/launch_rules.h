@@ -91,6 +91,16 @@ inline bool lane_faster(const LaneCost& c, int64_t n, int64_t nprim, int64_t wma
   return lane < 0.95 * ((double)c.rys_q * n + (double)c.rys_p * nprim);
 }
 
+// Layout off, classes of so large a block that few of a Rys kernel's slots
+// share a deep quartet ((df|ff) and (ff|ff): 3): a quartet's loop takes 0.8 to
+// 1.5 us a primitive quartet there, the generic kernel, which cuts it, 0.6 to
+// 1.4 ms and 0.045 to 0.075 us a primitive quartet of the class.  One quartet
+// of 4096 among 99 of 1: (df|ff) 3.4 against 0.74 ms, (ff|ff) 6.1 against 1.7;
+// 60 of them 3.5 against 11.9 ms.
+inline bool unsplit_generic(int64_t count, int64_t nprim, int64_t wmax, int64_t ncu) {
+  return count <= 16 * ncu && wmax > 1000 + nprim / 18;
+}
+
 // Pieces of a shell pair's (p|p) loop of w primitive quartets for its Schwarz
 // factor: 64 each, longer where one pair's would not fit a window of
 // kSchwarzDoubles (a piece leaves `stride` of them).

@@ -39,5 +39,9 @@ int main(int argc, char** argv) {
     std::printf("%d %d", lane_faster(k, std::atoll(argv[8]), std::atoll(argv[9]), std::atoll(argv[10])), lane_always(k));
     return 0;
   }
+  if (argc == 5 && !std::strcmp(argv[1], "unsplit")) {
+    std::printf("%d", unsplit_generic(std::atoll(argv[2]), std::atoll(argv[3]), std::atoll(argv[4]), 256));
+    return 0;
+  }
   return 1;
 }

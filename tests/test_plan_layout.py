@@ -242,3 +242,25 @@ def test_light_classes_have_the_same_bits_in_every_batch(ctx, c):
     for k in range(0, 200, 9):
         one = la.EriPlan(b, q[k:k + 1])
         assert np.array_equal(values(one, False)[0], v[0][off[k]:off[k + 1]]), k
+
+
+@pytest.mark.parametrize("count, nprim, wmax, generic", [
+    (100, 4096 + 99, 4096, True), (508, 8 * 4096 + 500, 4096, True), (20, 20 * 4096, 4096, False), (100, 1099, 1000, False),
+    (1, 1059, 1059, True), (1, 1058, 1058, False), (4096, 4095 + 4096, 4096, True), (4097, 4096 + 4096, 4096, False),
+])
+def test_deep_quartets_of_the_largest_classes_unsplit(rules, count, nprim, wmax, generic):
+    assert bool(rules("unsplit", count, nprim, wmax)[0]) == generic
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("c", ["3233", "3333"])
+def test_one_deep_quartet_unsplit(ctx, c):
+    """A quartet of 1536 primitive quartets among shallow ones, layout off, against the oracle."""
+    l = [int(x) for x in c]
+    rng = np.random.default_rng(l[1])
+    arrays = la.BasisArrays.from_shells(shells(rng, l, (8, 6, 8, 4)) + shells(rng, l, (1, 1, 1, 1)))
+    q = np.array([[4, 5, 6, 7]] * 30 + [[0, 1, 2, 3]], np.int32)
+    say(f"case: one deep ({c}) quartet")
+    v, nz = values(la.EriPlan(la.Basis(ctx, arrays), q), False)
+    o, _, onz = oracle.eri_quartets(arrays, q)
+    assert agree(v, o) and np.array_equal(nz, onz)
