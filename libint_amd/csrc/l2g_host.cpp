@@ -117,7 +117,7 @@ struct l2g_eri_plan_s {
   DevBuf pair_first, pair_np, pair_AB, ppP, ppPA, ppAux, ppNs;
   DevBuf out, ybuf, nz;
   std::vector<int> itemw;  // primitive quartets of each work item (host)
-  DevBuf gp_bra, gp_ket, gp_meta, gp_qidx, gp_range, gp_first, gpart;  // generic-class pieces
+  DevBuf gp_bra, gp_ket, gp_meta, gp_range, gp_first, gpart;  // pieces of primitive loops
   int64_t ymax = 0;  // largest scratch doubles per lane over the classes
   int block = 128;
   bool wave_split = true;  // layouts by batch, deep loops cut into pieces (l2g_eri_plan_set_wave_split)
@@ -153,7 +153,6 @@ namespace {
 // a plan's work-item arrays on the host, in launch order
 struct WorkLists {
   std::vector<int> bra, ket, meta;
-  std::vector<long long> qidx;
 };
 // launch layout, defined below; without `lists` the arrays are read back where needed
 void plan_layout(l2g_eri_plan_s* p, l2g_context_s* ctx, const WorkLists* lists);
@@ -554,7 +553,7 @@ static int plan_create_impl(l2g_basis B, int64_t nq, const int32_t* quartets, do
     // flatten: classes in table order, each sorted by contraction depth
     WorkLists wl;
     std::vector<int>&bra = wl.bra, &ket = wl.ket, &meta = wl.meta;
-    std::vector<long long> off, &qidx = wl.qidx;
+    std::vector<long long> off, qidx;
     bra.reserve(nq);
     ket.reserve(nq);
     meta.reserve(nq);
@@ -677,7 +676,7 @@ int class_l(const ClassWork& c) {
 // pieces leave more partial sums than loops saved.
 constexpr int64_t kRysPiece = 24, kRysSerial = 96;
 void plan_pieces(l2g_eri_plan_s* p, l2g_context_s* ctx, const WorkLists* lists, bool cut_rys = true) {
-  for (DevBuf* d : {&p->gp_bra, &p->gp_ket, &p->gp_meta, &p->gp_qidx, &p->gp_range, &p->gp_first, &p->gpart})
+  for (DevBuf* d : {&p->gp_bra, &p->gp_ket, &p->gp_meta, &p->gp_range, &p->gp_first, &p->gpart})
     *d = DevBuf();
   // which classes, in pieces of what length
   std::vector<int64_t> chunks(p->classes.size(), 0);
@@ -728,17 +727,15 @@ void plan_pieces(l2g_eri_plan_s* p, l2g_context_s* ctx, const WorkLists* lists, 
   WorkLists back;
   if (!lists) {  // read back once
     const size_t n = (size_t)p->nq;
-    back.bra.resize(n), back.ket.resize(n), back.meta.resize(n), back.qidx.resize(n);
+    back.bra.resize(n), back.ket.resize(n), back.meta.resize(n);
     // the context's stream does not wait for hipMemcpy, nor hipMemcpy for it
     HIPCHK(hipStreamSynchronize(ctx->stream));
     HIPCHK(hipMemcpy(back.bra.data(), p->bra.p, n * sizeof(int), hipMemcpyDeviceToHost));
     HIPCHK(hipMemcpy(back.ket.data(), p->ket.p, n * sizeof(int), hipMemcpyDeviceToHost));
     HIPCHK(hipMemcpy(back.meta.data(), p->meta.p, n * sizeof(int), hipMemcpyDeviceToHost));
-    HIPCHK(hipMemcpy(back.qidx.data(), p->qidx.p, n * sizeof(long long), hipMemcpyDeviceToHost));
     lists = &back;
   }
   std::vector<int> pb, pk, pm, pf;
-  std::vector<long long> pq;
   std::vector<int2> pr;
   int64_t gtotal = 0;
   bool rys = false;
@@ -749,15 +746,16 @@ void plan_pieces(l2g_eri_plan_s* p, l2g_context_s* ctx, const WorkLists* lists, 
     rys |= c.rys >= 0;
     c.piece_off = (int64_t)pb.size();
     c.pfirst_off = (int64_t)pf.size();
+    size_t n = 0;
+    for (int64_t i = c.first; i < c.first + c.count; ++i) n += (size_t)std::max<int64_t>(1, (p->itemw[(size_t)i] + chunk - 1) / chunk);
+    size_t at = pb.size();
+    pb.resize(at + n), pk.resize(at + n), pm.resize(at + n), pr.resize(at + n);
     for (int64_t i = c.first; i < c.first + c.count; ++i) {
-      pf.push_back((int)((int64_t)pb.size() - c.piece_off));
+      pf.push_back((int)((int64_t)at - c.piece_off));
       const int w = p->itemw[(size_t)i];
-      for (int a = 0; a < w || a == 0; a += (int)chunk) {
-        pb.push_back(lists->bra[(size_t)i]);
-        pk.push_back(lists->ket[(size_t)i]);
-        pm.push_back(lists->meta[(size_t)i]);
-        pq.push_back(lists->qidx[(size_t)i]);
-        pr.push_back(make_int2(a, (int)std::min<int64_t>(w, a + chunk)));
+      for (int64_t a = 0; a < w || a == 0; a += chunk, ++at) {
+        pb[at] = lists->bra[(size_t)i], pk[at] = lists->ket[(size_t)i], pm[at] = lists->meta[(size_t)i];
+        pr[at] = make_int2((int)a, (int)std::min<int64_t>(w, a + chunk));
       }
     }
     pf.push_back((int)((int64_t)pb.size() - c.piece_off));
@@ -771,7 +769,6 @@ void plan_pieces(l2g_eri_plan_s* p, l2g_context_s* ctx, const WorkLists* lists, 
     upload(p->gp_bra, pb, st);
     upload(p->gp_ket, pk, st);
     upload(p->gp_meta, pm, st);
-    upload(p->gp_qidx, pq, st);
     upload(p->gp_range, pr, st);
     upload(p->gp_first, pf, st);
   } catch (const L2gError& e) {
@@ -1021,7 +1018,6 @@ int l2g_eri_plan_execute(l2g_eri_plan p, double* d_out) {
           P.bra_pair = p->gp_bra.as<int>() + c.piece_off;
           P.ket_pair = p->gp_ket.as<int>() + c.piece_off;
           P.meta = p->gp_meta.as<int>() + c.piece_off;
-          P.qidx = p->gp_qidx.as<long long>() + c.piece_off;
           P.q_prange = p->gp_range.as<int2>() + c.piece_off;
           P.n = (int)c.npieces;
           P.gpart_mode = 1;
