@@ -3,10 +3,11 @@
 Each canonical class is compiled with a register budget (doubles per target
 group, codegen/gen_eri.plan_class): a larger budget means fewer groups and
 less recomputation, a smaller one fewer spills and more waves.  The best value
-differs between classes and is measured, not modelled.  Every class but
-(ss|..) evaluates its FP64 integrals on a Rys kernel (codegen/gen_rys.py),
-whose layout has no budget: for those the budget is the FP32 variant's (twice
-as many values) and the Schwarz kernel's.
+differs between classes and is measured, not modelled.  The budget concerns the
+per-lane kernels (codegen/gen_eri.py): FP32 and Schwarz factors, and FP64 ERI
+batches of the classes in gen_rys.LANE_COST.  The Rys kernels (codegen/gen_rys.py)
+that serve FP64 otherwise have no budget, so the other classes are tuned by their
+FP32 variant (twice as many values).
 
   python -m libint_amd.tune build   --dir D [--budgets 128,144,160] [--classes 2222,2122]
         (CPU) one library per budget, holding only the tuned classes (ERI
@@ -38,6 +39,7 @@ import sys
 HERE = os.path.dirname(os.path.abspath(__file__))
 DEFAULT_BUDGETS = (128, 144, 160)
 DEFAULT_BUDGET = 160  # the Makefile's BUDGET
+MODES = "eri,schwarz,fp32,rys"  # of the libraries that are timed: what the shipped one runs ERI batches on
 
 
 def heavy_classes():
@@ -54,7 +56,7 @@ def build(args):
         d = os.path.join(os.path.abspath(args.dir), f"b{b}")
         os.makedirs(d, exist_ok=True)
         cmd = ["make", "-s", "-C", HERE, f"GEN={d}/gen", f"OBJ={d}/obj", f"LIB={d}/libl2g.so",
-               f"ONLY={classes}", "MODES=eri,fp32", f"BUDGET={b}", "CLASSCFG=", "-j2"]
+               f"ONLY={classes}", f"MODES={MODES}", f"BUDGET={b}", "CLASSCFG=", "-j2"]
         procs.append((b, subprocess.Popen(cmd, stdout=subprocess.DEVNULL, stderr=subprocess.PIPE)))
     for b, p in procs:
         _, err = p.communicate()
@@ -176,16 +178,28 @@ def fp32_pays(t64, t32):
     return 1 if t32 is not None and t32 < 0.95 * t64 else 0
 
 
+def budget_time(c, r):
+    """The time of class c, in a library's timings r, that its budget decides: its FP64 kernel's where that is a per-lane
+    kernel, else its FP32 variant's (None: nothing of the class depends on the budget)."""
+    sys.path.insert(0, os.path.join(HERE, "codegen"))
+    import gen_rys
+    return r[c] if gen_rys.lane_cost(*map(int, c)) else r.get(c + "/fp32")
+
+
 def select(args):
     res = json.load(open(os.path.join(args.dir, "timings.json")))
     classes = sorted({c for r in res.values() for c in r if "/" not in c})
     cfg = read_cfg(args.out)
     for c in classes:
-        best = min((r[c], int(b)) for b, r in res.items() if c in r)
+        times = {int(b): budget_time(c, r) for b, r in res.items() if c in r}
+        if None in times.values():
+            print(f"{c}: no kernel with a budget")
+            continue
+        best = min((t, b) for b, t in times.items())
         r = res[str(best[1])]
         cfg[c] = [best[1], 0, fp32_pays(r.get(c + "/e64", r[c]), r.get(c + "/fp32"))]
         print(f"{c}: budget {best[1]} ({best[0]:.2f} ms), fp32 {cfg[c][2]}; " +
-              ", ".join(f"{b}: {r_[c]:.2f}" for b, r_ in sorted(res.items(), key=lambda x: int(x[0])) if c in r_))
+              ", ".join(f"{b}: {t:.2f}" for b, t in sorted(times.items())))
     write_cfg(args.out, cfg)
 
 
