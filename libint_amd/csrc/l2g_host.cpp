@@ -1665,6 +1665,8 @@ int l2g_onebody(l2g_basis B, int ncharge, const double* charges, const double* x
     }
     const long long nbf = bf0[n];
     if (n == 0) return;
+    for (double x : B->alpha)  // every shell is paired with itself, too
+      if (x < 0) throw std::invalid_argument("l2g_onebody: negative exponent");
     hipStream_t st = ctx->stream;
     // shell pairs by class, the shell of higher l first
     int first[17] = {};

@@ -637,6 +637,9 @@ struct PairBuilder {
       for (int p2 = 0; p2 < n2; ++p2) {
         const double a1 = B.alpha[B.off[i] + p1], a2 = B.alpha[B.off[j] + p2];
         const double gamma = a1 + a2, oog = 1.0 / gamma;
+        // no Gaussian: with a positive sum on the other side its T is
+        // negative, and the kernels' tables have no entries there
+        if (gamma < 0) throw std::invalid_argument("primitive pair with a negative sum of exponents");
         const double rho = a1 * a2 * oog;
         const double mr = -rho * AB2;
         double ln_scr = mr + B.lnc[B.off[i] + p1] + B.lnc[B.off[j] + p2];
