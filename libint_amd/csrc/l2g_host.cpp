@@ -1701,7 +1701,7 @@ int l2g_onebody(l2g_basis B, int ncharge, const double* charges, const double* x
                  ob = put(bf0.data(), bf0.size()), oq = put(charges, ncharge), ox = put(xyz, 3 * (size_t)ncharge);
     const size_t bytes = (size_t)nbf * nbf * sizeof(double), om = (h.size() + 255) & ~size_t(255);
     DevBuf d;
-    d.alloc(om + 3 * bytes);
+    d.alloc(om + ((S ? 1 : 0) + (T ? 1 : 0) + (V ? 1 : 0)) * bytes);  // of those asked for
     unsigned char* const dp = d.as<unsigned char>();
     HIPCHK(hipMemcpyAsync(dp, h.data(), h.size(), hipMemcpyHostToDevice, st));
     L2gOneBodyArgs A;
@@ -1721,7 +1721,8 @@ int l2g_onebody(l2g_basis B, int ncharge, const double* charges, const double* x
     A.rys = ctx->rys.as<double>();
     A.gauss = ctx->shg_gaussian;
     double* const dm = reinterpret_cast<double*>(dp + om);
-    double *const dS = dm, *const dT = dm + (size_t)nbf * nbf, *const dV = dT + (size_t)nbf * nbf;
+    const size_t NN = (size_t)nbf * nbf;
+    double *const dS = dm, *const dT = dS + (S ? NN : 0), *const dV = dT + (T ? NN : 0);
     A.S = S ? dS : nullptr, A.T = T ? dT : nullptr, A.V = V ? dV : nullptr;
     launch_onebody(A, reinterpret_cast<const int2*>(dp + opairs), first, st);
     hipError_t e = hipStreamSynchronize(st);

@@ -264,3 +264,22 @@ def test_one_deep_quartet_unsplit(ctx, c):
     v, nz = values(la.EriPlan(la.Basis(ctx, arrays), q), False)
     o, _, onz = oracle.eri_quartets(arrays, q)
     assert agree(v, o) and np.array_equal(nz, onz)
+
+
+@pytest.mark.gpu
+def test_one_body_matrices_asked_for(ctx):
+    """Every choice of S, T and V: the matrices of the call that takes all three, bit for bit."""
+    rng = np.random.default_rng(4)
+    arrays = la.BasisArrays.from_shells([x for l in (0, 1, 2, 3) for x in shells(rng, (l,), (3,))])
+    b = la.Basis(ctx, arrays)
+    charges = [(3.0, (0.1, 0.2, 0.3)), (1.0, (-0.4, 0.5, 0.0))]
+    full = la.one_body(b, charges)
+    n = len(full[0])
+    q, xyz = np.array([c[0] for c in charges]), np.array([c[1] for c in charges]).reshape(-1)
+    say("case: one-body matrices one by one and in pairs")
+    for k in range(1, 8):
+        out = [np.zeros((n, n)) if k >> m & 1 else None for m in range(3)]
+        rc = la.lib().l2g_onebody(b.handle, 2, q.ctypes.data, xyz.ctypes.data,
+                                  *[None if o is None else o.ctypes.data for o in out])
+        assert rc == 0
+        assert all(o is None or np.array_equal(o, f) for o, f in zip(out, full)), k
