@@ -283,3 +283,43 @@ def test_one_body_matrices_asked_for(ctx):
                                   *[None if o is None else o.ctypes.data for o in out])
         assert rc == 0
         assert all(o is None or np.array_equal(o, f) for o, f in zip(out, full)), k
+
+
+# primitive quartets of shells of (a, b, c, d) primitives, on both sides of the tiers (32 and 128) and of the largest
+# number of slots that share a quartet; many shallow ones keep the mean below 64, where the generic kernel would take
+# the heavy classes
+TIER_KS = [(31, 1, 1, 1), (4, 2, 4, 1), (11, 1, 3, 1), (127, 1, 1, 1), (8, 2, 8, 1), (43, 1, 3, 1), (17, 1, 13, 1)]
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("c", [(2, 1, 2, 1), (2, 2, 2, 2), (3, 2, 3, 2), (2, 2, 3, 3), (1, 1, 2, 1), (3, 3, 3, 3)])
+@pytest.mark.parametrize("pure", [True, False])
+def test_slots_of_a_block_share_deep_quartets(ctx, c, pure):
+    """Rys kernels unsplit, blocks of 7 to 3 slots in one and in four waves: quartets of the deep tiers next to shallow
+    ones, each operator, against the oracle; the same bits in another batch."""
+    rng = np.random.default_rng(41 + sum(c))
+    ks = TIER_KS if sum(c) < 9 else TIER_KS[:4]
+    sh = [x for k in ks for x in shells(rng, c, k, pure)] + shells(rng, c, (1, 1, 1, 1), pure)
+    arrays = la.BasisArrays.from_shells(sh)
+    deep = np.arange(4 * len(ks), dtype=np.int32).reshape(-1, 4)
+    one = np.arange(4 * len(ks), len(sh), dtype=np.int32)[None]
+    q = np.concatenate([np.tile(one, (20, 1)), deep, deep[::2]])
+    assert (arrays.nprim[q].prod(1)).mean() < 64
+    b = la.Basis(ctx, arrays)
+    Q = gen_rys.plan(*c).q
+    say(f"case: tiers of {c}, pure {pure}, {Q} slots a block")
+    over = sum(c) >= 11  # (df|ff) and (ff|ff) report the generic kernel's code on their Rys kernels, too
+    for oper, omega in ((la.COULOMB, 0.0), (la.ERF_COULOMB, 0.5), (la.ERFC_COULOMB, 0.5)):
+        plan = la.EriPlan(b, q)
+        plan.set_operator(oper, omega)
+        v, nz = values(plan, False)
+        assert over or not any(s["generic"] or s["wave"] for s in plan.stats())
+        o, _, onz = oracle.eri_quartets(arrays, q, **(dict(oper=oper, omega=omega) if oper else {}))
+        assert agree(v, o) and np.array_equal(nz, onz)
+        off = np.append(plan.offsets(), v.size)
+        for k in range(20, 20 + len(ks)):
+            few = la.EriPlan(b, np.concatenate([q[k:k + 1], np.tile(one, (6, 1))]))
+            few.set_operator(oper, omega)
+            w = values(few, False)[0]
+            assert over or not any(s["generic"] for s in few.stats())
+            assert np.array_equal(w[:off[k + 1] - off[k]], v[off[k]:off[k + 1]]), (k, oper)
