@@ -16,9 +16,10 @@ the Head-Gordon-Pople scheme libint uses by default
   4. a strided write that undoes the canonical reorder
      (include/libint2/engine.impl.h:1987-2067).
 
-These kernels serve FP32 and the Schwarz factors of s, p and d pairs; FP64
-ERIs and Fock builds run on the Rys kernels of gen_rys.py, which share the
-HRR and transform code here.
+These kernels serve FP32, the Schwarz factors of s, p and d pairs and, where
+they are faster, FP64 ERI batches of light classes (gen_rys.LANE_COST); other
+FP64 ERIs and Fock builds run on the Rys kernels of gen_rys.py, which share
+the HRR and transform code here.
 
 Mapping to the hardware: one lane owns one shell quartet and keeps every
 recurrence intermediate in VGPRs.  The contracted target set of a large class
@@ -990,14 +991,12 @@ def class_waves(plan, budget, waves):
 
 
 def generate(outdir, lmax=2, budget=160, nfiles=8, waves=0, only=None, budgets=None,
-             modes=('eri', 'fock', 'schwarz', 'fp32', 'rys'), generic_lmax=3, max_nodes=0, fp32_lmax=2):
+             modes=('eri', 'fock', 'schwarz', 'fp32'), generic_lmax=3, max_nodes=0, fp32_lmax=2):
     """Write the kernels and the dispatch tables.  `budgets` maps a class name
     ('2222') to its own (budget, waves).  Classes with an l above 2 whose
     partitioned recursion evaluates more than `max_nodes` nodes per primitive
-    quartet (0: no limit) get no per-lane kernel; FP32 variants are made for
-    classes with every l <= fp32_lmax.  Mode 'rys' adds the Rys kernels
-    (gen_rys.py) of every class, which replace the FP64 ERI and Fock kernels
-    here."""
+    quartet (0: no limit) get no per-lane kernel; FP32 variants (mode 'fp32')
+    are made for classes with every l <= fp32_lmax."""
     os.makedirs(outdir, exist_ok=True)
     classes = canonical_classes(lmax)
     if only:
@@ -1014,17 +1013,13 @@ def generate(outdir, lmax=2, budget=160, nfiles=8, waves=0, only=None, budgets=N
     # reduced-precision variants hold twice as many values per register
     plans32 = [plan_class(p.la, p.lb, p.lc, p.ld, budget=2 * cfg((p.la, p.lb, p.lc, p.ld))[0]) for p in plans
                if max(p.la, p.lb, p.lc, p.ld) <= fp32_lmax] if 'fp32' in modes else []
-    # classes on the Rys kernels (gen_rys.py) have no other FP64 Fock kernel, and an ERI kernel here where batches of
-    # them are faster on it
+    # FP64: Rys kernels (gen_rys.py) of every class, and an ERI kernel here where batches of a class are faster on it
     sys.path.insert(0, os.path.dirname(os.path.abspath(__file__)))
     import gen_rys
-    ryscls = [c for c in classes if gen_rys.use(*c)] if 'rys' in modes else []
+    ryscls = [c for c in classes if gen_rys.use(*c)]
     jobs = []  # (plan, mode, real)
     for p in plans:
-        c = (p.la, p.lb, p.lc, p.ld)
-        if c not in ryscls:
-            jobs += [(p, m, 'double') for m in ('eri', 'fock') if m in modes]
-        elif gen_rys.lane_cost(*c) and 'eri' in modes:
+        if gen_rys.lane_cost(p.la, p.lb, p.lc, p.ld) and 'eri' in modes:
             jobs += [(p, m, 'double') for m in ('eri', 'att')]
         if 'schwarz' in modes and (p.la, p.lb) == (p.lc, p.ld):
             jobs.append((p, 'schwarz', 'double'))
@@ -1041,8 +1036,8 @@ def generate(outdir, lmax=2, budget=160, nfiles=8, waves=0, only=None, budgets=N
         j = load.index(min(load))
         files[j].append(i)
         load[j] += w
-    tables = {('eri', 'double'): [], ('schwarz', 'double'): [], ('fock', 'double'): [],
-              ('eri', 'float'): [], ('fock', 'float'): [], ('att', 'double'): []}
+    tables = {('eri', 'double'): [], ('att', 'double'): [], ('schwarz', 'double'): [], ('eri', 'float'): [],
+              ('fock', 'float'): []}
     written = []
     for fi, idxs in enumerate(files):
         fn = os.path.join(outdir, f"eri_gen_{fi}.hip")
@@ -1066,12 +1061,11 @@ def generate(outdir, lmax=2, budget=160, nfiles=8, waves=0, only=None, budgets=N
         written.append(fn)
     for k in (('eri', 'double'), ('att', 'double')):  # the same order in both
         tables[k].sort(key=lambda x: x[0].name)
-    table, stable, ftable = tables[('eri', 'double')], tables[('schwarz', 'double')], tables[('fock', 'double')]
+    table, atable, stable = (tables[m, 'double'] for m in ('eri', 'att', 'schwarz'))
     table32, ftable32 = tables[('eri', 'float')], tables[('fock', 'float')]
     lines = ['// generated by libint_amd/codegen/gen_eri.py — do not edit',
              '#include "eri_device.h"', '']
-    atable = tables[('att', 'double')]
-    for p, k, _ in table + stable + ftable + table32 + ftable32 + atable:
+    for p, k, _ in table + atable + stable + table32 + ftable32:
         lines.append(f"void {k}_launch(const L2gEriArgs& A, int grid, int block, hipStream_t s);")
     lines.append('')
     rys = {m: gen_rys.generate(ryscls, m) for m in ('eri', 'fock') if m in modes}
@@ -1093,7 +1087,7 @@ def generate(outdir, lmax=2, budget=160, nfiles=8, waves=0, only=None, budgets=N
         for _, n, _ in v:
             lines.append(f"void {n}_launch(const L2gEriArgs& A, int grid, int block, hipStream_t s);")
     lines.append(f"extern const int l2g_gen_lmax = {lmax};")
-    for name, tab in (("l2g_gen_classes", table), ("l2g_gen_schwarz", stable), ("l2g_gen_fock", ftable),
+    for name, tab in (("l2g_gen_classes", table), ("l2g_gen_schwarz", stable), ("l2g_gen_fock", []),
                       ("l2g_gen_classes32", table32), ("l2g_gen_fock32", ftable32),
                       ("l2g_gen_classes_att", atable), ("l2g_gen_rys", [])):
         lines.append(f"extern const L2gClassInfo {name}[] = {{")
@@ -1103,7 +1097,7 @@ def generate(outdir, lmax=2, budget=160, nfiles=8, waves=0, only=None, budgets=N
             if not in_regs and name in ("l2g_gen_classes", "l2g_gen_classes32", "l2g_gen_classes_att"):
                 ybuf += ncart(p.la) * ncart(p.lb) * ncart(p.lc) * ncart(p.ld)  # staged output
             pays = cfg((p.la, p.lb, p.lc, p.ld))[2] if name in ("l2g_gen_classes32", "l2g_gen_fock32") else 0
-            cost = gen_rys.lane_cost(p.la, p.lb, p.lc, p.ld) if name == "l2g_gen_classes" and ryscls else None
+            cost = gen_rys.lane_cost(p.la, p.lb, p.lc, p.ld) if name == "l2g_gen_classes" else None
             lines.append(f"  {{{p.la}, {p.lb}, {p.lc}, {p.ld}, {len(p.groups)}, {ybuf}, "
                          f"{sum(p.group_nodes)}, {pays}, 0, 0, {{{', '.join(map(str, cost or (0,)))}}}, &{k}_launch}},")
         rest = rys.get({'l2g_gen_fock': 'fock', 'l2g_gen_rys': 'eri'}.get(name), [])
@@ -1116,7 +1110,7 @@ def generate(outdir, lmax=2, budget=160, nfiles=8, waves=0, only=None, budgets=N
         lines.append("};")
     lines.append(f"extern const int l2g_gen_nclasses = {len(table)};")
     lines.append(f"extern const int l2g_gen_nschwarz = {len(stable)};")
-    lines.append(f"extern const int l2g_gen_nfock = {len(ftable) + len(rys.get('fock', []))};")
+    lines.append(f"extern const int l2g_gen_nfock = {len(rys.get('fock', []))};")
     lines.append(f"extern const int l2g_gen_nrys = {len(rys.get('eri', []))};")
     lines.append(f"extern const int l2g_gen_nclasses_att = {len(atable)};")
     lines.append(f"extern const int l2g_gen_nclasses32 = {len(table32)};")
@@ -1150,7 +1144,7 @@ if __name__ == '__main__':
                     help="per class budget:waves[:fp32], e.g. 2222=64:2,2122=80:2:1 (fp32 1: the class's FP32 "
                          "variant measured faster than its FP64 kernel, so mixed batches route quartets to it)")
     ap.add_argument("--nfiles", type=int, default=8)
-    ap.add_argument("--modes", default="eri,fock,schwarz,fp32,rys")
+    ap.add_argument("--modes", default="eri,fock,schwarz,fp32")
     ap.add_argument("--generic-lmax", type=int, default=3, help="highest l of the generic kernel's classes")
     ap.add_argument("--max-nodes", type=int, default=0,
                     help="classes with l > 2 and more recursion nodes than this run on the generic kernel")

@@ -783,8 +783,7 @@ def emit(p, mode):
 
 
 def use(la, lb, lc, ld):
-    """Whether a class runs on its Rys kernel: every class does (0.8 to 28 times
-    the speed of the per-lane kernels on 2000 to 40000 quartets)."""
+    """Whether a class has a Rys kernel: every class does."""
     return True
 
 

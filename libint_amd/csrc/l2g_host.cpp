@@ -85,7 +85,7 @@ struct ClassWork {
   int spec_cls = -1;            // the class's own table index (cls before the layout's choice)
   bool fp32 = false;
   bool generic = false;
-  bool native_generic = false;  // no register kernel for this class
+  bool native_generic = false;  // no per-lane kernel for this class, or the generic kernel forced
   int rys = -1;       // index into l2g_gen_rys where the class runs on its Rys kernel
   int rys_cls = -1;   // the class's Rys kernel, whether it runs on it or not
   int rys_deep[2] = {0, 0};  // items in its tiers of deep quartets (rys_tier_of)
@@ -510,8 +510,8 @@ static int plan_create_impl(l2g_basis B, int64_t nq, const int32_t* quartets, do
       const int b2 = sbk ? (stk ? s[2] : s[3]) : (stb ? s[0] : s[1]);
       const int k1 = sbk ? (stb ? s[1] : s[0]) : (stk ? s[3] : s[2]);
       const int k2 = sbk ? (stb ? s[0] : s[1]) : (stk ? s[2] : s[3]);
-      // FP64: the class's register kernel where it has one, else the bucket of
-      // its generic program (its Rys kernel, or the generic kernel)
+      // FP64: the bucket of the class's per-lane kernel where it has one, else of
+      // its generic program; which kernel runs is the layout's choice
       int cls = bucket64(B->l[b1], B->l[b2], B->l[k1], B->l[k2]);
       if (cls < 0) throw L2gError(L2G_E_LMAX, "no kernel for this angular momentum class");
       if (!ctx->force_generic && fp32_threshold > 0) {

@@ -20,7 +20,7 @@ using namespace l2g_impl;
 namespace {
 
 constexpr int kMaxL = 3;          // f shells
-constexpr size_t kMaxYLane = 9216;  // lane scratch doubles per lane
+constexpr size_t kMaxYLane = 256;  // lane scratch doubles per lane (quartet_ylane)
 constexpr size_t kInBytes = QuartetLayout(2 * (size_t)L2G_NOALLOC_MAX_NPRIM * L2G_NOALLOC_MAX_NPRIM).total;
 constexpr size_t kOutDoubles = 10 * 10 * 10 * 10;  // (ff|ff) in Cartesian functions
 constexpr size_t kYDoubles = kMaxYLane * kQuartetBlock;
