@@ -92,8 +92,8 @@ int l2g_fp32_paying_classes(int cap, int* n, int* codes);
 int l2g_init(int device, l2g_context* ctx);
 
 /* Routes every class through the generic kernel (l2g_generic.hip), which
- * otherwise serves only the classes with an f shell; on = 0 restores the
- * generated register-resident kernels for s, p and d classes.  A testing
+ * otherwise serves only classes of few deep quartets with the layout by batch
+ * off (l2g_eri_plan_set_wave_split); on = 0 restores the generated kernels.  A testing
  * aid with no counterpart in the reference: it lets the generic kernel be
  * checked on every class.  Affects plans, Schwarz factors and Fock builds
  * created afterwards. */

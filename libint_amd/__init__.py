@@ -464,10 +464,11 @@ class EriPlan:
         _check(lib().l2g_eri_plan_set_operator(self._h, int(oper), float(omega)))
 
     def set_wave_split(self, on=True):
-        """Split of deep primitive loops over lanes or blocks (on by default;
-        2 is accepted as 1): each contraction is then summed as partial sums
-        in a fixed order instead of libint's serial one.  False (0) turns it
-        off (l2g_eri_plan_set_wave_split)."""
+        """Layout by batch (on by default; 2 is accepted as 1): kernels, lanes
+        per quartet and pieces of deep primitive loops follow from the whole
+        batch; each contraction is summed as partial sums in a fixed order
+        instead of libint's serial one.  False (0): they follow from the class
+        and the quartet alone (l2g_eri_plan_set_wave_split)."""
         _check(lib().l2g_eri_plan_set_wave_split(self._h, int(on)))
 
     def elapsed_ms(self):

@@ -1,9 +1,8 @@
 """Programs for the generic (table-driven) ERI kernel, libint_amd/csrc/l2g_generic.hip.
 
-The register-resident kernels of gen_eri.py stop at (dd|dd): from f shells on,
-a class's contracted [e0|f0] targets and recursion graph no longer fit a lane
-(for (ff|ff): 5476 targets, 16-17k recursion values per primitive quartet).
-The generic kernel evaluates one contracted quartet per 256-thread block with
+A class's contracted [e0|f0] targets and recursion graph do not fit a lane from f
+shells on (for (ff|ff): 5476 targets, 16-17k recursion values per primitive
+quartet).  The generic kernel evaluates one contracted quartet per block with
 everything in LDS, and reads the work of each class from data written here:
 
 * OS VRR, one record per [e0|f0] node carrying the node's whole m-vector

@@ -1,6 +1,6 @@
-// Generic (table-driven) kernel for the classes the register-resident
-// kernels do not cover: every class with an f shell.  One 256-thread block
-// evaluates one contracted shell quartet at a time with all intermediates in
+// Generic (table-driven) kernel of every class: forced on (a testing aid), and
+// for ERI classes of few deep quartets with the layout by batch off; else the
+// generated kernels run.  One block of 256 to 1024 threads evaluates one contracted shell quartet at a time with all intermediates in
 // LDS; the per-class work comes from the programs of codegen/gen_generic.py:
 //
 //   1. per primitive quartet: screening and prefactors (every thread, the

@@ -482,8 +482,8 @@ void onebody_init(const double* sh);  // sh[4][7][10] solid-harmonic coefficient
 void launch_deriv1_combine(const double* raw, const long long* raw_off, const long long* out_off, const int* qinfo,
                            long long nq, long long total, double* out, const L2gDerivTab& tab, hipStream_t s);
 
-// l2g_generic.hip: the table-driven kernel for classes without a generated
-// register-resident kernel (f shells); modes ERI store, Fock digest, Schwarz
+// l2g_generic.hip: the table-driven kernel, any class; modes ERI store, Fock
+// digest, Schwarz
 enum { kGenericEri = 0, kGenericFock = 1, kGenericSchwarz = 2 };
 void generic_init(const double* sh);  // sh[4][7][10] solid-harmonic coefficients
 void launch_generic(int mode, const L2gEriArgs& A, const L2gGenericClass& C, const int4* prog, const int* idx,
